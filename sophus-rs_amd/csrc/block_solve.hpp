@@ -80,9 +80,8 @@ BlockSolveBufs bind_block_solve(const Symbolic& S, const std::vector<double>& bl
   df.ltbuf = a.template alloc<double>(size_t(S.t_elems));
   df.tinv = a.template alloc<double>(size_t(S.p_elems));
   df.wbuf = a.template alloc<double>(size_t(S.w_elems));
-  df.piv_L = a.template alloc<double>(size_t(36) * nb);
   df.piv_d = a.template alloc<double>(size_t(6) * nb);
-  df.piv_M = a.template alloc<double>(size_t(36) * nb);
+  df.piv_r = a.template alloc<double>(size_t(6) * nb);
   df.front_elems = S.front_elems;
   df.host = &S;
   b.blocks = bind_up(a, blocks);

@@ -774,29 +774,12 @@ __global__ void k_zero_scalars(DevScalars* sc) {
 
 // ---- supernodal multifrontal LDLt ---------------------------------------------------------
 // Fronts are dense column-major F x F (F = 6 * front rows); the first K = 6 * node columns
-// are eliminated with 6x6 pivots (the reference's block LDLt, block_sparse_ldlt.rs:614-747):
-// for pivot j: (L_jj, d_j) = ldlt6(C_jj); L_ij = C_ij L_jj^-T D^-1 L_jj^-1 for rows i > j;
-// trailing C_ik -= L_ij C_kj^T.  Panels of kPanelBlocks pivots are factored by one
-// workgroup per node; the rank-24 trailing update runs as 64x64 tiles over many workgroups.
-
-// x <- x L^-T D^-1 L^-1 for a 6x6 pivot (unit lower L, dinv = reciprocal pivots, 0 for a
-// zero pivot)
-__device__ __forceinline__ void right_solve6(const double* L, const double* dinv, double x[6]) {
-#pragma unroll
-  for (int c = 0; c < 6; ++c) {
-    double v = x[c];
-    for (int t = 0; t < c; ++t) v -= x[t] * L[6 * c + t];
-    x[c] = v;
-  }
-#pragma unroll
-  for (int c = 0; c < 6; ++c) x[c] *= dinv[c];
-#pragma unroll
-  for (int c = 5; c >= 0; --c) {
-    double v = x[c];
-    for (int t = c + 1; t < 6; ++t) v -= x[t] * L[6 * t + c];
-    x[c] = v;
-  }
-}
+// are eliminated as L D L^T with the reference's 6x6 pivot rule (its block LDLt,
+// block_sparse_ldlt.rs:614-747: pivot block j gives (L_jj, d_j) = ldlt6(C_jj) and
+// L_ij = C_ij L_jj^-T D^+ L_jj^-1).  Here L is the scalar unit lower factor, the reference's
+// times blockdiag(L_jj): its columns are U D^+ with U = C L_PP^-T, so a panel's rows need one
+// product and a scaling.  Panels of kPanelBlocks pivot blocks are factored by one
+// workgroup per node; the rank-48 trailing update runs as 64x64 tiles over many workgroups.
 
 constexpr int kPW = 6 * kPanelBlocks;
 
@@ -806,97 +789,182 @@ __device__ __forceinline__ double (*as_square(double (*t)[kTile + 1]))[kPW + 1] 
   return reinterpret_cast<double (*)[kPW + 1]>(&t[0][0]);
 }
 
-// Trailing update of pivot JB of a diagonal block: the rows below the next pivot block,
-// four threads per row (thread t3 of 192), each forming the row's L from its W and
-// updating every fourth column; the updated values of the next pivot's columns are also
-// kept in Wd (the next pivot's W).  The pivot index is a template argument so that the
-// column loop has a fixed length and its LDS reads can be issued together.
-template <int JB>
-__device__ __forceinline__ void diag_trailing(int t3, int np, const double* cL, const double* cdi,
-                                              double (*D)[kPW + 1], double (*Wd)[kPW + 1]) {
-  constexpr int J0 = 6 * JB, J1 = J0 + 6, kSplit = 4;
-  const int rr = t3 / kSplit, cg = t3 % kSplit;
-  const int r = J1 + 6 + rr;
-  if (J1 + 6 >= kPW || r >= np) return;
-  double x[6];
-#pragma unroll
-  for (int t = 0; t < 6; ++t) x[t] = Wd[r][J0 + t];
-  right_solve6(cL, cdi, x);
-  if (cg == 0)
-#pragma unroll
-    for (int t = 0; t < 6; ++t) D[r][J0 + t] = x[t];
-  constexpr int kCols = J1 < kPW ? (kPW - 1 - J1) / kSplit + 1 : 0;
-#pragma unroll
-  for (int i = 0; i < kCols; ++i) {
-    const int c = J1 + cg + kSplit * i;
-    if (c <= r) {
-      double acc = 0.0;
-#pragma unroll
-      for (int t = 0; t < 6; ++t) acc += x[t] * Wd[c][J0 + t];
-      const double v = D[r][c] - acc;
-      D[r][c] = v;
-      if (i < 2 && c < J1 + 6) Wd[r][c] = v;
-    }
+typedef double mfma_d4 __attribute__((ext_vector_type(4)));
+
+// f(integral_constant<int, I>) for I = B..E-1: indices that are constants, so that an array
+// indexed by them stays in registers (a nest of this depth is past the loop unroller).
+template <int B, int E, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (B < E) {
+    f(std::integral_constant<int, B>{});
+    static_for<B + 1, E>(f);
   }
 }
 
-// Row block JB of T = L^-1 for the unit block-lower L held below the pivot blocks of D
-// (its column blocks < JB are final), kept transposed in D's free upper triangle:
-// D[c][r] = T[r][c] for block(c) < block(r).  Entries slot, slot + stride, ...; each a
-// fixed-length sum (terms outside the entry's range masked) in four partial sums.
-template <int JB>
-__device__ __forceinline__ void diag_trows(int slot, int stride, double (*D)[kPW + 1]) {
-  constexpr int J0 = 6 * JB;
-  for (int e = slot; e < 6 * J0; e += stride) {
-    const int a = e % 6, c = e / 6, cb = c / 6;
-    double acc[4] = {-D[J0 + a][c], 0.0, 0.0, 0.0};
-#pragma unroll
-    for (int kb = 1; kb < JB; ++kb)
-#pragma unroll
-      for (int t = 0; t < 6; ++t) {
-        const double tv = D[c][6 * kb + t];
-        acc[(6 * kb + t) & 3] -= D[J0 + a][6 * kb + t] * (kb > cb ? tv : 0.0);
+// The value of lane N of each 16-lane row, in all its lanes.
+template <int N>
+__device__ __forceinline__ double row_value(double v) {
+  constexpr int kNewBcast = 0x150 + N;  // DPP row_newbcast:N
+  const int2 b = __builtin_bit_cast(int2, v);
+  return __builtin_bit_cast(double,
+                            make_int2(__builtin_amdgcn_mov_dpp(b.x, kNewBcast, 0xf, 0xf, true),
+                                      __builtin_amdgcn_mov_dpp(b.y, kNewBcast, 0xf, 0xf, true)));
+}
+
+// acc += row_value<N>(v) * m in one instruction.  v must have been written two instructions
+// before (the DPP read hazard); the callers' m depends on row_value of the same register.
+template <int N>
+__device__ __forceinline__ void fmac_row_value(double& acc, double v, double m) {
+  asm("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+      : "+v"(acc)
+      : "v"(v), "v"(m), "n"(N));
+}
+
+constexpr int kSub = 16;  // columns a wavefront eliminates at a time
+static_assert(kPW == 3 * kSub, "three parts of a diagonal block");
+
+// Eliminates the first ncol (even) of kSub columns by one wavefront: lane i of each 16-lane
+// row holds pivot row i in p (the same in every row of lanes), every lane one row below in q.
+// No pivot test: a column is scaled by the reciprocal of what it finds.  On return p and q
+// hold U = C L^-T and lane c (of each 16) the pivot d_c in dv.
+//
+// The next pivot's reciprocal is a chain of six dependent instructions; each is placed behind
+// some of the column's independent updates (the scheduling barriers keep that order, which
+// the compiler's scheduler would undo: it takes an asm statement's result as ready at once).
+__device__ __forceinline__ void eliminate_part(double (&p)[kSub], double (&q)[kSub], int ncol,
+                                               double& dv) {
+  const int li = threadIdx.x & 15;
+  double d = row_value<0>(p[0]), r = recip_nr(d);
+  static_for<0, kSub / 2>([&](auto pair) __attribute__((always_inline)) {
+    if (2 * pair >= ncol) return;
+    static_for<2 * pair, 2 * pair + 2>([&](auto c) __attribute__((always_inline)) {
+      dv = li == c ? d : dv;
+      const double lp = -(p[c] * r), lq = -(q[c] * r);
+      // update k of the column: p[c + 1], then p and q in turn
+      constexpr int kUp = 2 * (kSub - 1 - c);
+      auto update = [&](auto k) __attribute__((always_inline)) {
+        constexpr int i = c + 1 + k / 2;
+        if constexpr (k % 2 == 0) fmac_row_value<i>(p[i], p[c], lp);
+        else fmac_row_value<i>(q[i], p[c], lq);
+      };
+      auto updates = [&](auto from, auto to) __attribute__((always_inline)) {
+        static_for<(from < kUp ? int(from) : kUp), (to < kUp ? int(to) : kUp)>(update);
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      using std::integral_constant;
+      if constexpr (kUp > 0) {
+        updates(integral_constant<int, 0>{}, integral_constant<int, 4>{});
+        d = row_value<(c + 1 < kSub ? c + 1 : 0)>(p[c + 1 < kSub ? c + 1 : 0]);
+        updates(integral_constant<int, 4>{}, integral_constant<int, 6>{});
+        r = __builtin_amdgcn_rcp(d);
+        updates(integral_constant<int, 6>{}, integral_constant<int, 12>{});
+        double e = fma(-d, r, 1.0);
+        updates(integral_constant<int, 12>{}, integral_constant<int, 14>{});
+        r = fma(r, e, r);
+        updates(integral_constant<int, 14>{}, integral_constant<int, 16>{});
+        e = fma(-d, r, 1.0);
+        updates(integral_constant<int, 16>{}, integral_constant<int, 18>{});
+        r = fma(r, e, r);
+        updates(integral_constant<int, 18>{}, integral_constant<int, kUp>{});
       }
-    D[c][J0 + a] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
-  }
+    });
+  });
 }
 
 // The per-node values a diagonal factorization needs, read at kernel entry (ahead of the
 // barriers, which would otherwise keep these loads from being hoisted).
 struct DiagNode {
-  int c0, K;                        // first column block, node columns
+  int c0;                           // first column block
   int64_t loff, toff, poff, uoff;   // L panel, row-major L_KK copy, L_PP^-T slots, RHS
 };
 __device__ __forceinline__ DiagNode diag_node(const DevFactor& f, int X) {
-  return DiagNode{f.sn_c0[X],   6 * f.sn_nc[X], f.sn_loff[X],
-                  f.sn_toff[X], f.sn_poff[X],   f.sn_uoff[X]};
+  return DiagNode{f.sn_c0[X], f.sn_loff[X], f.sn_toff[X], f.sn_poff[X], f.sn_uoff[X]};
 }
 
-// Factor the np x np diagonal block of the panel at column k0 of one front in LDS (block
-// LDLt with 6x6 pivots and the PSD rule), then store L_PP (strictly below the pivot
-// blocks) into the factor and its row-major copy, the pivots (L_jj, d_j, M_j) into
-// piv_L / piv_d / piv_M and L_PP^-T into the panel's slot of tinv.  Called by all threads
-// of one workgroup.  D holds the block's lower triangle already when `loaded` (else it is
-// read from the front).  sL / sdi hold each pivot's factor (L_jj, then d_j in
-// sL[j][36..41]; 1 / d_j in sdi[j]).
-//
-// Per pivot j (one barrier each):
-//   wavefront 0   the next pivot block: lane (a, b), a >= b, of 21 forms row j1 + a of L
-//                 from its W (the row's values before the solve) and subtracts L_a W_b^T;
-//                 thread 0 gathers the 21 entries and factors the block, so its factor is
-//                 ready at the next barrier;
-//   wavefronts 1-3  the trailing update of the rows below the next pivot block (four
-//                 consecutive threads per row, each row's L formed from its W; the updated
-//                 values of the next pivot's columns are also kept in Wd, the next
-//                 pivot's W) and row block j of T = L_PP^-1 (its L columns are final),
-//                 spread from the last thread down so that it falls on the threads whose
-//                 rows have no trailing work.
-// The pivots' inverses M_j and the stores follow the loop.
-__device__ void factor_panel_diag(const DevFactor& f, const DiagNode& dn, double* A, int F, int k0,
-                                  int np, DevScalars* sc, double (*D)[kPW + 1],
-                                  double (*Wd)[kPW + 1], double (*sL)[42], double (*sdi)[6],
-                                  bool loaded, double* __restrict__ z) {
+// The np x np diagonal block in D (lower triangle) by 6x6 pivot blocks with the solver's
+// pivot rule, for blocks with a pivot that the rule zeroes or could zero later: D's columns
+// become U, T's rows (any initial values) rows of L_PP^-T, xd / xr the pivots and their reciprocals
+// (0 for a zero pivot); w is scratch for 48 doubles.  Called by all threads of a workgroup.
+__device__ __forceinline__ void factor_diag_general(int np, bool scalar_rule, DevScalars* sc,
+                                                    double (*D)[kPW + 1], double (*T)[kPW + 1],
+                                                    double* xd, double* xr, double* w) {
   const int tid = threadIdx.x;
+  for (int e = tid; e < kPW * kPW; e += kThreads) T[e / kPW][e % kPW] = e / kPW == e % kPW && e % kPW < np ? 1.0 : 0.0;
+#pragma unroll 1
+  for (int j0 = 0; j0 < np; j0 += 6) {
+    __syncthreads();
+    if (tid == 0) {
+      double a6[36], L[36], d[6], di[6];
+      for (int a = 0; a < 6; ++a)
+        for (int b = 0; b < 6; ++b) a6[6 * a + b] = a >= b ? D[j0 + a][j0 + b] : D[j0 + b][j0 + a];
+      if (!(scalar_rule ? ldlt6<true>(a6, L, d, di) : ldlt6<false>(a6, L, d, di))) {
+        atomicOr(&sc->bad_pivot, 1);
+        for (int k = 0; k < 36; ++k) L[k] = (k % 7 == 0) ? 1.0 : 0.0;
+        for (int k = 0; k < 6; ++k) d[k] = di[k] = 0.0;
+      }
+      for (int k = 0; k < 36; ++k) w[k] = L[k];
+      for (int k = 0; k < 6; ++k) {
+        xd[j0 + k] = d[k];
+        xr[j0 + k] = di[k];
+      }
+    }
+    __syncthreads();
+    const int j1 = j0 + 6, m = np - j1;  // rows of the block below, then the rows of T
+    auto row = [&](int r) { return r < m ? D[j1 + r] : T[r - m]; };
+    for (int r = tid; r < m + np; r += kThreads) {
+      double* x = row(r) + j0;
+#pragma unroll 1
+      for (int c = 1; c < 6; ++c) {
+        double v = x[c];
+        for (int t = 0; t < c; ++t) v -= x[t] * w[6 * c + t];
+        x[c] = v;
+      }
+    }
+    __syncthreads();
+    for (int e = tid; e < (m + np) * m; e += kThreads) {
+      const int r = e / m, c = j1 + e % m;
+      if (r < m && c > j1 + r) continue;
+      double* x = row(r);
+      double v = x[c];
+      for (int t = 0; t < 6; ++t) v -= x[j0 + t] * xr[j0 + t] * D[c][j0 + t];
+      x[c] = v;
+    }
+  }
+  __syncthreads();
+}
+
+constexpr int kDiagScratch = 3 * kSub * kPW + 3 * kPW + 2;  // doubles of factor_panel_diag's X
+static_assert(kDiagScratch <= kPW * (kTile + 1), "a staged tile's memory holds it");
+
+// Factor the np x np diagonal block of the panel at column k0 of one front in LDS (LDL^T
+// with the solver's rule on each 6x6 pivot block): the pivots d and 1 / d (0 for a zero
+// pivot) go to piv_d / piv_r and L_PP^-T to the panel's slot of tinv (zeros past np).
+// Called by all threads of one workgroup; D holds the block's lower triangle already when
+// `loaded` (else it is read from the front), X and T are scratch.  No later kernel reads L_PP.
+//
+// The bound is the serial chain of np pivots.  The block is taken in three parts of 16
+// columns, each eliminated by one wavefront in registers, a row per lane and the pivot rows
+// repeated in each 16 lanes, so that a column's update is one multiply-add whose other factor
+// is read across the lanes (no barrier or LDS access between pivots).  L_PP^-T comes from
+// the same instructions: rows of the identity appended below the block become its rows when
+// eliminated, and 48 rows lie below the pivot rows in every part.  Between the parts the
+// other three wavefronts apply the rank-16 update on the matrix cores.  The pivot rule is
+// checked at the end: where it has nothing to zero (every |d| above 1e-12 of 1 and of the
+// block's largest) the result stands, otherwise factor_diag_general does the block again.
+// Entries above the diagonal and past np are whatever the memory holds: they only reach
+// entries of their own kind, which no output reads.
+//
+// Measured alone (one workgroup, loads and stores included) against 6x6 pivot blocks with
+// an LDS trailing update and a barrier each: 45.0k -> 17.1k cycles at np = 48, 20.0k -> 10.9k at
+// 24, 6.0k -> 5.3k at 6; a fused round of panel steps (500-camera walk) 29.0 -> 18.2 us.  Of
+// the 17.1k, 8.2k are the three parts, 3.6k the two exchanges.  A readlane and multiply-add per
+// update instead of the cross-lane operand took 24 cycles to its 5.
+__device__ __forceinline__ void factor_panel_diag(const DevFactor& f, const DiagNode& dn, double* A,
+                                                  int F, int k0, int np, DevScalars* sc,
+                                                  double (*D)[kPW + 1], double* X,
+                                                  double (*T)[kPW + 1], bool loaded,
+                                                  double* __restrict__ z) {
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   if (!loaded) {
     stage_lds<(kPW * kPW + kThreads - 1) / kThreads>(
         np * np,
@@ -907,188 +975,115 @@ __device__ void factor_panel_diag(const DevFactor& f, const DiagNode& dn, double
         [&](int e, double v) { D[e % np][e / np] = v; });
     __syncthreads();
   }
-  // W of the first pivot: its columns below its block
-  for (int e = 36 + tid; e < 6 * np; e += blockDim.x) Wd[e / 6][e % 6] = D[e / 6][e % 6];
-  // L_PP^-T (row-major kPW x kPW) for the panel rows: its unit diagonal blocks and zeros
-  // here, the blocks above the diagonal as T's row blocks are formed
-  double* Tg = f.tinv + dn.poff + int64_t(k0 / kPW) * kPW * kPW;
-  for (int e = tid - 64; e >= 0 && e < kPW * kPW; e += blockDim.x - 64) {  // beside pivot 0
-    const int r = e / kPW, c = e % kPW;
-    if (r / 6 >= c / 6 || c >= np) Tg[e] = r == c && r < np ? 1.0 : 0.0;
-  }
-  double* Lout = f.lbuf + dn.loff;
-  double* Lt = f.ltbuf + dn.toff;
-  const int K = dn.K;
-  // thread 0 factors the 6x6 block a6 into slot s
-  auto factor_pivot = [&](const double* a6, int s) {
-    double L[36], d[6], di[6];
-    const bool ok = f.scalar_pivots ? ldlt6<true>(a6, L, d, di) : ldlt6<false>(a6, L, d, di);
-    if (!ok) {
-      atomicOr(&sc->bad_pivot, 1);
-      for (int k = 0; k < 36; ++k) L[k] = (k % 7 == 0) ? 1.0 : 0.0;
-      for (int k = 0; k < 6; ++k) d[k] = di[k] = 0.0;
-    }
-    for (int k = 0; k < 36; ++k) sL[s][k] = L[k];
-    for (int k = 0; k < 6; ++k) {
-      sL[s][36 + k] = d[k];
-      sdi[s][k] = di[k];
-    }
+  // [part][column][row]: U of the 48 rows below each part; before the last part's, its memory
+  // holds the next part's initial rows
+  double (*xu)[kSub][kPW] = reinterpret_cast<double (*)[kSub][kPW]>(X);
+  double (*xo)[kPW] = xu[2];
+  double *xd = X + 3 * kSub * kPW, *xr = xd + kPW, *xb = xr + kPW;
+  int* general = reinterpret_cast<int*>(xb + kPW);
+  // no rows below the panel (the last panel of a root), so no panel step follows: its
+  // right-hand side is final here
+  const bool root = k0 + np == F;
+  if (root && tid < np) xb[tid] = f.usolve[dn.uoff + k0 + tid];
+  const int lr = lane & 15, lc = lane >> 4;
+  // acc -= L U^T for the 16 rows of part P's U from R (scaled by 1 / d) and those from C
+  auto rank16 = [&](int P, int R, int C, mfma_d4 acc) {
+#pragma unroll
+    for (int k = 0; k < kSub; k += 4)
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(-xr[kSub * P + k + lc] * xu[P][k + lc][R + lr],
+                                                 xu[P][k + lc][C + lr], acc, 0, 0, 0);
+    return acc;
   };
-  if (tid == 0) {
-    double a6[36];
-    for (int a = 0; a < 6; ++a)
-      for (int b = 0; b < 6; ++b) a6[6 * a + b] = a >= b ? D[a][b] : D[b][a];
-    factor_pivot(a6, 0);
-  }
-  for (int j0 = 0; j0 < np; j0 += 6) {
-    __syncthreads();  // pivot j0 is in slot j0 / 6; the previous pivot's work is done
-    const int jb = j0 / 6;
-    const double* cL = sL[jb];
-    const double* cdi = sdi[jb];
-    const int j1 = j0 + 6, m = np - j1;  // the next pivot; rows of the block below this one
-    if (tid < 64) {
-      if (m > 0) {
-        const int e = tid < 21 ? tid : 0;
-        int a = 0;
-        while ((a + 1) * (a + 2) / 2 <= e) ++a;
-        const int b = e - a * (a + 1) / 2;
-        double x[6];
+  auto block = [&](int R, int C) {  // the block's 16x16 tile at (R, C)
+    mfma_d4 v;
 #pragma unroll
-        for (int t = 0; t < 6; ++t) x[t] = Wd[j1 + a][j0 + t];
-        right_solve6(cL, cdi, x);
-        if (tid < 21 && b == 0)
+    for (int i = 0; i < 4; ++i) v[i] = D[R + lc + 4 * i][C + lr];
+    return v;
+  };
+  auto next_rows = [&](int R, mfma_d4 v) {
 #pragma unroll
-          for (int t = 0; t < 6; ++t) D[j1 + a][j0 + t] = x[t];
-        double acc = D[j1 + a][j1 + b];
-#pragma unroll
-        for (int t = 0; t < 6; ++t) acc -= x[t] * Wd[j1 + b][j0 + t];
-        // gather the 21 entries into thread 0 (uniform reads of lanes 0..20)
-        const int2 bits = __builtin_bit_cast(int2, acc);
-        double a6[36];
-#pragma unroll
-        for (int q = 0; q < 21; ++q) {
-          int qa = 0;
-          while ((qa + 1) * (qa + 2) / 2 <= q) ++qa;
-          const int qb = q - qa * (qa + 1) / 2;
-          const int2 vb = make_int2(__builtin_amdgcn_readlane(bits.x, q),
-                                    __builtin_amdgcn_readlane(bits.y, q));
-          const double v = __builtin_bit_cast(double, vb);
-          a6[6 * qa + qb] = v;
-          a6[6 * qb + qa] = v;
+    for (int i = 0; i < 4; ++i) xo[lr][R + lc + 4 * i] = v[i];
+  };
+  const mfma_d4 none = {0.0, 0.0, 0.0, 0.0};
+  mfma_d4 keep = none;  // wavefronts 1, 2: the last part's columns of identity / block rows
+  static_for<0, 3>([&](auto part) __attribute__((always_inline)) {
+    constexpr int P = part, c0 = kSub * P;
+    if (c0 >= np) return;
+    if (wv == 0) {
+      // rows below: those of the block (32 - c0, in order), then of the identity
+      constexpr int nblk = kPW - c0 - kSub;
+      const int row = min(lane, kPW - 1);
+      double p[kSub], q[kSub], dv = 1.0;
+      static_for<0, kSub>([&](auto c) __attribute__((always_inline)) {
+        const double unit = row - nblk == c0 + c ? 1.0 : 0.0;
+        if constexpr (P == 0) {
+          p[c] = D[lr][c];
+          const double v = D[kSub + min(row, nblk - 1)][c];
+          q[c] = row < nblk ? v : unit;
+        } else {
+          p[c] = xo[c][lr];
+          const double v = xo[c][kSub + min(row, 2 * kSub - 1)];
+          q[c] = row < 2 * kSub ? v : unit;
         }
-        if (tid == 0) factor_pivot(a6, jb + 1);
-      }
-    } else {
-      static_assert(kThreads - 64 == 4 * kPW && kPanelBlocks == 8, "four threads per block row");
-      switch (jb) {
-#define SGPU_TRAIL(J) \
-  case J: diag_trailing<J>(tid - 64, np, cL, cdi, D, Wd); break;
-        SGPU_TRAIL(0) SGPU_TRAIL(1) SGPU_TRAIL(2) SGPU_TRAIL(3)
-        SGPU_TRAIL(4) SGPU_TRAIL(5) SGPU_TRAIL(6) SGPU_TRAIL(7)
-#undef SGPU_TRAIL
+      });
+      eliminate_part(p, q, min(np - c0, kSub), dv);
+      if (lane < kPW)
+        static_for<0, kSub>([&](auto c) __attribute__((always_inline)) { xu[P][c][lane] = q[c]; });
+      if (lane < kSub) {
+        xd[c0 + lane] = dv;
+        xr[c0 + lane] = recip_nr(dv);
       }
     }
-    // Beside the look-ahead: row block jb of T = L_PP^-1 (its L columns are final), kept
-    // transposed in the free upper triangle, D[c][r] = T[r][c] for block(c) < block(r),
-    // four partial sums per entry; then the outputs of pivot jb - 1 (M_j, L_jj, d_j) and
-    // the stores of L's column block jb - 1 and T's row block jb - 1.  The entries of T go
-    // first to the wavefronts with the least trailing work (wavefront 1, then 3 and 2 while
-    // wavefront 2's rows are updated, 2 and 3 after); the last pivot has no look-ahead,
-    // so there wavefront 0 joins and also handles that pivot's outputs.
-    const bool look = m > 0;
-    const int wv = tid >> 6, lane = tid & 63;
-    if (!look || wv > 0) {
-      const int pos = !look ? wv : (jb >= 4 ? wv - 1 : (wv == 1 ? 0 : (wv == 3 ? 1 : 2)));
-      const int slot = 64 * pos + lane, stride = look ? kThreads - 64 : kThreads;
-      switch (jb) {
-#define SGPU_TROWS(J) \
-  case J: diag_trows<J>(slot, stride, D); break;
-        SGPU_TROWS(1) SGPU_TROWS(2) SGPU_TROWS(3) SGPU_TROWS(4)
-        SGPU_TROWS(5) SGPU_TROWS(6) SGPU_TROWS(7)
-#undef SGPU_TROWS
-      }
-      // M_j = L^-T D^+ L^-1 (lane (a, b) of 36, from the columns of L^-1), L_jj and d_j
-      auto pivot_outputs = [&](int j) {
-        const int gb = dn.c0 + k0 / 6 + j;
-        if (lane < 36) {
-          const int a = lane / 6, b = lane % 6;
-          double ua[6], ub[6];
-#pragma unroll
-          for (int k = 0; k < 6; ++k) {
-            ua[k] = k == a ? 1.0 : 0.0;
-            ub[k] = k == b ? 1.0 : 0.0;
-          }
-#pragma unroll
-          for (int k = 1; k < 6; ++k)
-#pragma unroll
-            for (int t = 0; t < k; ++t) {
-              ua[k] -= sL[j][6 * k + t] * ua[t];
-              ub[k] -= sL[j][6 * k + t] * ub[t];
-            }
-          double mm = 0.0;
-#pragma unroll
-          for (int k = 0; k < 6; ++k) mm += ua[k] * sdi[j][k] * ub[k];
-          f.piv_M[36 * int64_t(gb) + lane] = mm;
-          f.piv_L[36 * int64_t(gb) + lane] = sL[j][lane];
-        } else if (lane < 42) {
-          f.piv_d[6 * int64_t(gb) + lane - 36] = sL[j][lane];
-        }
-      };
-      if (jb > 0 && wv == (jb >= 4 ? 2 : 3)) {
-        pivot_outputs(jb - 1);
-        const int p0 = j0 - 6, nr = np - j0;
-        for (int e = lane; e < 6 * nr; e += 64) {
-          const int rr2 = e % nr, t = e / nr;
-          Lout[int64_t(k0 + p0 + t) * F + k0 + j0 + rr2] = D[j0 + rr2][p0 + t];
-        }
-        for (int e = lane; e < 6 * nr; e += 64) {  // row-major copy
-          const int rr2 = e / 6, t = e % 6;
-          Lt[int64_t(k0 + j0 + rr2) * K + k0 + p0 + t] = D[j0 + rr2][p0 + t];
-        }
-        for (int e = lane; e < 6 * p0; e += 64) {
-          const int cp = e / 6, a = e % 6;
-          Tg[cp * kPW + p0 + a] = D[cp][p0 + a];
-        }
-      }
-      if (!look && wv == 0) pivot_outputs(jb);
-    }
-  }
-  __syncthreads();  // T's last row block is in D
-  const int pl = np - 6;
-  for (int e = tid; e < 6 * pl; e += blockDim.x) {
-    const int cp = e / 6, a = e % 6;
-    Tg[cp * kPW + pl + a] = D[cp][pl + a];
-  }
-  if (k0 + np == F) {
-    // no rows below the panel (the last panel of a root), so no panel step follows: its
-    // right-hand side is final here; z_P = D^-1 L_PP^-1 b_P for the panel's columns
-    const double* bx = f.usolve + dn.uoff + k0;
-    double* yv = Wd[0];  // the block's W copy is done with
-    if (tid < np) {
-      double y = bx[tid];
-      for (int r = 0; r < 6 * (tid / 6); ++r) y += D[r][tid] * bx[r];  // T[c][r] = D[r][c]
-      yv[tid] = y;
-    }
+    if (c0 + kSub >= np) return;
     __syncthreads();
-    if (tid < np / 6) {
-      const int j = tid;
-      double v[6];
-#pragma unroll
-      for (int i = 0; i < 6; ++i) {
-        double t = yv[6 * j + i];
-        for (int k = 0; k < i; ++k) t -= sL[j][6 * i + k] * v[k];
-        v[i] = t;
+    if constexpr (P == 0) {  // rows of xu[0]: block 16..47, identity 0..15
+      if (wv == 1) next_rows(0, rank16(0, 0, 0, block(16, 16)));
+      if (wv == 2) next_rows(16, rank16(0, 16, 0, block(32, 16)));
+      if (wv == 3) next_rows(32, rank16(0, 32, 0, none));
+      __syncthreads();
+      if (np > 2 * kSub) {  // beside the next part
+        if (wv == 1) keep = rank16(0, 32, 16, none);
+        if (wv == 2) keep = rank16(0, 16, 16, block(32, 32));
       }
+    } else {  // rows of xu[1]: block 32..47, identity 0..31
+      if (wv == 1) next_rows(16, rank16(1, 16, 0, keep));
+      if (wv == 2) next_rows(0, rank16(1, 0, 0, keep));
+      if (wv == 3) next_rows(32, rank16(1, 32, 0, none));
+      __syncthreads();
+    }
+  });
+  if (wv == 0) {
+    // a pivot that the rule zeroes, or would once a larger one follows it (or not finite)
+    const double ad = fabs(xd[min(lane, np - 1)]);
+    double mx = 1.0;
+    if (!f.scalar_pivots)
+      for (int t = 0; t < 6; ++t) mx = fmax(mx, fabs(xd[min(lane, np - 1) / 6 * 6 + t]));
+    const bool any = __any(!(ad > mx * 1e-12 && ad < __builtin_inf()));
+    if (lane == 0) *general = any;
+  }
+  __syncthreads();
+  double* Tg = f.tinv + dn.poff + int64_t(k0 / kPW) * kPW * kPW;
+  const bool redo = *general;
+  if (redo) factor_diag_general(np, f.scalar_pivots, sc, D, T, xd, xr, X);
+  // row r of L_PP^-T is row (block rows below part P) + r of part P's U
+  auto tinv = [&](int r, int c) {
+    const int P = c / kSub;
+    if (redo) return T[r][c];
+    return r < kSub * (P + 1) && r < np && c < np ? xu[P][c % kSub][kPW - kSub * (P + 1) + min(r, kSub * (P + 1) - 1)] : 0.0;
+  };
 #pragma unroll
-      for (int i = 0; i < 6; ++i) v[i] *= sdi[j][i];
-#pragma unroll
-      for (int i = 5; i >= 0; --i) {
-        double t = v[i];
-        for (int k = i + 1; k < 6; ++k) t -= sL[j][6 * k + i] * v[k];
-        v[i] = t;
-      }
-#pragma unroll
-      for (int i = 0; i < 6; ++i) z[6 * int64_t(dn.c0) + k0 + 6 * j + i] = v[i];
+  for (int i = 0; i < kPW * kPW / kThreads; ++i) {
+    const int e = tid + kThreads * i;
+    Tg[e] = tinv(e / kPW, e % kPW);
+  }
+  if (tid < np) {
+    const int64_t at = 6 * int64_t(dn.c0) + k0 + tid;
+    f.piv_d[at] = xd[tid];
+    f.piv_r[at] = xr[tid];
+    if (root) {  // z_P = D^+ L_PP^-1 b_P
+      double y = 0.0;
+      for (int t = 0; t <= tid; ++t) y += tinv(t, tid) * xb[t];
+      z[at] = y * xr[tid];
     }
   }
 }
@@ -1099,12 +1094,10 @@ __global__ void __launch_bounds__(kThreads)
     k_mf_diag0(DevFactor f, const int32_t* __restrict__ nodes, DevScalars* sc, double* __restrict__ z) {
   const int X = nodes[blockIdx.x];
   const int F = 6 * f.sn_nf[X], K = 6 * f.sn_nc[X];
-  __shared__ double D[kPW][kPW + 1], Wd[kPW][kPW + 1], sL[kPanelBlocks][42], sdi[kPanelBlocks][6];
-  factor_panel_diag(f, diag_node(f, X), f.front + f.sn_off[X], F, 0, min(K, kPW), sc, D, Wd, sL,
-                    sdi, false, z);
+  __shared__ double D[kPW][kPW + 1], Xs[kDiagScratch], T[kPW][kPW + 1];
+  factor_panel_diag(f, diag_node(f, X), f.front + f.sn_off[X], F, 0, min(K, kPW), sc, D, Xs, T,
+                    false, z);
 }
-
-typedef double mfma_d4 __attribute__((ext_vector_type(4)));
 
 // Position in the parent's front of row u of node X's update matrix (front row K + u):
 // update row block b is the parent's row block upos[b].
@@ -1230,7 +1223,7 @@ __device__ __forceinline__ void extend_tile_hand(const DevFactor& f, int X, int 
 __device__ __forceinline__ void panel_rows_out(const DevFactor& f, const DiagNode& dn, int P, int X,
                                                int F, int K, int k0, int np, int r0,
                                                const mfma_d4 (&L4)[3], const double (*sT)[kPW + 1],
-                                               const double* sb, const double (*pM)[36],
+                                               const double* sb, const double* sR,
                                                const double* bt, double* sy, double* __restrict__ z,
                                                int lane, bool zp) {
   const int lr = lane & 15, lc = lane >> 4;
@@ -1275,22 +1268,16 @@ __device__ __forceinline__ void panel_rows_out(const DevFactor& f, const DiagNod
           f.usolve[f.sn_uoff[P] + parent_row(f, X, r - K)] += bt[i] - part[q];
       }
     }
-  if (zp && lane < np) {  // z_P = D^-1 y_P (blockwise M_j)
-    const int jb = lane / 6, a = lane % 6;
-    double zz = 0.0;
-#pragma unroll
-    for (int t = 0; t < 6; ++t) zz += pM[jb][6 * a + t] * sy[6 * jb + t];
-    z[6 * int64_t(dn.c0) + k0 + lane] = zz;
-  }
+  if (zp && lane < np) z[6 * int64_t(dn.c0) + k0 + lane] = sy[lane] * sR[lane];  // z_P = D^+ y_P
 }
 
 // One round of panel steps, one workgroup per item (node, panel, tr, tc): the 64x64 tile
 // (tr, tc) of the node's lower trailing region below the panel:
 //   1. the tile's values, the panel columns of its row block tr and column block tc (C),
-//      L_PP^-T and the pivot inverses M_j are loaded (every global load first);
-//   2. W = C L_PP^-T for both blocks and L = W blockdiag(M_j) for block tr on the matrix
-//      cores (v_mfma_f64_16x16x4; each wavefront its own 16 rows of a 64-row block, so
-//      W and L need no barrier between them);
+//      L_PP^-T and the pivots' reciprocals are loaded (every global load first);
+//   2. W = C L_PP^-T for both blocks on the matrix cores (v_mfma_f64_16x16x4; each
+//      wavefront its own 16 rows of a 64-row block, so no barrier before the results
+//      replace C) and L = W D^+ for block tr;
 //   3. A -= L W^T on the matrix cores: four wavefronts x 2 x 2 tiles of 16x16, (-W) L^T so
 //      that each lane's results run down 16 rows of the column-major front, accumulators
 //      seeded with the front's values;
@@ -1342,8 +1329,7 @@ __global__ void __launch_bounds__(kThreads)
   const int rw = 16 * wv;                              // the wavefront's 16-row slice
   __shared__ double sA[kPW][kTile + 1], sB[kPW][kTile + 1];  // C^T, then L^T / W^T
   __shared__ double sT[kPW][kPW + 1];                          // L_PP^-T
-  __shared__ double pM[kPanelBlocks][36];
-  __shared__ double sL[kPanelBlocks][42], sdi[kPanelBlocks][6];
+  __shared__ double sR[kPW];  // 1 / d of the panel's pivots
   __shared__ double sb[kPW], sy[kThreads / 64][kPW];
   __shared__ double sbt[kTile];  // the output row block's rows of the right-hand side
   // the node's last panel step: its update matrix goes to the parent (-1: none)
@@ -1355,11 +1341,9 @@ __global__ void __launch_bounds__(kThreads)
   const bool hand = P >= 0 && tr == 0 && tc == 0 && f.sn_hand[X];
   bool diag = false;  // this workgroup factors the node's next diagonal block
   {
-    const int gb0 = dn.c0 + k0 / 6, nbp = np / 6;
     constexpr int kNC = kPW * kTile / kThreads, kNT = kPW * kPW / kThreads;
-    constexpr int kNM = (kPanelBlocks * 36 + kThreads - 1) / kThreads;
     static_assert(kPW * kTile % kThreads == 0 && kPW * kPW % kThreads == 0, "whole rounds");
-    double va[kNC], vb[kNC], vt[kNT], vm[kNM];
+    double va[kNC], vb[kNC], vt[kNT];
 #pragma unroll
     for (int it = 0; it < kNC; ++it) {
       const int e = tid + kThreads * it, t = e / kTile, i = e % kTile;
@@ -1368,11 +1352,7 @@ __global__ void __launch_bounds__(kThreads)
     }
 #pragma unroll
     for (int it = 0; it < kNT; ++it) vt[it] = Tg[tid + kThreads * it];
-#pragma unroll
-    for (int it = 0; it < kNM; ++it) {
-      const int e = tid + kThreads * it;
-      vm[it] = load_or_zero(f.piv_M, int64_t(36) * gb0 + e, e < kPanelBlocks * 36 && e / 36 < nbp);
-    }
+    const double vr = load_or_zero(f.piv_r, 6 * int64_t(dn.c0) + k0 + tid, tid < np);
     const double vbb = load_or_zero(bx, k0 + tid, out && tid < np);
     const double vbt = load_or_zero(bx, ro + tid - kPW, out && tid >= kPW && tid < kPW + kTile &&
                                                             ro + tid - kPW < F);
@@ -1387,12 +1367,10 @@ __global__ void __launch_bounds__(kThreads)
       const int e = tid + kThreads * it;
       sT[e / kPW][e % kPW] = vt[it];
     }
-#pragma unroll
-    for (int it = 0; it < kNM; ++it) {
-      const int e = tid + kThreads * it;
-      if (e < kPanelBlocks * 36) pM[e / 36][e % 36] = vm[it];
+    if (tid < kPW) {
+      sb[tid] = vbb;
+      sR[tid] = vr;
     }
-    if (tid < kPW) sb[tid] = vbb;
     if (tid >= kPW && tid < kPW + kTile) sbt[tid - kPW] = vbt;
   }
   __syncthreads();
@@ -1409,9 +1387,9 @@ __global__ void __launch_bounds__(kThreads)
         const int r = r0 + rb + 16 * mi + lr, c = c0 + cb + 16 * nj + lc + 4 * q;
         acc[mi][nj][q] = load_or_zero(A, int64_t(c) * F + r, r < F && c < F && r >= c);
       }
-  // W = C L_PP^-T for the wavefront's slice of both row blocks; L_PP^-T is block upper
+  // W = C L_PP^-T for the wavefront's slice of both row blocks; L_PP^-T is upper
   // triangular, so column tile ct stops at row kW[ct] (C and L_PP^-T are zero past np)
-  constexpr int kW[3] = {18, 36, 48};
+  constexpr int kW[3] = {16, 32, 48};
   mfma_d4 wa[3], wb[3];
 #pragma unroll
   for (int ct = 0; ct < 3; ++ct) wa[ct] = wb[ct] = mfma_d4{0.0, 0.0, 0.0, 0.0};
@@ -1437,57 +1415,25 @@ __global__ void __launch_bounds__(kThreads)
         }
     }
   }
-  __syncthreads();  // every wavefront is done with C
-  // W^T of both blocks (a diagonal tile's column block is its row block)
+  // L^T = D^+ W^T of the row block and W^T of the column block (a diagonal tile's is its row
+  // block's) replace C; a wavefront has read only its own slice of C, so no barrier
 #pragma unroll
-  for (int ct = 0; ct < 3; ++ct)
+  for (int ct = 0; ct < 3; ++ct) {
+    const double rd = sR[16 * ct + lr];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      sA[16 * ct + lr][rw + lc + 4 * q] = wa[ct][q];
+      sA[16 * ct + lr][rw + lc + 4 * q] = wa[ct][q] * rd;
       sB[16 * ct + lr][rw + lc + 4 * q] = dg ? wa[ct][q] : wb[ct][q];
     }
-  // L = W blockdiag(M_j) for the slice of row block tr: column tile ct meets the pivot
-  // blocks with rows [kL0[ct], kL1[ct]); the block-diagonal operand is read from the M_j
-  constexpr int kL0[3] = {0, 12, 30}, kL1[3] = {18, 36, 48};
-#pragma unroll
-  for (int ct = 0; ct < 3; ++ct) wa[ct] = mfma_d4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-  for (int k4 = 0; k4 < kPW; k4 += 4) {
-    const int k = k4 + lc;
-    const double av = sA[k][rw + lr];
-#pragma unroll
-    for (int ct = 0; ct < 3; ++ct)
-      if (k4 + 4 > kL0[ct] && k4 < kL1[ct]) {
-        const int n = 16 * ct + lr;
-        const double mv = k / 6 == n / 6 ? pM[k / 6][6 * (k % 6) + n % 6] : 0.0;
-        wa[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, mv, wa[ct], 0, 0, 0);
-      }
   }
   if (own0) {
-    // row block 0's outputs, from L of the block (the column block's W times the M_j) in
+    // row block 0's outputs, from L of the block (the column block's W times 1 / d) in
     // registers: component q of wb[ct] is L row rw + lc + 4 q, column 16 ct + lr
 #pragma unroll
-    for (int ct = 0; ct < 3; ++ct) wb[ct] = mfma_d4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-    for (int k4 = 0; k4 < kPW; k4 += 4) {
-      const int k = k4 + lc;
-      const double av = sB[k][rw + lr];
-#pragma unroll
-      for (int ct = 0; ct < 3; ++ct)
-        if (k4 + 4 > kL0[ct] && k4 < kL1[ct]) {
-          const int n = 16 * ct + lr;
-          const double mv = k / 6 == n / 6 ? pM[k / 6][6 * (k % 6) + n % 6] : 0.0;
-          wb[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, mv, wb[ct], 0, 0, 0);
-        }
-    }
-    panel_rows_out(f, dn, P, X, F, K, k0, np, ro + rw, wb, sT, sb, pM, sbt + rw, sy[wv], z,
+    for (int ct = 0; ct < 3; ++ct) wb[ct] *= sR[16 * ct + lr];
+    panel_rows_out(f, dn, P, X, F, K, k0, np, ro + rw, wb, sT, sb, sR, sbt + rw, sy[wv], z,
                    lane, wv == 0);
   }
-  // L^T replaces the slice's W^T in sA
-#pragma unroll
-  for (int ct = 0; ct < 3; ++ct)
-#pragma unroll
-    for (int q = 0; q < 4; ++q) sA[16 * ct + lr][rw + lc + 4 * q] = wa[ct][q];
   __syncthreads();  // the update reads every row of L^T and W^T
 #pragma unroll
   for (int s = 0; s < kPW / 4; ++s) {
@@ -1556,19 +1502,15 @@ __global__ void __launch_bounds__(kThreads)
           f.usolve[f.sn_uoff[P] + parent_row(f, X, r - K)] += sbt[i] - s4;
       }
     }
-    if (ro == kend && wv == 0 && lane < np) {  // row block 0: z_P = D^-1 y_P (blockwise M_j)
-      const int jb = lane / 6, a = lane % 6;
-      double zz = 0.0;
-#pragma unroll
-      for (int t = 0; t < 6; ++t) zz += pM[jb][6 * a + t] * sy[0][6 * jb + t];
-      z[6 * int64_t(dn.c0) + k0 + lane] = zz;
-    }
+    // row block 0: z_P = D^+ y_P
+    if (ro == kend && wv == 0 && lane < np)
+      z[6 * int64_t(dn.c0) + k0 + lane] = sy[0][lane] * sR[lane];
   }
   if (tr == 0 && tc == 0 && kend < K) {
     // the next panel's diagonal block is the top-left of this tile: hand the updated
     // values to LDS directly
     const int npn = min(K, kend + kPW) - kend;
-    double (*D)[kPW + 1] = as_square(sA);
+    double (*D)[kPW + 1] = as_square(sB);
     __syncthreads();  // every read of sA / sB is done
 #pragma unroll
     for (int mi = 0; mi < 2; ++mi)
@@ -1579,16 +1521,13 @@ __global__ void __launch_bounds__(kThreads)
           const int rl = rb + 16 * mi + lr, cl = cb + 16 * nj + lc + 4 * q;
           if (rl < npn && cl < npn) D[rl][cl] = rl >= cl ? acc[mi][nj][q] : 0.0;
         }
-    __syncthreads();
     diag = true;
   }
-  if (diag) {
-    factor_panel_diag(f, dn, A, F, kend, min(K, kend + kPW) - kend, sc, as_square(sA),
-                      as_square(sB), sL, sdi, true, z);
-  } else if (hand) {
-    __syncthreads();  // the work above that reads sA is done
-    factor_panel_diag(f, diag_node(f, P), f.front + f.sn_off[P], 6 * f.sn_nf[P], 0,
-                      min(6 * f.sn_nc[P], kPW), sc, as_square(sB), as_square(sA), sL, sdi, true, z);
+  if (diag || hand) {
+    __syncthreads();  // the block is in sB; the work above that reads sA is done
+    const int Y = diag ? X : P, kd = diag ? kend : 0;
+    factor_panel_diag(f, diag_node(f, Y), f.front + f.sn_off[Y], 6 * f.sn_nf[Y], kd,
+                      min(6 * f.sn_nc[Y] - kd, kPW), sc, as_square(sB), &sA[0][0], sT, true, z);
   }
 }
 
@@ -1597,10 +1536,9 @@ __global__ void __launch_bounds__(kThreads)
 // matrix-core time than the extra launch costs).
 //
 // Panel rows of one round of panel steps (items = (node, panel, kPanelRows-row chunk)
-// below the panel's diagonal block), as two products instead of a substitution:
-//   W_r = C_r L_PP^-T            (the rows' values after the panel's own eliminations)
-//   L_r,j = W_r,j M_j,  M_j = L_jj^-T D_j^-1 L_jj^-1
-// with L_PP^-T from the diagonal factorization.  Both run on the matrix cores as 4 x 3
+// below the panel's diagonal block), as a product instead of a substitution:
+//   W_r = C_r L_PP^-T   (the rows' values after the panel's own eliminations),  L_r = W_r D^+
+// with L_PP^-T from the diagonal factorization.  It runs on the matrix cores as 4 x 3
 // tiles of v_mfma_f64_16x16x4, three per wavefront.  W goes to the node's W scratch, L to
 // the factor and, for the node's own rows, to its row-major copy.
 __global__ void __launch_bounds__(kThreads)
@@ -1621,14 +1559,12 @@ __global__ void __launch_bounds__(kThreads)
   __shared__ double sC[kPW][kPanelRows + 1];  // the rows' panel columns, C^T
   __shared__ double sT[kPW][kPW + 1];         // L_PP^-T
   __shared__ double sW[kPanelRows][kPW + 1];
-  __shared__ double pM[kPanelBlocks][36];
+  __shared__ double sR[kPW];  // 1 / d of the panel's pivots
   __shared__ double sb[kPW], sy[kThreads / 64][kPW];  // the panel's RHS; y_P per wavefront
   double* bx = f.usolve + f.sn_uoff[X];  // the node's right-hand side (front row order)
-  const int gb0 = f.sn_c0[X] + k0 / 6, nbp = np / 6;
   // every global load of the thread first, then the LDS stores
   constexpr int kNC = kPW * kPanelRows / kThreads, kNT = kPW * kPW / kThreads;
-  constexpr int kNM = (kPanelBlocks * 36 + kThreads - 1) / kThreads;
-  double vc[kNC], vt[kNT], vm[kNM];
+  double vc[kNC], vt[kNT];
 #pragma unroll
   for (int it = 0; it < kNC; ++it) {
     const int e = tid + kThreads * it, t = e / kPanelRows, r = rbase + e % kPanelRows;
@@ -1636,11 +1572,7 @@ __global__ void __launch_bounds__(kThreads)
   }
 #pragma unroll
   for (int it = 0; it < kNT; ++it) vt[it] = Tg[tid + kThreads * it];
-#pragma unroll
-  for (int it = 0; it < kNM; ++it) {
-    const int e = tid + kThreads * it;
-    vm[it] = load_or_zero(f.piv_M, int64_t(36) * gb0 + e, e < kPanelBlocks * 36 && e / 36 < nbp);
-  }
+  const double vr = load_or_zero(f.piv_r, 6 * int64_t(f.sn_c0[X]) + k0 + tid, tid < np);
   const double vb = load_or_zero(bx, k0 + tid, tid < np);
 #pragma unroll
   for (int it = 0; it < kNC; ++it) {
@@ -1652,12 +1584,10 @@ __global__ void __launch_bounds__(kThreads)
     const int e = tid + kThreads * it;
     sT[e / kPW][e % kPW] = vt[it];
   }
-#pragma unroll
-  for (int it = 0; it < kNM; ++it) {
-    const int e = tid + kThreads * it;
-    if (e < kPanelBlocks * 36) pM[e / 36][e % 36] = vm[it];
+  if (tid < kPW) {
+    sb[tid] = vb;
+    sR[tid] = vr;
   }
-  if (tid < kPW) sb[tid] = vb;
   __syncthreads();
   // forward elimination of the right-hand side: y_P = L_PP^-1 b_P (each wavefront forms
   // its own copy; lane c < kPW entry c), and z_P = D^-1 y_P to the solve vector
@@ -1667,18 +1597,13 @@ __global__ void __launch_bounds__(kThreads)
     for (int t = 0; t < kPW; ++t) a4[t & 3] += sT[t][lane] * sb[t];  // L_PP^-T (t, c) = L_PP^-1 (c, t)
     sy[wv][lane] = (a4[0] + a4[1]) + (a4[2] + a4[3]);
   }
-  if (chunk == 0 && wv == 0 && lane < np) {
-    const int jb = lane / 6, a = lane % 6;
-    double zz = 0.0;
-#pragma unroll
-    for (int t = 0; t < 6; ++t) zz += pM[jb][6 * a + t] * sy[0][6 * jb + t];
-    z[6 * int64_t(f.sn_c0[X]) + k0 + lane] = zz;
-  }
+  if (chunk == 0 && wv == 0 && lane < np)
+    z[6 * int64_t(f.sn_c0[X]) + k0 + lane] = sy[0][lane] * sR[lane];
   // Wavefront wv owns row tile wv (16 rows) and its three 16-column tiles; it reads only
   // its own rows of C, W and L after the barrier above, so it needs no further barrier.
-  // W = C L_PP^-T: L_PP^-T is block upper triangular, so column tile ct stops at row
+  // W = C L_PP^-T: L_PP^-T is upper triangular, so column tile ct stops at row
   // kW[ct] (C and L_PP^-T are zero past np).
-  constexpr int kW[3] = {18, 36, 48};
+  constexpr int kW[3] = {16, 32, 48};
   const int rw = 16 * wv;
   mfma_d4 acc[3];
 #pragma unroll
@@ -1691,32 +1616,16 @@ __global__ void __launch_bounds__(kThreads)
       if (k4 < kW[ct])
         acc[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, sT[k4 + lk][16 * ct + lr], acc[ct], 0, 0, 0);
   }
+  // W, and L^T = D^+ W^T into this wavefront's columns of sC
 #pragma unroll
-  for (int ct = 0; ct < 3; ++ct)
+  for (int ct = 0; ct < 3; ++ct) {
+    const double rd = sR[16 * ct + lr];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) sW[rw + lk + 4 * q][16 * ct + lr] = acc[ct][q];
-  // L = W blockdiag(M_j): column tile ct meets the pivot blocks with rows
-  // [kL0[ct], kL1[ct]); the block-diagonal operand is read from the M_j directly
-  constexpr int kL0[3] = {0, 12, 30}, kL1[3] = {18, 36, 48};
-#pragma unroll
-  for (int ct = 0; ct < 3; ++ct) acc[ct] = mfma_d4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-  for (int k4 = 0; k4 < kPW; k4 += 4) {
-    const int k = k4 + lk;
-    const double av = sW[rw + lr][k];
-#pragma unroll
-    for (int ct = 0; ct < 3; ++ct)
-      if (k4 + 4 > kL0[ct] && k4 < kL1[ct]) {
-        const int n = 16 * ct + lr;
-        const double bv = k / 6 == n / 6 ? pM[k / 6][6 * (k % 6) + n % 6] : 0.0;
-        acc[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv, acc[ct], 0, 0, 0);
-      }
+    for (int q = 0; q < 4; ++q) {
+      sW[rw + lk + 4 * q][16 * ct + lr] = acc[ct][q];
+      sC[16 * ct + lr][rw + lk + 4 * q] = acc[ct][q] * rd;
+    }
   }
-  // L^T into this wavefront's columns of sC
-#pragma unroll
-  for (int ct = 0; ct < 3; ++ct)
-#pragma unroll
-    for (int q = 0; q < 4; ++q) sC[16 * ct + lr][rw + lk + 4 * q] = acc[ct][q];
   // the right-hand side of the wavefront's 16 rows: b_r -= L_r y_P (four lanes per row,
   // every fourth column, combined by two xor shuffles)
   {
@@ -1780,7 +1689,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
   const int lr = lane & 15, lc = lane >> 4;
   const int rb = 32 * (wv >> 1), cb = 32 * (wv & 1);  // the wavefront's quadrant
   __shared__ double sA[kPW][kTile + 1], sB[kPW][kTile + 1];
-  __shared__ double sL[kPanelBlocks][42], sdi[kPanelBlocks][6];
+  __shared__ double sT[kPW][kPW + 1];
   // the node's last panel step: its update matrix goes to the parent (-1: none)
   const int P = kend == K ? f.sn_parent[X] : -1;
   // the last child of its parent (in round order) factors the parent's first diagonal
@@ -1850,7 +1759,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
     // the next panel's diagonal block is the top-left of this tile: hand the updated
     // values to LDS directly
     const int npn = min(K, kend + kPW) - kend;
-    double (*D)[kPW + 1] = as_square(sA);
+    double (*D)[kPW + 1] = as_square(sB);
     __syncthreads();  // every MFMA operand read of sA / sB is done
 #pragma unroll
     for (int mi = 0; mi < 2; ++mi)
@@ -1861,16 +1770,13 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
           const int rl = rb + 16 * mi + lr, cl = cb + 16 * nj + lc + 4 * q;
           if (rl < npn && cl < npn) D[rl][cl] = rl >= cl ? acc[mi][nj][q] : 0.0;
         }
-    __syncthreads();
     diag = true;
   }
-  if (diag) {
-    factor_panel_diag(f, dn, A, F, kend, min(K, kend + kPW) - kend, sc, as_square(sA),
-                      as_square(sB), sL, sdi, true, z);
-  } else if (hand) {
-    __syncthreads();  // the work above that reads sA is done
-    factor_panel_diag(f, diag_node(f, P), f.front + f.sn_off[P], 6 * f.sn_nf[P], 0,
-                      min(6 * f.sn_nc[P], kPW), sc, as_square(sB), as_square(sA), sL, sdi, true, z);
+  if (diag || hand) {
+    __syncthreads();  // the block is in sB; the work above that reads sA is done
+    const int Y = diag ? X : P, kd = diag ? kend : 0;
+    factor_panel_diag(f, diag_node(f, Y), f.front + f.sn_off[Y], 6 * f.sn_nf[Y], kd,
+                      min(6 * f.sn_nc[Y] - kd, kPW), sc, as_square(sB), &sA[0][0], sT, true, z);
   }
 }
 
@@ -2001,7 +1907,7 @@ __global__ void __launch_bounds__(kTriMax)
 // Forward solve of one level's nodes (one workgroup each) for a right-hand side already in
 // the nodes' front row order: first the children's finished update rows are added into the
 // node's (children one after another, so the adds are plain), then panel by panel y_P =
-// L_PP^-1 b_P (the stored L_PP^-T), z_P = blockdiag(M_j) y_P and b_r -= L_r y_P for every
+// L_PP^-1 b_P (the stored L_PP^-T), z_P = D^+ y_P and b_r -= L_r y_P for every
 // row below the panel, the same eliminations the factorization applies to the step's own
 // right-hand side.
 __global__ void __launch_bounds__(kThreads)
@@ -2033,12 +1939,8 @@ __global__ void __launch_bounds__(kThreads)
     }
     __syncthreads();
     if (tid < np) {
-      const int jb = tid / 6, a = tid % 6;
-      const double* M = f.piv_M + 36 * int64_t(f.sn_c0[X] + k0 / 6 + jb);
-      double zz = 0.0;
-#pragma unroll
-      for (int t = 0; t < 6; ++t) zz += M[6 * a + t] * sy[6 * jb + t];
-      z[6 * int64_t(c0) + k0 + tid] = zz;
+      const int64_t at = 6 * int64_t(c0) + k0 + tid;
+      z[at] = sy[tid] * f.piv_r[at];
     }
     for (int r = k0 + np + tid; r < F; r += blockDim.x) {
       double acc = 0.0;

@@ -110,9 +110,8 @@ struct DevFactor {
   const int64_t* sn_toff;
   double* front;   // all fronts, column-major (workspace)
   double* lbuf;    // per node F x K: the factor's L columns (column-major, ld F)
-  double* piv_L;   // nb x 36 unit-lower pivot factors (row-major)
   double* piv_d;   // nb x 6
-  double* piv_M;   // nb x 36: (L_jj D_j L_jj^T)^+ = L_jj^-T D_j^-1 L_jj^-1 (0 rows for zero pivots)
+  double* piv_r;   // nb x 6: 1 / piv_d, 0 for a zero pivot
   int64_t front_elems;
   const Symbolic* host;  // launch schedule
   const int32_t* sn_child_ptr;  // children of each node (standalone forward solve; may be null

@@ -376,9 +376,8 @@ struct sgpu_optimizer {
       df.tinv = arena.alloc<double>(size_t(S.p_elems));
       df.wbuf = arena.alloc<double>(size_t(S.w_elems));
     }
-    df.piv_L = arena.alloc<double>(size_t(36) * S.nb);
     df.piv_d = arena.alloc<double>(size_t(6) * S.nb);
-    df.piv_M = arena.alloc<double>(size_t(36) * S.nb);
+    df.piv_r = arena.alloc<double>(size_t(6) * S.nb);
     df.front_elems = S.front_elems;
     df.host = &S;
     // workspace
@@ -618,13 +617,13 @@ struct sgpu_optimizer {
   // ---- inverse blocks (SchurFactor::inverse_block, schur_ldlt.rs:814-958) ----------------
   // The matrix is the damped Hessian of build_solution's final linearization at the current
   // variables (nu = 0, or the current nu with skip_final_hessian), as DampedHessian holds it
-  // (damped_hessian.rs:98).  S is factored with the direct solver's kernels, S = L B L^T with
-  // B = blockdiag(L_jj diag(d) L_jj^T).  Like the reference's min-norm LDLt
+  // (damped_hessian.rs:98).  S is factored with the direct solver's kernels, S = L diag(d) L^T
+  // with unit lower L.  Like the reference's min-norm LDLt
   // (block_sparse_min_norm_ldlt.rs:63-88), only positive pivots span the range: with S' = S
-  // minus the non-positive pivots' terms, S'^+ b = P S'^- P b where S'^- = L^-T M' L^-1,
-  // M'_j = L_jj^-T diag(d+)^-1 L_jj^-1 (non-positive pivots give 0), and P projects off the
-  // null space of S', spanned by n = L^-T (L_jj^-T e_c) for each non-positive pivot c of
-  // block j (S' n = 0).  This is the Moore-Penrose inverse the reference forms from E and G.
+  // minus the non-positive pivots' terms, S'^+ b = P S'^- P b where S'^- = L^-T diag(d+)^-1 L^-1
+  // (non-positive pivots give 0), and P projects off the null space of S', spanned by
+  // n = L^-T e_i for each non-positive pivot i (S' n = 0).  This is the Moore-Penrose inverse
+  // the reference forms from E and G.
   void ensure_cov() {
     if (cov_ready) return;
     if (iterative()) throw Error(SGPU_ERR_UNSUPPORTED, "inverse blocks need the direct RCS solver");
@@ -647,10 +646,9 @@ struct sgpu_optimizer {
     launch_gather_s_diag(stream, dp, df.front, cov_sdiag);
     launch_rcs_factor(stream, df, d_sc, dl.rhs_nat, dl.x_perm);
     SGPU_HIP(hipMemcpyAsync(h_sc, d_sc, sizeof(DevScalars), hipMemcpyDeviceToHost, stream));
-    std::vector<double> d(n), Lp(size_t(6) * n), sdiag(n);
+    std::vector<double> d(n), sdiag(n);
     SGPU_HIP(hipMemcpyAsync(d.data(), df.piv_d, n * 8, hipMemcpyDeviceToHost, stream));
     SGPU_HIP(hipMemcpyAsync(sdiag.data(), cov_sdiag, n * 8, hipMemcpyDeviceToHost, stream));
-    SGPU_HIP(hipMemcpyAsync(Lp.data(), df.piv_L, size_t(6) * n * 8, hipMemcpyDeviceToHost, stream));
     SGPU_HIP(hipStreamSynchronize(stream));
     if (h_sc->singular_marg) throw Error(SGPU_ERR_NON_FINITE, "singular marginal block in the final Hessian");
     if (h_sc->bad_pivot) throw Error(SGPU_ERR_NON_FINITE, "non-finite pivot in the final Hessian");
@@ -665,50 +663,30 @@ struct sgpu_optimizer {
       cov_pivot_ratio = std::isfinite(lo) ? lo : 0.0;
     }
     std::vector<double> e(n), v(n);
-    for (int64_t gb = 0; gb < S.nb; ++gb) {
-      bool any = false;
-      for (int c = 0; c < 6; ++c) any = any || !(d[6 * gb + c] > 0.0);
-      if (!any) continue;
-      // Li = L_jj^-1 (unit lower, row-major) by forward substitution
-      const double* Lj = &Lp[36 * gb];
-      double Li[36];
-      for (int c = 0; c < 6; ++c)
-        for (int r = 0; r < 6; ++r) {
-          double x = r == c ? 1.0 : 0.0;
-          for (int t = c; t < r; ++t) x -= Lj[6 * r + t] * Li[6 * t + c];
-          Li[6 * r + c] = r < c ? 0.0 : x;
-        }
-      double Mj[36];  // L_jj^-T diag(1/d+) L_jj^-1
-      for (int a = 0; a < 6; ++a)
-        for (int b = 0; b < 6; ++b) {
-          double acc = 0.0;
-          for (int k = 0; k < 6; ++k) {
-            const double dk = d[6 * gb + k];
-            if (dk > 0.0) acc += Li[6 * k + a] * (1.0 / dk) * Li[6 * k + b];
-          }
-          Mj[6 * a + b] = acc;
-        }
-      SGPU_HIP(hipMemcpyAsync(df.piv_M + 36 * gb, Mj, 36 * 8, hipMemcpyHostToDevice, stream));
-      for (int c = 0; c < 6; ++c) {
-        if (d[6 * gb + c] > 0.0) continue;
-        std::fill(e.begin(), e.end(), 0.0);
-        for (int r = 0; r < 6; ++r) e[6 * gb + r] = Li[6 * c + r];  // L_jj^-T e_c
-        SGPU_HIP(hipMemcpyAsync(cov_z, e.data(), n * 8, hipMemcpyHostToDevice, stream));
-        launch_rcs_solve(stream, df, cov_z, cov_x);
-        SGPU_HIP(hipMemcpyAsync(v.data(), cov_x, n * 8, hipMemcpyDeviceToHost, stream));
-        SGPU_HIP(hipStreamSynchronize(stream));
-        for (const auto& q : cov_null) {  // Gram-Schmidt against the earlier ones
-          double dot = 0.0;
-          for (int64_t i = 0; i < n; ++i) dot += q[i] * v[i];
-          for (int64_t i = 0; i < n; ++i) v[i] -= dot * q[i];
-        }
-        double nrm = 0.0;
-        for (double x : v) nrm += x * x;
-        nrm = std::sqrt(nrm);
-        if (nrm > 0.0) {
-          for (double& x : v) x /= nrm;
-          cov_null.push_back(v);
-        }
+    const double zero = 0.0;
+    for (int64_t i = 0; i < n; ++i) {
+      if (d[i] > 0.0) continue;
+      SGPU_HIP(hipMemcpyAsync(df.piv_r + i, &zero, 8, hipMemcpyHostToDevice, stream));
+    }
+    for (int64_t i = 0; i < n; ++i) {
+      if (d[i] > 0.0) continue;
+      std::fill(e.begin(), e.end(), 0.0);
+      e[i] = 1.0;
+      SGPU_HIP(hipMemcpyAsync(cov_z, e.data(), n * 8, hipMemcpyHostToDevice, stream));
+      launch_rcs_solve(stream, df, cov_z, cov_x);
+      SGPU_HIP(hipMemcpyAsync(v.data(), cov_x, n * 8, hipMemcpyDeviceToHost, stream));
+      SGPU_HIP(hipStreamSynchronize(stream));
+      for (const auto& q : cov_null) {  // Gram-Schmidt against the earlier ones
+        double dot = 0.0;
+        for (int64_t r = 0; r < n; ++r) dot += q[r] * v[r];
+        for (int64_t r = 0; r < n; ++r) v[r] -= dot * q[r];
+      }
+      double nrm = 0.0;
+      for (double x : v) nrm += x * x;
+      nrm = std::sqrt(nrm);
+      if (nrm > 0.0) {
+        for (double& x : v) x /= nrm;
+        cov_null.push_back(v);
       }
     }
     SGPU_HIP(hipStreamSynchronize(stream));
