@@ -2,17 +2,30 @@
 //
 // Every window (one shared pinhole, SE(3) poses with pose 0 constant, marginalized
 // points, Huber reprojection terms) has at most kBatchMaxCams cameras, so its reduced
-// camera system (n = 6 (cameras - 1) <= 180) lives in LDS as a packed lower triangle.
+// camera system (n = 6 (cameras - 1) <= 180) lives in LDS as a packed lower triangle, its
+// right-hand side as one more row.
 // One workgroup runs one complete LM iteration of one window:
-//   per point (threads): A_o, M_o = A^T A, H_ll + nu n I, H_ll^-1, s, y; the point's
-//     Schur terms go into S with LDS atomics (diagonal own term M H^-1 (H - M),
-//     off-diagonal -M_i H^-1 M_j, lifted by P = [hat(-x) | I]), rhs, gradient;
-//   dense block LDLt of S in LDS (6x6 pivots, the reference's PSD rule), solves;
+//   per point (threads): M_o = A^T A of its observations, H_ll + nu n I, H_ll^-1, s;
+//   per camera (16 lanes): the own terms M H^-1 (H - M) of its observations, rhs and
+//     gradient, summed in registers;
+//   per segment of at most 8 points that two cameras share (threads): the cross terms
+//     -M_i H^-1 M_j, lifted by P = [hat(-x) | I] and summed in registers, into S with
+//     LDS atomics;
+//   dense LDLt of S in LDS (the reference's rule on each 6x6 pivot block), solves;
 //   back-substitution, T <- exp(delta) T, merit of the proposal (FP64), and the LM
 //   decision with the same rules and check order as the single-problem optimizer.
 // One launch advances every unfinished window by one iteration; the host captures a
 // sequence of launches in a hipGraph.  Precision T = float computes the Jacobians and
 // Schur products in FP32 (S, the factorization, the merit and the decisions stay FP64).
+//
+// An iteration is bound by the latency of dependent LDS and FP64 steps, its data (0.2 MB a
+// window) lies in L2.  Cycles of one iteration of a window of 9 cameras and 5300 observations
+// at 512 threads: points 57k, own terms 99k, cross terms 139k (a thread per point that added
+// all its terms to S with LDS atomics, 36 a pair at about 40 cycles a wavefront: 621k to
+// 668k for the three); factor 71k in panels of 12 columns (258k to 544k with one thread per 6x6
+// pivot); solves 18k, back-substitution 33k, merit 27k (57k with a search for the point of
+// each observation).  24 windows of 6 to 31 cameras, 20 persistent iterations: 16.1 -> 5.55 ms;
+// 1000 windows of 6 to 11 cameras, FP32 products, 10 launches: 33.8 -> 12.2 ms.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -24,11 +37,14 @@
 
 #include "api_internal.hpp"
 #include "block6.hpp"
+#include "eliminate.hpp"
 #include "lie.hpp"
 
 namespace sgpu {
 
 constexpr int kBatchMaxCams = 31;
+constexpr int kRec = 21;     // doubles of a point's record
+constexpr int kSegment = 8;  // most pairs of a segment
 
 struct BatchDev {
   int32_t nprob;
@@ -44,10 +60,20 @@ struct BatchDev {
   const int32_t* obs_cam;    // camera within the problem, sorted by point
   const double* obs_uv;
   const int32_t* pt_obs;     // global point -> first observation (npt_total + 1)
+  const int32_t* obs_pt;     // observation -> point within the problem
+  const int32_t* cam_pt;     // observations camera by camera: their point within the problem
+  const double* cam_uv;      // and uv
+  const int32_t* cam_ptr;    // camera -> its first entry of those (prefix)
+  const int32_t* seg;        // (camera block i, block j < i, first pair in the problem, pairs)
+  const int32_t* seg_ptr;    // problem -> first segment (prefix, nprob + 1)
+  const int64_t* pair_ptr;   // problem -> its first pair (prefix, nprob + 1)
+  const int32_t* pair_pt;    // point within the problem of each pair
+  const int32_t* same;       // an observation per pair of observations of a point by one camera
+  const int32_t* same_ptr;   // problem -> first entry of same (prefix, nprob + 1)
   const int32_t* pt_nu;      // reduced terms per point
   const int32_t* cam_nu;     // reduced terms per camera
-  double* hinv;              // 9 per point
-  double* pts;               // 3 per point (the point's neg-gradient s)
+  double* rec;               // kRec per point: x, H_ll^-1 (all 9: its triangles differ by rounding), damped
+                             // H_ll upper (00, 01, 02, 11, 12, 22), neg-gradient s
   // per-problem LM state
   int32_t* cur;
   double* nu;
@@ -70,7 +96,9 @@ struct BatchDev {
 
 namespace {
 
-__host__ __device__ __forceinline__ int64_t pk(int r, int c) { return int64_t(r) * (r + 1) / 2 + c; }  // r >= c
+__host__ __device__ __forceinline__ int pk(int r, int c) {  // r >= c
+  return int((unsigned(r) * unsigned(r + 1)) >> 1) + c;
+}
 
 template <int NT>
 __device__ double wg_sum(double v, double* red) {
@@ -134,6 +162,35 @@ __device__ __forceinline__ void obs_eval(const double* cc, const double* K, cons
   }
 }
 
+// The Jacobian's Gram matrix of a point in one camera.
+template <typename T>
+__device__ __forceinline__ void obs_gram(const double* cc, const double* K, const double x[3], T M[9]) {
+  const double uv[2] = {0.0, 0.0};
+  double r[2];
+  T A[6];
+  obs_eval<T>(cc, K, uv, x, r, A);
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int j = 0; j < 3; ++j) M[3 * i + j] = A[i] * A[j] + A[3 + i] * A[3 + j];
+}
+
+// v + v of the lane that the DPP control kCtrl selects.
+template <int kCtrl>
+__device__ __forceinline__ double dpp_add(double v) {
+  const int2 b = __builtin_bit_cast(int2, v);
+  return v + __builtin_bit_cast(double, make_int2(__builtin_amdgcn_mov_dpp(b.x, kCtrl, 0xf, 0xf, true),
+                                                  __builtin_amdgcn_mov_dpp(b.y, kCtrl, 0xf, 0xf, true)));
+}
+
+// Sum over each 16 consecutive lanes, in all of them.
+__device__ __forceinline__ double row_sum(double v) {
+  v = dpp_add<0xb1>(v);     // quad_perm [1, 0, 3, 2]
+  v = dpp_add<0x4e>(v);     // quad_perm [2, 3, 0, 1]
+  v = dpp_add<0x124>(v);    // row_ror:4
+  return dpp_add<0x128>(v);  // row_ror:8
+}
+
 template <typename T>
 __device__ __forceinline__ void gram3(const T A[6], T M[9]) {
 #pragma unroll
@@ -150,55 +207,337 @@ __device__ __forceinline__ void mul3(const T* A, const T* B, T* C) {
     for (int j = 0; j < 3; ++j) C[3 * i + j] = A[3 * i] * B[j] + A[3 * i + 1] * B[3 + j] + A[3 * i + 2] * B[6 + j];
 }
 
-// S(ci, cj) += sign * P_i^T N P_j (P = [hat(-x) | I], the same point x), lower packed,
-// block row ci >= block column cj.
-template <typename T>
-__device__ void lift_add(double* S, int ci, int cj, const T x[3], const T N[9], double sign) {
+// u v - w t with the rounding fixed: w t rounded first, u v rounded first, or both.
+__device__ __forceinline__ float fma_t(float a, float b, float c) { return fmaf(a, b, c); }
+__device__ __forceinline__ double fma_t(double a, double b, double c) { return fma(a, b, c); }
+template <int kRounded, typename T>
+__device__ __forceinline__ T cross(T u, T v, T w, T t) {
+#pragma clang fp contract(off)
+  if constexpr (kRounded == 1) return fma_t(u, v, -(w * t));
+  if constexpr (kRounded == 2) return fma_t(-w, t, u * v);
+  return u * v - w * t;
+}
+
+// B = P^T N P (P = [hat(-x) | I]): f(a, b, B_ab) for its 36 entries. The FP32 products of a
+// mixed run are summed in FP64, and their rounding decides how a window goes on whose steps are
+// often rejected: ends differed by up to 1e-3 in such windows when only the choice of the fused
+// product was left to the compiler, which changes it with the code around. So it is written
+// down, for the own term of an observation (kOwn) and the cross terms as each has always been.
+template <bool kOwn, typename T, typename F>
+__device__ __forceinline__ void lift(const T x[3], const T N[9], F f) {
   T HN[9], NHt[9], HNHt[9];
-#pragma unroll
-  for (int j = 0; j < 3; ++j) {
-    HN[j] = -x[2] * N[3 + j] + x[1] * N[6 + j];
-    HN[3 + j] = x[2] * N[j] - x[0] * N[6 + j];
-    HN[6 + j] = -x[1] * N[j] + x[0] * N[3 + j];
-  }
+  HN[0] = cross<1>(x[1], N[6], x[2], N[3]);
+  HN[1] = cross<1>(x[1], N[7], x[2], N[4]);
+  HN[2] = cross<2>(x[1], N[8], x[2], N[5]);
+  HN[3] = cross<2>(x[2], N[0], x[0], N[6]);
+  HN[4] = cross<1>(x[2], N[1], x[0], N[7]);
+  HN[5] = cross<1>(x[2], N[2], x[0], N[8]);
+  HN[6] = cross<1>(x[0], N[3], x[1], N[0]);
+  HN[7] = cross<2>(x[0], N[4], x[1], N[1]);
+  HN[8] = cross<1>(x[0], N[5], x[1], N[2]);
+  NHt[0] = cross<0>(x[1], N[2], x[2], N[1]);
+  NHt[1] = cross<2>(x[2], N[0], x[0], N[2]);
+  NHt[2] = cross<1>(x[0], N[1], x[1], N[0]);
+  NHt[3] = cross<1>(x[1], N[5], x[2], N[4]);
+  NHt[4] = cross<kOwn ? 1 : 0>(x[2], N[3], x[0], N[5]);
+  NHt[5] = cross<2>(x[0], N[4], x[1], N[3]);
+  NHt[6] = cross<2>(x[1], N[8], x[2], N[7]);
+  NHt[7] = cross<1>(x[2], N[6], x[0], N[8]);
+  NHt[8] = cross<kOwn ? 2 : 0>(x[0], N[7], x[1], N[6]);
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
-    NHt[3 * i + 0] = -N[3 * i + 1] * x[2] + N[3 * i + 2] * x[1];
-    NHt[3 * i + 1] = N[3 * i + 0] * x[2] - N[3 * i + 2] * x[0];
-    NHt[3 * i + 2] = -N[3 * i + 0] * x[1] + N[3 * i + 1] * x[0];
-    HNHt[3 * i + 0] = -HN[3 * i + 1] * x[2] + HN[3 * i + 2] * x[1];
-    HNHt[3 * i + 1] = HN[3 * i + 0] * x[2] - HN[3 * i + 2] * x[0];
-    HNHt[3 * i + 2] = -HN[3 * i + 0] * x[1] + HN[3 * i + 1] * x[0];
+    HNHt[3 * i] = cross<1>(x[1], HN[3 * i + 2], x[2], HN[3 * i + 1]);
+    HNHt[3 * i + 1] = i == 0 ? cross<2>(x[2], HN[0], x[0], HN[2])
+                             : cross<1>(x[2], HN[3 * i], x[0], HN[3 * i + 2]);
+    HNHt[3 * i + 2] = cross<1>(x[0], HN[3 * i + 1], x[1], HN[3 * i]);
   }
-  for (int a = 0; a < 6; ++a)
-    for (int b = 0; b < 6; ++b) {
-      const int r = 6 * ci + a, c = 6 * cj + b;
-      if (ci == cj && c > r) continue;  // lower triangle of a diagonal block
-      T v;
-      if (a < 3 && b < 3) v = HNHt[3 * a + b];
-      else if (a < 3) v = HN[3 * a + b - 3];
-      else if (b < 3) v = NHt[3 * (a - 3) + b];
-      else v = N[3 * (a - 3) + b - 3];
-      if (v != T(0)) atomicAdd(&S[pk(r, c)], sign * double(v));
+#pragma unroll
+  for (int a = 0; a < 3; ++a)
+#pragma unroll
+    for (int b = 0; b < 3; ++b) {
+      f(a, b, HNHt[3 * a + b]);
+      f(a, b + 3, HN[3 * a + b]);
+      f(a + 3, b, NHt[3 * a + b]);
+      f(a + 3, b + 3, N[3 * a + b]);
     }
 }
 
-__device__ __forceinline__ double sym_at(const double* S, int r, int c) {
-  return r >= c ? S[pk(r, c)] : S[pk(c, r)];
+constexpr int kPanel = 12;  // columns factored at a time: two 6x6 pivot blocks
+typedef double mfma_d4 __attribute__((ext_vector_type(4)));
+
+// eliminate_columns by the block pivot rule itself, for a panel with a pivot that it zeroes or
+// could zero later: p and q as there; false if a pivot is not finite.
+__device__ __forceinline__ bool eliminate_general(double (&p)[kPanel], double (&q)[kPanel], int w, double& dv,
+                                  double& rv) {
+  const int li = threadIdx.x & 15;
+  bool ok = true;
+  static_for<0, kPanel / 6>([&](auto blk) __attribute__((always_inline)) {
+    constexpr int b0 = 6 * blk;
+    if (b0 >= w) return;
+    double a6[36], L[36], d[6], di[6];
+    static_for<0, 6>([&](auto i) __attribute__((always_inline)) {
+      static_for<0, i + 1>([&](auto j) __attribute__((always_inline)) {
+        a6[6 * i + j] = a6[6 * j + i] = row_value<b0 + i>(p[b0 + j]);
+      });
+    });
+    if (!ldlt6(a6, L, d, di)) {
+      ok = false;
+      for (int k = 0; k < 36; ++k) L[k] = (k % 7 == 0) ? 1.0 : 0.0;
+      for (int k = 0; k < 6; ++k) d[k] = di[k] = 0.0;
+    }
+    static_for<0, 6>([&](auto i) __attribute__((always_inline)) {
+      static_for<0, i>([&](auto t) __attribute__((always_inline)) {
+        p[b0 + i] -= p[b0 + t] * L[6 * i + t];
+        q[b0 + i] -= q[b0 + t] * L[6 * i + t];
+      });
+      dv = li == b0 + i ? d[i] : dv;
+      rv = li == b0 + i ? di[i] : rv;
+    });
+    static_for<0, 6>([&](auto t) __attribute__((always_inline)) {
+      const double lp = p[b0 + t] * di[t], lq = q[b0 + t] * di[t];
+      static_for<b0 + 6, kPanel>([&](auto c) __attribute__((always_inline)) {
+        const double u = row_value<c>(p[b0 + t]);
+        p[c] -= lp * u;
+        q[c] -= lq * u;
+      });
+    });
+    // the pivot rows' own U: L_jj diag(d)
+    static_for<0, 6>([&](auto i) __attribute__((always_inline)) {
+      static_for<0, i>([&](auto t) __attribute__((always_inline)) {
+        p[b0 + t] = li == b0 + i ? L[6 * i + t] * d[t] : p[b0 + t];
+      });
+    });
+  });
+  return ok;
 }
 
-// Solve D x = v with D = L6 diag(d) L6^T stored in the packed diagonal block of k
-// (strict lower: L6, diagonal: d); zero pivots map to 0.
-__device__ void d_solve(const double* S, int k, double v[6]) {
+// LDLt of the n x n system in S (packed lower triangle) with its right-hand side as row n, in
+// place: S's columns become U = L D, row n the forward-solved right-hand side times D, rd
+// the reciprocal pivots (0 for a zero pivot).
+//
+// Panels of 12 columns.  Each wavefront repeats the panel's pivot rows and eliminates 64 of
+// the rows below in registers (eliminate_columns: no barrier or LDS access between pivots),
+// then the trailing update runs on the matrix cores in 16x16 tiles.  The bound is the chain of
+// n pivots and the tiles' LDS accesses (17 per lane and tile).
+template <int NT>
+__device__ __forceinline__ void window_ldlt(double* S, int n, double* rd, int* flags) {
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int lr = lane & 15, lc = lane >> 4;
+  for (int o = 0; o < n; o += kPanel) {
+    const int w = min(kPanel, n - o), r0 = o + w;  // rows below: r0..n (n: the right-hand side)
+    double p[kPanel], q[kPanel], dv = 1.0, rv = 0.0;
+    for (int c0 = r0 + 64 * wv; c0 <= n; c0 += NT) {
+      const int r = min(c0 + lane, n), pr = o + min(lr, w - 1);
+      auto load = [&] {
+#pragma unroll
+        for (int c = 0; c < kPanel; ++c) {
+          const int cc = o + min(c, w - 1);
+          p[c] = S[pk(max(pr, cc), min(pr, cc))];
+          q[c] = S[pk(r, cc)];
+        }
+      };
+      load();
+      eliminate_columns<kPanel>(p, q, w, dv);
+      rv = recip_nr(dv);
+      // a pivot that the rule zeroes, or would once a larger one follows it (or not finite)
+      double mx[2] = {1.0, 1.0};
+      static_for<0, kPanel>([&](auto c) __attribute__((always_inline)) {
+        mx[c / 6] = fmax(mx[c / 6], fabs(row_value<c>(dv)));
+      });
+      const double ad = fabs(dv);
+      if (__any(lr < w && !(ad > (lr < 6 ? mx[0] : mx[1]) * 1e-12 && ad < __builtin_inf()))) {
+        load();
+        if (!eliminate_general(p, q, w, dv, rv)) flags[1] = 1;
+      }
+      if (c0 + lane <= n)
+#pragma unroll
+        for (int c = 0; c < kPanel; ++c)
+          if (c < w) S[pk(r, o + c)] = q[c];
+    }
+    __syncthreads();  // every wavefront has read the pivot rows
+    if (wv == 0 && lane < w) {
+#pragma unroll
+      for (int c = 0; c < kPanel; ++c)
+        if (c < lane) S[pk(o + lane, o + c)] = p[c];
+      rd[o + lane] = rv;
+    }
+    __syncthreads();
+    // S(r, c) -= U(r, :) D^+ U(c, :)^T for r0 <= c <= r <= n, c < n
+    const int nt = (n + 1 - r0 + 15) / 16;
+    for (int t = wv; t < nt * (nt + 1) / 2; t += NT / 64) {
+      int ti = int((sqrtf(8.0f * t + 1.0f) - 1.0f) * 0.5f);
+      ti += (ti + 1) * (ti + 2) / 2 <= t;
+      ti -= ti * (ti + 1) / 2 > t;
+      const int tj = t - ti * (ti + 1) / 2;
+      const int R = r0 + 16 * ti, c = r0 + 16 * tj + lr;
+      mfma_d4 acc;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int r = R + lc + 4 * i;
+        acc[i] = S[c <= r && r <= n ? pk(r, c) : 0];
+      }
+      const int ra = min(R + lr, n), rc = min(c, n);
+#pragma unroll
+      for (int k = 0; k < kPanel; k += 4) {
+        const int kk = o + min(k + lc, w - 1);
+        const double rk = (k + lc < w ? -1.0 : 0.0) * rd[kk];  // a product, so that the load has no branch
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(rk * S[pk(ra, kk)], S[pk(rc, kk)], acc, 0, 0, 0);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int r = R + lc + 4 * i;
+        if (c <= r && r <= n && c < n) S[pk(r, c)] = acc[i];
+      }
+    }
+    __syncthreads();
+  }
+}
+
+// x = L^-T D^+ (row n of S) with the factor of window_ldlt.
+template <int NT>
+__device__ __forceinline__ void window_backsolve(const double* S, int n, const double* rd, double* x) {
+  const int tid = threadIdx.x, lr = tid & 15;
+  for (int e = tid; e < n; e += NT) x[e] = S[pk(n, e)] * rd[e];
+  __syncthreads();
+  for (int o = (n - 1) / kPanel * kPanel; o >= 0; o -= kPanel) {
+    const int w = min(kPanel, n - o), me = o + min(lr, w - 1);
+    if (tid < 64) {  // the panel's own columns, each 16 lanes alike
+      double l[kPanel], v = x[me];
+      const double rme = rd[me];
+#pragma unroll
+      for (int c = 1; c < kPanel; ++c) {  // the masks are products, so that the loads have no branches
+        const int row = o + min(c, w - 1);
+        l[c] = S[pk(row, min(me, row))] * (c < w && lr < c ? rme : 0.0);
+      }
+      static_for<0, kPanel - 1>([&](auto i) __attribute__((always_inline)) {
+        constexpr int c = kPanel - 1 - i;
+        v -= l[c] * row_value<c>(v);
+      });
+      if (tid < w) x[me] = v;
+    }
+    __syncthreads();
+    for (int r = tid; r < o; r += NT) {
+      double s[2] = {0.0, 0.0};
+      if (w == kPanel) {
+#pragma unroll
+        for (int c = 0; c < kPanel; ++c) s[c & 1] += S[pk(o + c, r)] * x[o + c];
+      } else {
+        for (int c = 0; c < w; ++c) s[0] += S[pk(o + c, r)] * x[o + c];
+      }
+      x[r] -= (s[0] + s[1]) * rd[r];
+    }
+    __syncthreads();
+  }
+}
+
+// The same system by 6x6 pivot blocks, L(:, k) = S(:, k) D_k^+ with D_k = L_6 diag(d) L_6^T
+// (stored in the packed diagonal block, strict lower L_6 and diagonal d), and its solution
+// into x.  The windows with FP32 Schur products keep this elimination: their S is near
+// singular once nu has fallen, and LM magnifies the rounding of single windows by 1e11.  Over
+// 12 batches of 1000 windows two runs of the same code differ by up to 6e-5 (norms, the
+// largest in one window; S is summed by atomics) and runs before and after the panels by no
+// more with this order, but by 7e-5 where repeated runs agree to 2e-7 with the order of
+// window_ldlt, which takes 9.9 ms for 10 iterations of such a batch instead of 12.2 ms.
+__device__ __forceinline__ void d_solve(const double* S, int k, double v[6]) {
   const int o = 6 * k;
+#pragma unroll
   for (int i = 0; i < 6; ++i)
+#pragma unroll
     for (int j = 0; j < i; ++j) v[i] -= S[pk(o + i, o + j)] * v[j];
+#pragma unroll
   for (int i = 0; i < 6; ++i) {
     const double d = S[pk(o + i, o + i)];
     v[i] = d == 0.0 ? 0.0 : v[i] / d;
   }
+#pragma unroll
   for (int i = 5; i >= 0; --i)
+#pragma unroll
     for (int j = i + 1; j < 6; ++j) v[i] -= S[pk(o + j, o + i)] * v[j];
+}
+
+template <int NT>
+__device__ __forceinline__ void window_block_solve(double* S, int n, double* W, double* x, int* flags) {
+  const int tid = threadIdx.x, nbk = n / 6;
+  for (int k = 0; k < nbk; ++k) {
+    const int o = 6 * k, m = n - o - 6;
+    if (tid == 0) {
+      double Dk[36], L6[36], dk[6];
+#pragma unroll
+      for (int a = 0; a < 6; ++a)
+#pragma unroll
+        for (int b = 0; b <= a; ++b) Dk[6 * a + b] = Dk[6 * b + a] = S[pk(o + a, o + b)];
+      if (!ldlt6(Dk, L6, dk)) {
+        flags[1] = 1;
+        for (int a = 0; a < 6; ++a) dk[a] = 0.0;
+      }
+#pragma unroll
+      for (int a = 0; a < 6; ++a) {
+#pragma unroll
+        for (int b = 0; b < a; ++b) S[pk(o + a, o + b)] = L6[6 * a + b];
+        S[pk(o + a, o + a)] = dk[a];
+      }
+    }
+    __syncthreads();
+    // W = S(:, k) below the diagonal block; L(:, k) = W D_k^+
+    for (int r = o + 6 + tid; r < n; r += NT) {
+      double v[6];
+#pragma unroll
+      for (int t = 0; t < 6; ++t) {
+        v[t] = S[pk(r, o + t)];
+        W[6 * (r - o - 6) + t] = v[t];
+      }
+      d_solve(S, k, v);
+#pragma unroll
+      for (int t = 0; t < 6; ++t) S[pk(r, o + t)] = v[t];
+    }
+    __syncthreads();
+    // trailing update S(r, c) -= L(r, k) . W(c, k) for o + 6 <= c <= r, a row's columns over as
+    // many threads as there are per row
+    const int parts = m > 0 ? NT / m : 0;
+    for (int e = tid; e < max(parts, 1) * m; e += NT) {
+      const int i = e % m, part = e / m, r = o + 6 + i;
+      double l[6];
+#pragma unroll
+      for (int t = 0; t < 6; ++t) l[t] = S[pk(r, o + t)];
+      const int per = (i + 1 + max(parts, 1) - 1) / max(parts, 1);
+      const int c1 = min((part + 1) * per, i + 1);
+#pragma unroll 4
+      for (int j = part * per; j < c1; ++j) {
+        const double* w = W + 6 * j;
+        S[pk(r, o + 6 + j)] -= l[0] * w[0] + l[1] * w[1] + l[2] * w[2] + l[3] * w[3] + l[4] * w[4] + l[5] * w[5];
+      }
+    }
+    __syncthreads();
+  }
+  for (int e = tid; e < n; e += NT) x[e] = S[pk(n, e)];
+  __syncthreads();
+  for (int k = 0; k < nbk; ++k) {
+    const int o = 6 * k;
+    for (int r = o + 6 + tid; r < n; r += NT) {
+      double s = 0.0;
+#pragma unroll
+      for (int t = 0; t < 6; ++t) s += S[pk(r, o + t)] * x[o + t];
+      x[r] -= s;
+    }
+    __syncthreads();
+  }
+  for (int k = tid; k < nbk; k += NT) {
+    double v[6];
+    for (int t = 0; t < 6; ++t) v[t] = x[6 * k + t];
+    d_solve(S, k, v);
+    for (int t = 0; t < 6; ++t) x[6 * k + t] = v[t];
+  }
+  __syncthreads();
+  for (int k = nbk - 1; k > 0; --k) {
+    const int o = 6 * k;
+    for (int r = tid; r < o; r += NT) {
+      double s = 0.0;
+#pragma unroll
+      for (int a = 0; a < 6; ++a) s += S[pk(o + a, r)] * x[o + a];
+      x[r] -= s;
+    }
+    __syncthreads();
+  }
 }
 
 // One LM iteration of unfinished window p by the whole workgroup (lds: the dynamic LDS, red
@@ -206,7 +545,7 @@ __device__ void d_solve(const double* S, int k, double v[6]) {
 // the LM decision and writes the window's state; the other threads return before it, so a
 // caller that goes on synchronizes first.
 template <typename T, int NT>
-__device__ void batch_iteration(const BatchDev& d, int p, double* lds, double* red, int* flags) {
+__device__ __forceinline__ void batch_iteration(const BatchDev& d, int p, double* lds, double* red, int* flags) {
   const int c0 = d.cam0[p], nc = d.cam0[p + 1] - c0;
   const int q0 = d.pt0[p], np = d.pt0[p + 1] - q0;
   const int o0 = d.obs0[p], no = d.obs0[p + 1] - o0;
@@ -214,22 +553,17 @@ __device__ void batch_iteration(const BatchDev& d, int p, double* lds, double* r
   const int cur = d.cur[p], nxt = 1 - cur;
   const double nu = d.nu[p];
   const double* K = d.intr + 4 * p;
-  double* S = lds;
-  double* W = S + pk(d.n_max, 0);
-  double* rhs = W + 6 * d.n_max;
-  double* grad = rhs + d.n_max;
+  double* S = lds;                    // packed, row n the right-hand side
+  double* grad = S + pk(d.n_max + 1, 0);
   double* xs = grad + d.n_max;
-  double* cams = xs + d.n_max;  // 15 per camera
+  double* rd = xs + d.n_max;          // reciprocal pivots (FP32 Schur products: 6 columns of S)
+  double* cams = rd + (std::is_same<T, double>::value ? 1 : 6) * d.n_max;  // 15 per camera
   const int tid = threadIdx.x;
   const double* poses = d.poses[cur] + 7 * int64_t(c0);
   const double* points = d.points[cur] + 3 * int64_t(q0);
   // ---- linearize + Schur -------------------------------------------------------------------
   for (int c = tid; c < nc; c += NT) cam_cache(poses + 7 * c, cams + 15 * c);
-  for (int64_t e = tid; e < pk(n, 0); e += NT) S[e] = 0.0;
-  for (int e = tid; e < n; e += NT) {
-    rhs[e] = 0.0;
-    grad[e] = 0.0;
-  }
+  for (int e = tid; e < pk(n + 1, 0); e += NT) S[e] = 0.0;
   if (tid < 4) flags[tid] = 0;
   __syncthreads();
   double gmax = 0.0;
@@ -269,154 +603,165 @@ __device__ void batch_iteration(const BatchDev& d, int p, double* lds, double* r
       Hi[7] = (H[1] * H[6] - H[7] * H[0]) / det;
       Hi[8] = (H[0] * H[4] - H[3] * H[1]) / det;
     }
-    for (int k = 0; k < 9; ++k) d.hinv[9 * int64_t(gb) + k] = Hi[k];
-    double y[3];
+    double* rec = d.rec + kRec * int64_t(gb);
+    constexpr int up[6] = {0, 1, 2, 4, 5, 8};
     for (int k = 0; k < 3; ++k) {
-      d.pts[3 * int64_t(gb) + k] = s[k];
+      rec[k] = x[k];
+      rec[18 + k] = s[k];
       gmax = fmax(gmax, fabs(s[k]));
-      y[k] = Hi[3 * k] * s[0] + Hi[3 * k + 1] * s[1] + Hi[3 * k + 2] * s[2];
     }
-    const T xt[3] = {T(x[0]), T(x[1]), T(x[2])};
-    T HiT[9];
-    for (int k = 0; k < 9; ++k) HiT[k] = T(Hi[k]);
-    for (int oi = ob; oi < oe; ++oi) {
-      const int ci = d.obs_cam[oi] - 1;
-      if (ci < 0) continue;
+    for (int k = 0; k < 9; ++k) rec[3 + k] = Hi[k];
+    for (int k = 0; k < 6; ++k) rec[12 + k] = H[up[k]];
+  }
+  __syncthreads();  // the point records are read below
+  // own terms, camera by camera: 21 entries of M H^-1 (H - M) lifted, rhs and gradient
+  for (int c = 1 + tid / 16; c < nc; c += NT / 16) {
+    const int ci = c - 1;
+    double own[33];
+#pragma unroll
+    for (int e = 0; e < 33; ++e) own[e] = 0.0;
+    for (int q = d.cam_ptr[c0 + c] + (tid & 15); q < d.cam_ptr[c0 + c + 1]; q += 16) {
+      const double* rec = d.rec + kRec * int64_t(q0 + d.cam_pt[q]);
+      double h[kRec];
+#pragma unroll
+      for (int k = 0; k < kRec; ++k) h[k] = rec[k];
+      const double x[3] = {h[0], h[1], h[2]};
       double r[2];
-      T Ai[6], Mi[9];
-      obs_eval<T>(cams + 15 * (ci + 1), K, d.obs_uv + 2 * int64_t(oi), x, r, Ai);
+      T A[6], M[9], R[9], Z[9], N[9];
+      obs_eval<T>(cams + 15 * c, K, d.cam_uv + 2 * int64_t(q), x, r, A);
       const double w = huber_weight(d.robust, d.delta, sqrt(r[0] * r[0] + r[1] * r[1]));
       const double rw0 = d.robust == 1 ? w * r[0] : r[0], rw1 = d.robust == 1 ? w * r[1] : r[1];
-      gram3(Ai, Mi);
+      gram3(A, M);
+      const T Hi[9] = {T(h[3]), T(h[4]), T(h[5]), T(h[6]), T(h[7]), T(h[8]), T(h[9]), T(h[10]), T(h[11])};
+      const double y[3] = {h[3] * h[18] + h[4] * h[19] + h[5] * h[20], h[6] * h[18] + h[7] * h[19] + h[8] * h[20],
+                           h[9] * h[18] + h[10] * h[19] + h[11] * h[20]};
       double v[3], t[3];
-      for (int k = 0; k < 3; ++k) v[k] = double(Ai[k]) * rw0 + double(Ai[3 + k]) * rw1;
-      for (int k = 0; k < 3; ++k)
-        t[k] = double(Mi[3 * k]) * y[0] + double(Mi[3 * k + 1]) * y[1] + double(Mi[3 * k + 2]) * y[2] - v[k];
-      // rhs += P^T t = [x cross t; t]; gradient -= P^T v
-      const double pt[6] = {x[1] * t[2] - x[2] * t[1], x[2] * t[0] - x[0] * t[2], x[0] * t[1] - x[1] * t[0],
-                            t[0], t[1], t[2]};
-      const double pv[6] = {x[1] * v[2] - x[2] * v[1], x[2] * v[0] - x[0] * v[2], x[0] * v[1] - x[1] * v[0],
-                            v[0], v[1], v[2]};
-      for (int k = 0; k < 6; ++k) {
-        atomicAdd(&rhs[6 * ci + k], pt[k]);
-        atomicAdd(&grad[6 * ci + k], -pv[k]);
+#pragma unroll
+      for (int k = 0; k < 9; ++k) {
+        constexpr int at[9] = {12, 13, 14, 13, 15, 16, 14, 16, 17};
+        R[k] = T(h[at[k]] - double(M[k]));
       }
-      // own term M_i H^-1 (H - M_i)
-      T R[9], Z[9], N[9];
-      for (int k = 0; k < 9; ++k) R[k] = T(H[k] - double(Mi[k]));
-      mul3(Mi, HiT, Z);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        v[k] = double(A[k]) * rw0 + double(A[3 + k]) * rw1;
+        t[k] = double(M[3 * k]) * y[0] + double(M[3 * k + 1]) * y[1] + double(M[3 * k + 2]) * y[2] - v[k];
+      }
+      // rhs += P^T t = [x cross t; t]; gradient -= P^T v
+      own[21] += x[1] * t[2] - x[2] * t[1];
+      own[22] += x[2] * t[0] - x[0] * t[2];
+      own[23] += x[0] * t[1] - x[1] * t[0];
+      own[27] -= x[1] * v[2] - x[2] * v[1];
+      own[28] -= x[2] * v[0] - x[0] * v[2];
+      own[29] -= x[0] * v[1] - x[1] * v[0];
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        own[24 + k] += t[k];
+        own[30 + k] -= v[k];
+      }
+      mul3(M, Hi, Z);
       mul3(Z, R, N);
-      lift_add(S, ci, ci, xt, N, 1.0);
-      for (int oj = ob; oj < oe; ++oj) {
-        const int cj = d.obs_cam[oj] - 1;
-        if (oj == oi || cj < 0 || cj > ci) continue;
-        double rj[2];
-        T Aj[6], Mj[9];
-        obs_eval<T>(cams + 15 * (cj + 1), K, d.obs_uv + 2 * int64_t(oj), x, rj, Aj);
-        gram3(Aj, Mj);
-        mul3(Z, Mj, N);
-        lift_add(S, ci, cj, xt, N, -1.0);
+      const T xt[3] = {T(x[0]), T(x[1]), T(x[2])};
+      lift<true>(xt, N, [&](int a, int b2, T val) {
+        if (b2 <= a) own[a * (a + 1) / 2 + b2] += double(val);
+      });
+    }
+#pragma unroll
+    for (int e = 0; e < 33; ++e) own[e] = row_sum(own[e]);
+    // the diagonal block also takes the damping (one per reduced term), and below the terms of
+    // a point's repeated observations of one camera: atomic, as those may come first
+    if ((tid & 15) == 0) {
+#pragma unroll
+      for (int a = 0; a < 6; ++a) {
+#pragma unroll
+        for (int b = 0; b <= a; ++b)
+          atomicAdd(&S[pk(6 * ci + a, 6 * ci + b)],
+                    own[a * (a + 1) / 2 + b] + (a == b ? nu * double(d.cam_nu[c0 + c]) : 0.0));
+        S[pk(n, 6 * ci + a)] = own[21 + a];
+        grad[6 * ci + a] = own[27 + a];
       }
     }
   }
+  // cross terms: a thread per segment of points shared by two cameras
+  const int32_t* pairs = d.pair_pt + d.pair_ptr[p];
+  for (int e = d.seg_ptr[p] + tid; e < d.seg_ptr[p + 1]; e += NT) {
+    const int4 sg = reinterpret_cast<const int4*>(d.seg)[e];
+    double acc[36], ci[12], cj[12];
+#pragma unroll
+    for (int k = 0; k < 36; ++k) acc[k] = 0.0;
+#pragma unroll
+    for (int k = 0; k < 12; ++k) {
+      ci[k] = cams[15 * (sg.x + 1) + k];
+      cj[k] = cams[15 * (sg.y + 1) + k];
+    }
+    for (int q = sg.z; q < sg.z + sg.w; ++q) {
+      const double* h = d.rec + kRec * int64_t(q0 + pairs[q]);
+      const double x[3] = {h[0], h[1], h[2]};
+      const T xt[3] = {T(x[0]), T(x[1]), T(x[2])};
+      const T Hi[9] = {T(h[3]), T(h[4]), T(h[5]), T(h[6]), T(h[7]), T(h[8]), T(h[9]), T(h[10]), T(h[11])};
+      T M[9], Z[9], N[9];
+      obs_gram<T>(ci, K, x, M);
+      mul3(M, Hi, Z);
+      obs_gram<T>(cj, K, x, M);
+      mul3(Z, M, N);
+      lift<false>(xt, N, [&](int a, int b2, T val) { acc[6 * a + b2] -= double(val); });
+    }
+    double* row = S + pk(6 * sg.x, 6 * sg.y);
+#pragma unroll
+    for (int a = 0; a < 6; ++a)
+#pragma unroll
+      for (int b2 = 0; b2 < 6; ++b2) atomicAdd(row + (6 * sg.x * a + a * (a + 1) / 2 + b2), acc[6 * a + b2]);
+  }
+  // a point's repeated observations of one camera: the pair in both orders, B + B^T
+  for (int e = d.same_ptr[p] + tid; e < d.same_ptr[p + 1]; e += NT) {
+    const int ci = d.obs_cam[d.same[e]] - 1;
+    const double* h = d.rec + kRec * int64_t(q0 + d.obs_pt[d.same[e]]);
+    const double x[3] = {h[0], h[1], h[2]};
+    const T xt[3] = {T(x[0]), T(x[1]), T(x[2])};
+    const T Hi[9] = {T(h[3]), T(h[4]), T(h[5]), T(h[6]), T(h[7]), T(h[8]), T(h[9]), T(h[10]), T(h[11])};
+    T M[9], Z[9], N[9];
+    obs_gram<T>(cams + 15 * (ci + 1), K, x, M);
+    mul3(M, Hi, Z);
+    mul3(Z, M, N);
+    lift<false>(xt, N, [&](int a, int b2, T val) {
+      atomicAdd(&S[pk(6 * ci + max(a, b2), 6 * ci + min(a, b2))], (a == b2 ? -2.0 : -1.0) * double(val));
+    });
+  }
   __syncthreads();
-  // per-term damping on the camera diagonal
-  for (int e = tid; e < n; e += NT) S[pk(e, e)] += nu * double(d.cam_nu[c0 + 1 + e / 6]);
   for (int e = tid; e < n; e += NT) gmax = fmax(gmax, fabs(grad[e]));
   const double max_grad = wg_max<NT>(gmax, red);
-  // ---- dense block LDLt in LDS --------------------------------------------------------------
-  for (int k = 0; k < nbk; ++k) {
-    const int o = 6 * k;
-    if (tid == 0) {
-      double Dk[36], L6[36], dk[6];
-      for (int a = 0; a < 6; ++a)
-        for (int b = 0; b < 6; ++b) Dk[6 * a + b] = sym_at(S, o + a, o + b);
-      if (!ldlt6(Dk, L6, dk)) {
-        flags[1] = 1;
-        for (int a = 0; a < 6; ++a) dk[a] = 0.0;
-      }
-      for (int a = 0; a < 6; ++a) {
-        for (int b = 0; b < a; ++b) S[pk(o + a, o + b)] = L6[6 * a + b];
-        S[pk(o + a, o + a)] = dk[a];
-      }
-    }
-    __syncthreads();
-    // W = S(:, k) below the diagonal block; L(:, k) = W D_k^+
-    for (int r = o + 6 + tid; r < n; r += NT) {
-      double v[6];
-      for (int t = 0; t < 6; ++t) {
-        v[t] = S[pk(r, o + t)];
-        W[6 * r + t] = v[t];
-      }
-      d_solve(S, k, v);
-      for (int t = 0; t < 6; ++t) S[pk(r, o + t)] = v[t];
-    }
-    __syncthreads();
-    // trailing update S(r, c) -= L(r, k) . W(c, k) for o + 6 <= c <= r
-    for (int r = o + 6 + tid; r < n; r += NT) {
-      double l[6];
-      for (int t = 0; t < 6; ++t) l[t] = S[pk(r, o + t)];
-      for (int c = o + 6; c <= r; ++c) {
-        const double* w = W + 6 * c;
-        S[pk(r, c)] -= l[0] * w[0] + l[1] * w[1] + l[2] * w[2] + l[3] * w[3] + l[4] * w[4] + l[5] * w[5];
-      }
-    }
-    __syncthreads();
-  }
-  // ---- solves -----------------------------------------------------------------------------
-  for (int e = tid; e < n; e += NT) xs[e] = rhs[e];
-  __syncthreads();
-  for (int k = 0; k < nbk; ++k) {
-    const int o = 6 * k;
-    for (int r = o + 6 + tid; r < n; r += NT) {
-      double s = 0.0;
-      for (int t = 0; t < 6; ++t) s += S[pk(r, o + t)] * xs[o + t];
-      xs[r] -= s;
-    }
-    __syncthreads();
-  }
-  for (int k = tid; k < nbk; k += NT) {
-    double v[6];
-    for (int t = 0; t < 6; ++t) v[t] = xs[6 * k + t];
-    d_solve(S, k, v);
-    for (int t = 0; t < 6; ++t) xs[6 * k + t] = v[t];
-  }
-  __syncthreads();
-  for (int k = nbk - 1; k > 0; --k) {
-    const int o = 6 * k;
-    for (int r = tid; r < o; r += NT) {
-      double s = 0.0;
-      for (int a = 0; a < 6; ++a) s += S[pk(o + a, r)] * xs[o + a];
-      xs[r] -= s;
-    }
-    __syncthreads();
+  if constexpr (std::is_same<T, double>::value) {
+    window_ldlt<NT>(S, n, rd, flags);
+    window_backsolve<NT>(S, n, rd, xs);
+  } else {
+    window_block_solve<NT>(S, n, rd, xs, flags);
   }
   // ---- back-substitution, update, proposal merit ----------------------------------------------
   double dd = 0.0, dg = 0.0, dmax = 0.0;
   double* pnew = d.points[nxt] + 3 * int64_t(q0);
   for (int b = tid; b < np; b += NT) {
     const int gb = q0 + b;
-    const double x[3] = {points[3 * b], points[3 * b + 1], points[3 * b + 2]};
-    double acc[3] = {d.pts[3 * int64_t(gb)], d.pts[3 * int64_t(gb) + 1], d.pts[3 * int64_t(gb) + 2]};
+    double h[kRec];
+#pragma unroll
+    for (int k = 0; k < kRec; ++k) h[k] = d.rec[kRec * int64_t(gb) + k];
+    const double x[3] = {h[0], h[1], h[2]};
+    double acc[3] = {h[18], h[19], h[20]};
     for (int o = d.pt_obs[gb]; o < d.pt_obs[gb + 1]; ++o) {
       const int ci = d.obs_cam[o] - 1;
       if (ci < 0) continue;
-      double r[2];
-      T A[6], M[9];
-      obs_eval<T>(cams + 15 * (ci + 1), K, d.obs_uv + 2 * int64_t(o), x, r, A);
-      gram3(A, M);
+      T M[9];
+      obs_gram<T>(cams + 15 * (ci + 1), K, x, M);
       const double* dx = xs + 6 * ci;
       const double q[3] = {dx[1] * x[2] - dx[2] * x[1] + dx[3], dx[2] * x[0] - dx[0] * x[2] + dx[4],
                            dx[0] * x[1] - dx[1] * x[0] + dx[5]};
       for (int k = 0; k < 3; ++k)
         acc[k] += double(M[3 * k]) * q[0] + double(M[3 * k + 1]) * q[1] + double(M[3 * k + 2]) * q[2];
     }
-    const double* Hi = d.hinv + 9 * int64_t(gb);
+    const double* Hi = h + 3;
     for (int k = 0; k < 3; ++k) {
       const double dk = Hi[3 * k] * acc[0] + Hi[3 * k + 1] * acc[1] + Hi[3 * k + 2] * acc[2];
       pnew[3 * b + k] = x[k] + dk;
       dd += dk * dk;
-      dg += dk * d.pts[3 * int64_t(gb) + k];
+      dg += dk * h[18 + k];
       dmax = fmax(dmax, fabs(dk));
     }
   }
@@ -443,14 +788,7 @@ __device__ void batch_iteration(const BatchDev& d, int p, double* lds, double* r
   double cost = 0.0;
   for (int o = tid; o < no; o += NT) {
     const int go = o0 + o;
-    // point of the observation: observations are sorted by point; find by binary search
-    int lo = q0, hi = q0 + np - 1;
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) / 2;
-      if (d.pt_obs[mid] <= go) lo = mid;
-      else hi = mid - 1;
-    }
-    const double* xp = pnew + 3 * (lo - q0);
+    const double* xp = pnew + 3 * d.obs_pt[go];
     const double x[3] = {xp[0], xp[1], xp[2]};
     double r[2];
     double A[6];
@@ -562,6 +900,89 @@ __global__ void __launch_bounds__(NT)
   }
 }
 
+// Every window's current variables, side by side.
+__global__ void __launch_bounds__(256)
+    k_batch_gather(BatchDev d, double* __restrict__ poses, double* __restrict__ points) {
+  const int p = blockIdx.x, cur = d.cur[p];
+  const int64_t c0 = 7 * int64_t(d.cam0[p]), c1 = 7 * int64_t(d.cam0[p + 1]);
+  const int64_t q0 = 3 * int64_t(d.pt0[p]), q1 = 3 * int64_t(d.pt0[p + 1]);
+  for (int64_t e = c0 + threadIdx.x; e < c1; e += 256) poses[e] = d.poses[cur][e];
+  for (int64_t e = q0 + threadIdx.x; e < q1; e += 256) points[e] = d.points[cur][e];
+}
+
+// The lists of a window that follow from its sorted observations, one workgroup per window:
+// the point of each observation, the observations camera by camera, and the points that two
+// cameras share.  A wavefront takes a camera and goes through the window's observations 64 at
+// a time, in order; an entry's place is the camera's (the pair's) count so far plus the
+// entries of lower lanes, so the lists come out as if written one by one.  Built on the host
+// they cost 250 ms for 1000 windows of 5300 observations, most of it page faults of 230 MB.
+constexpr int kListThreads = 512;
+__global__ void __launch_bounds__(kListThreads)
+    k_batch_lists(BatchDev d, const int32_t* __restrict__ slots, const int32_t* __restrict__ slot_ptr,
+                  int32_t* obs_pt, int32_t* __restrict__ cam_pt, double* __restrict__ cam_uv,
+                  int32_t* __restrict__ pair_pt) {
+  const int p = blockIdx.x, lane = threadIdx.x & 63;
+  const int c0 = d.cam0[p], nc = d.cam0[p + 1] - c0, q0 = d.pt0[p], np = d.pt0[p + 1] - q0;
+  const int o0 = d.obs0[p], o1 = d.obs0[p + 1];
+  for (int b = threadIdx.x; b < np; b += kListThreads)
+    for (int o = d.pt_obs[q0 + b]; o < d.pt_obs[q0 + b + 1]; ++o) obs_pt[o] = b;
+  __syncthreads();
+  const unsigned long long below = (1ull << lane) - 1;
+  int32_t* pairs = pair_pt + d.pair_ptr[p];
+  for (int c = threadIdx.x >> 6; c < nc; c += kListThreads / 64) {
+    const int ci = c - 1;
+    int q = d.cam_ptr[c0 + c];
+    // lane j: where the next pair of blocks ci and j goes
+    int to = lane < ci ? slots[slot_ptr[p] + ci * (ci - 1) / 2 + lane] : 0;
+    for (int z = o0; z < o1; z += 64) {
+      const int o = z + lane;
+      const bool mine = o < o1 && d.obs_cam[min(o, o1 - 1)] == c;
+      const unsigned long long m = __ballot(mine);
+      if (m == 0) continue;
+      int b = 0, first = 0;
+      unsigned with = 0;  // blocks j < ci that see the point, and whether one does twice
+      bool twice = false;
+      if (mine) {
+        const int at = q + __popcll(m & below);
+        b = obs_pt[o];
+        cam_pt[at] = b;
+        cam_uv[2 * int64_t(at)] = d.obs_uv[2 * int64_t(o)];
+        cam_uv[2 * int64_t(at) + 1] = d.obs_uv[2 * int64_t(o) + 1];
+        first = d.pt_obs[q0 + b];
+        for (int j = first; j < o; ++j) {
+          const int cj = d.obs_cam[j] - 1;
+          if (cj < 0 || cj == ci) continue;
+          twice |= (with >> cj & 1) != 0;
+          with |= 1u << cj;
+        }
+      }
+      q += __popcll(m);
+      const bool counts = __ballot(twice) != 0;
+      for (int cj = 0; cj < ci; ++cj) {
+        const unsigned long long see = __ballot(with >> cj & 1);
+        if (see == 0) continue;
+        int n = with >> cj & 1, before = __popcll(see & below), all = __popcll(see);
+        if (counts) {  // several pairs of one point: a running sum over the lanes
+          if (n) {
+            n = 0;
+            for (int j = first; j < o; ++j) n += d.obs_cam[j] - 1 == cj;
+          }
+          int sum = n;
+          for (int s = 1; s < 64; s *= 2) {
+            const int lower = __shfl_up(sum, s);
+            if (lane >= s) sum += lower;
+          }
+          before = sum - n;
+          all = __shfl(sum, 63);
+        }
+        const int at = __shfl(to, cj) + before;
+        for (int k = 0; k < n; ++k) pairs[at + k] = b;
+        if (lane == cj) to += all;
+      }
+    }
+  }
+}
+
 __global__ void k_batch_zero_queue(int32_t* queue) {
   if (threadIdx.x == 0) *queue = 0;
 }
@@ -583,13 +1004,7 @@ __global__ void __launch_bounds__(NT) k_batch_init(BatchDev d) {
   double cost = 0.0;
   for (int o = threadIdx.x; o < no; o += NT) {
     const int go = o0 + o;
-    int lo = q0, hi = q0 + np - 1;
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) / 2;
-      if (d.pt_obs[mid] <= go) lo = mid;
-      else hi = mid - 1;
-    }
-    const double* xp = d.points_init + 3 * int64_t(lo);
+    const double* xp = d.points_init + 3 * int64_t(q0 + d.obs_pt[go]);
     const double x[3] = {xp[0], xp[1], xp[2]};
     double r[2], A[6];
     obs_eval<double>(cams + 15 * d.obs_cam[go], K, d.obs_uv + 2 * int64_t(go), x, r, A);
@@ -632,6 +1047,7 @@ struct sgpu_batch {
   hipGraphExec_t graph_exec = nullptr;
   int graph_iters = 0;
   // the persistent launch: queue counter, per-window wall-clock stamps, its own graph
+  double *out_poses = nullptr, *out_points = nullptr;  // results, gathered
   int32_t* queue = nullptr;
   unsigned long long* t_start = nullptr;
   unsigned long long* t_end = nullptr;
@@ -712,14 +1128,15 @@ sgpu_status sgpu_batch_create(const sgpu_batch_desc* desc, const sgpu_opt_params
         Q > INT32_MAX || C > INT32_MAX)
       throw Error(SGPU_ERR_INVALID_ARGUMENT, "bad prefix arrays");
     int n_max = 0;
-    std::vector<int32_t> cam0(P + 1), pt0(P + 1), obs0(P + 1), obs_cam(O), pt_obs(Q + 1), pt_nu(Q, 0),
-        cam_nu(C, 0);
-    std::vector<double> uv(2 * O);
+    std::vector<int32_t> cam0(P + 1), pt0(P + 1), obs0(P + 1), pt_obs(Q + 1), pt_nu(Q, 0), cam_nu(C, 0),
+        cam_ptr(C + 1, 0), seg, seg_ptr(P + 1, 0), same, same_ptr(P + 1, 0), slots, slot_ptr(P + 1, 0);
+    std::vector<int64_t> pair_ptr(P + 1, 0);
     for (int64_t p = 0; p <= P; ++p) {
       cam0[p] = int32_t(desc->cam_ptr[p]);
       pt0[p] = int32_t(desc->point_ptr[p]);
       obs0[p] = int32_t(desc->obs_ptr[p]);
     }
+    bool sorted = true;
     for (int64_t p = 0; p < P; ++p) {
       const int64_t nc = cam0[p + 1] - cam0[p], np = pt0[p + 1] - pt0[p], no = obs0[p + 1] - obs0[p];
       if (nc < 2 || nc > kBatchMaxCams || np < 1 || no < 1)
@@ -727,43 +1144,97 @@ sgpu_status sgpu_batch_create(const sgpu_batch_desc* desc, const sgpu_opt_params
                     "each window needs 2.." + std::to_string(kBatchMaxCams) +
                         " cameras, points and observations");
       n_max = std::max<int>(n_max, int(6 * (nc - 1)));
-      // observations of the window sorted by (point, camera) (CostFn::sort order)
-      std::vector<int32_t> ord(no);
-      std::iota(ord.begin(), ord.end(), 0);
-      const int64_t ob = obs0[p];
-      for (int64_t o = ob; o < ob + no; ++o) {
-        if (desc->obs_cam[o] < 0 || desc->obs_cam[o] >= nc || desc->obs_point[o] < 0 || desc->obs_point[o] >= np)
-          throw Error(SGPU_ERR_INDEX_OUT_OF_RANGE, "observation index out of range");
-      }
-      std::stable_sort(ord.begin(), ord.end(), [&](int32_t a, int32_t b) {
-        const int64_t pa = desc->obs_point[ob + a], pb = desc->obs_point[ob + b];
-        if (pa != pb) return pa < pb;
-        return desc->obs_cam[ob + a] < desc->obs_cam[ob + b];
-      });
-      std::vector<int32_t> cnt(np + 1, 0);
+      const int32_t* oc = desc->obs_cam + obs0[p];
+      const int32_t* op = desc->obs_point + obs0[p];
+      int32_t* first = pt_obs.data() + pt0[p];
       for (int64_t k = 0; k < no; ++k) {
-        const int64_t o = ob + ord[k];
-        obs_cam[ob + k] = desc->obs_cam[o];
-        uv[2 * (ob + k)] = desc->obs_uv[2 * o];
-        uv[2 * (ob + k) + 1] = desc->obs_uv[2 * o + 1];
-        ++cnt[desc->obs_point[o] + 1];
-      }
-      for (int64_t b = 0; b < np; ++b) cnt[b + 1] += cnt[b];
-      for (int64_t b = 0; b <= np; ++b) pt_obs[pt0[p] + b] = int32_t(ob + cnt[b]);
-      // reduced terms: distinct (camera, point) pairs
-      for (int64_t b = 0; b < np; ++b) {
-        int32_t last = -1;
-        for (int32_t o = pt_obs[pt0[p] + b]; o < pt_obs[pt0[p] + b + 1]; ++o) {
-          if (obs_cam[o] == last) continue;
-          last = obs_cam[o];
-          ++pt_nu[pt0[p] + b];
-          ++cam_nu[cam0[p] + last];
-        }
+        if (oc[k] < 0 || oc[k] >= nc || op[k] < 0 || op[k] >= np)
+          throw Error(SGPU_ERR_INDEX_OUT_OF_RANGE, "observation index out of range");
+        ++first[op[k]];
+        sorted &= k == 0 || op[k] > op[k - 1] || (op[k] == op[k - 1] && oc[k] >= oc[k - 1]);
       }
     }
+    // observations of each window by (point, camera) (CostFn::sort order): two stable counting
+    // passes, none if they come that way
+    for (int64_t q = 0, at = 0; q <= Q; ++q) {
+      const int32_t c = pt_obs[q];
+      pt_obs[q] = int32_t(at);
+      at += c;
+    }
+    const int32_t* obs_cam = desc->obs_cam;
+    const double* uv = desc->obs_uv;
+    std::vector<int32_t> cam_sorted;
+    std::vector<double> uv_sorted;
+    if (!sorted) {
+      cam_sorted.resize(O);
+      uv_sorted.resize(2 * O);
+      std::vector<int32_t> by_cam, to(pt_obs);
+      for (int64_t p = 0; p < P; ++p) {
+        const int64_t no = obs0[p + 1] - obs0[p], ob = obs0[p];
+        int32_t at[kBatchMaxCams + 1] = {};
+        by_cam.resize(no);
+        for (int64_t k = 0; k < no; ++k) ++at[desc->obs_cam[ob + k] + 1];
+        for (int c = 0; c < kBatchMaxCams; ++c) at[c + 1] += at[c];
+        for (int64_t k = 0; k < no; ++k) by_cam[at[desc->obs_cam[ob + k]]++] = int32_t(k);
+        for (int64_t k = 0; k < no; ++k) {
+          const int64_t o = ob + by_cam[k], q = to[pt0[p] + desc->obs_point[o]]++;
+          cam_sorted[q] = desc->obs_cam[o];
+          uv_sorted[2 * q] = desc->obs_uv[2 * o];
+          uv_sorted[2 * q + 1] = desc->obs_uv[2 * o + 1];
+        }
+      }
+      obs_cam = cam_sorted.data();
+      uv = uv_sorted.data();
+    }
+    for (int64_t p = 0; p < P; ++p) {
+      const int64_t nc = cam0[p + 1] - cam0[p], np = pt0[p + 1] - pt0[p];
+      // reduced terms (distinct (camera, point) pairs), and how many points each two cameras
+      // (other than camera 0) share
+      const int64_t nslot = (nc - 1) * (nc - 2) / 2;
+      int64_t slot[kBatchMaxCams * kBatchMaxCams / 2 + 1] = {};
+      int32_t at[kBatchMaxCams + 1] = {};
+      for (int64_t b = 0; b < np; ++b) {
+        const int32_t o0 = pt_obs[pt0[p] + b], o1 = pt_obs[pt0[p] + b + 1];
+        int32_t last = -1, nu = 0;
+        for (int32_t i = o0; i < o1; ++i) {
+          const int32_t c = obs_cam[i], ci = c - 1;
+          ++at[c + 1];
+          if (c != last) ++nu, ++cam_nu[cam0[p] + c];
+          last = c;
+          if (ci < 0) continue;
+          int64_t* row = slot + ci * (ci - 1) / 2 + 1;
+          for (int32_t j = o0; j < i; ++j) {
+            const int32_t cj = obs_cam[j] - 1;
+            if (cj == ci) same.push_back(i);
+            else if (cj >= 0) ++row[cj];
+          }
+        }
+        pt_nu[pt0[p] + b] = nu;
+      }
+      // the observations camera by camera
+      for (int64_t c = 0; c < nc; ++c) at[c + 1] += at[c];
+      for (int64_t c = 0; c < nc; ++c) cam_ptr[cam0[p] + c + 1] = obs0[p] + at[c + 1];
+      // the points that two cameras share, pair by pair, in segments: full ones first, so that
+      // the threads of a wavefront run alike
+      for (int64_t k = 0; k < nslot; ++k) slot[k + 1] += slot[k];
+      if (slot[nslot] > INT32_MAX) throw Error(SGPU_ERR_UNSUPPORTED, "too many Schur pairs in a window");
+      pair_ptr[p + 1] = pair_ptr[p] + slot[nslot];
+      for (int pass = 0; pass < 2; ++pass)
+        for (int32_t ci = 1, k = 0; ci < nc - 1; ++ci)
+          for (int32_t cj = 0; cj < ci; ++cj, ++k) {
+            const int32_t z = int32_t(slot[k]), n = int32_t(slot[k + 1]) - z, full = n / kSegment * kSegment;
+            if (pass == 0)
+              for (int32_t t = 0; t < full; t += kSegment) seg.insert(seg.end(), {ci, cj, z + t, kSegment});
+            else if (n > full)
+              seg.insert(seg.end(), {ci, cj, z + full, n - full});
+          }
+      slots.insert(slots.end(), slot, slot + nslot);
+      slot_ptr[p + 1] = int32_t(slots.size());
+      seg_ptr[p + 1] = int32_t(seg.size() / 4);
+      same_ptr[p + 1] = int32_t(same.size());
+    }
     const int nt_max = 512;
-    const size_t lds_doubles = size_t(pk(n_max, 0)) + 6 * size_t(n_max) + 3 * size_t(n_max) +
-                               15 * size_t(kBatchMaxCams);
+    const size_t lds_doubles = size_t(pk(n_max + 1, 0)) + (params->precision == SGPU_PRECISION_MIXED ? 8 : 3) * size_t(n_max) + 15 * size_t(kBatchMaxCams);
     const size_t lds_bytes = lds_doubles * 8;
     if (lds_bytes + 8 * (nt_max / 64) + 16 + 8 > 160 * 1024)  // + red, flags, queue slot
       throw Error(SGPU_ERR_UNSUPPORTED, "window too large for the LDS-resident solve");
@@ -799,13 +1270,39 @@ sgpu_status sgpu_batch_create(const sgpu_batch_desc* desc, const sgpu_opt_params
         d.poses[i] = A.alloc<double>(size_t(7) * C);
         d.points[i] = A.alloc<double>(size_t(3) * Q);
       }
-      d.obs_cam = A.upload(obs_cam, nullptr);
-      d.obs_uv = A.upload(uv, nullptr);
+      int32_t* oc = A.alloc<int32_t>(O);
+      double* ouv = A.alloc<double>(2 * size_t(O));
+      SGPU_HIP(hipMemcpy(oc, obs_cam, size_t(O) * sizeof(int32_t), hipMemcpyHostToDevice));
+      SGPU_HIP(hipMemcpy(ouv, uv, size_t(O) * 2 * sizeof(double), hipMemcpyHostToDevice));
+      d.obs_cam = oc;
+      d.obs_uv = ouv;
       d.pt_obs = A.upload(pt_obs, nullptr);
+      d.cam_ptr = A.upload(cam_ptr, nullptr);
+      d.pair_ptr = A.upload(pair_ptr, nullptr);
+      d.seg = A.upload(seg, nullptr);
+      d.seg_ptr = A.upload(seg_ptr, nullptr);
+      {
+        int32_t* obs_pt = A.alloc<int32_t>(O);
+        int32_t* cam_pt = A.alloc<int32_t>(O);
+        double* cam_uv = A.alloc<double>(2 * size_t(O));
+        int32_t* pair_pt = A.alloc<int32_t>(size_t(pair_ptr[P]));
+        DeviceArena tmp;  // freed once the lists are there
+        const int32_t* sl = tmp.upload(slots, nullptr);
+        const int32_t* sp = tmp.upload(slot_ptr, nullptr);
+        hipLaunchKernelGGL(k_batch_lists, dim3(unsigned(P)), dim3(kListThreads), 0, b->stream, d, sl, sp, obs_pt,
+                           cam_pt, cam_uv, pair_pt);
+        SGPU_HIP(hipGetLastError());
+        SGPU_HIP(hipStreamSynchronize(b->stream));
+        d.obs_pt = obs_pt;
+        d.cam_pt = cam_pt;
+        d.cam_uv = cam_uv;
+        d.pair_pt = pair_pt;
+      }
+      d.same = A.upload(same, nullptr);
+      d.same_ptr = A.upload(same_ptr, nullptr);
       d.pt_nu = A.upload(pt_nu, nullptr);
       d.cam_nu = A.upload(cam_nu, nullptr);
-      d.hinv = A.alloc<double>(size_t(9) * Q);
-      d.pts = A.alloc<double>(size_t(3) * Q);
+      d.rec = A.alloc<double>(size_t(kRec) * Q);
       d.cur = A.alloc<int32_t>(P);
       d.nu = A.alloc<double>(P);
       d.merit = A.alloc<double>(P);
@@ -836,6 +1333,8 @@ sgpu_status sgpu_batch_create(const sgpu_batch_desc* desc, const sgpu_opt_params
       set_lds(k_batch_persistent<float, 128>, lds_bytes);
       set_lds(k_batch_persistent<float, 256>, lds_bytes);
       set_lds(k_batch_persistent<float, 512>, lds_bytes);
+      b->out_poses = A.alloc<double>(size_t(7) * C);
+      b->out_points = A.alloc<double>(size_t(3) * Q);
       b->queue = A.alloc<int32_t>(1);
       b->t_start = A.alloc<unsigned long long>(P);
       b->t_end = A.alloc<unsigned long long>(P);
@@ -1016,25 +1515,14 @@ sgpu_status sgpu_batch_results(sgpu_batch* b, double* poses_out, double* points_
     if (!b) throw Error(SGPU_ERR_INVALID_ARGUMENT, "null batch");
     const BatchDev& d = b->d;
     const size_t P = size_t(d.nprob);
-    std::vector<int32_t> cur(P);
-    SGPU_HIP(hipMemcpy(cur.data(), d.cur, P * 4, hipMemcpyDeviceToHost));
     if (poses_out || points_out) {
-      std::vector<double> p0(7 * b->ncam), p1(7 * b->ncam), x0(3 * b->npt), x1(3 * b->npt);
-      std::vector<int32_t> cam0(P + 1), pt0(P + 1);
-      SGPU_HIP(hipMemcpy(cam0.data(), d.cam0, (P + 1) * 4, hipMemcpyDeviceToHost));
-      SGPU_HIP(hipMemcpy(pt0.data(), d.pt0, (P + 1) * 4, hipMemcpyDeviceToHost));
-      SGPU_HIP(hipMemcpy(p0.data(), d.poses[0], p0.size() * 8, hipMemcpyDeviceToHost));
-      SGPU_HIP(hipMemcpy(p1.data(), d.poses[1], p1.size() * 8, hipMemcpyDeviceToHost));
-      SGPU_HIP(hipMemcpy(x0.data(), d.points[0], x0.size() * 8, hipMemcpyDeviceToHost));
-      SGPU_HIP(hipMemcpy(x1.data(), d.points[1], x1.size() * 8, hipMemcpyDeviceToHost));
-      for (size_t p = 0; p < P; ++p) {
-        const auto& ps = cur[p] ? p1 : p0;
-        const auto& xs = cur[p] ? x1 : x0;
-        if (poses_out)
-          std::copy(ps.begin() + 7 * cam0[p], ps.begin() + 7 * cam0[p + 1], poses_out + 7 * cam0[p]);
-        if (points_out)
-          std::copy(xs.begin() + 3 * pt0[p], xs.begin() + 3 * pt0[p + 1], points_out + 3 * pt0[p]);
-      }
+      hipLaunchKernelGGL(k_batch_gather, dim3(d.nprob), dim3(256), 0, b->stream, d, b->out_poses, b->out_points);
+      SGPU_HIP(hipGetLastError());
+      if (poses_out)
+        SGPU_HIP(hipMemcpyAsync(poses_out, b->out_poses, size_t(7) * b->ncam * 8, hipMemcpyDeviceToHost, b->stream));
+      if (points_out)
+        SGPU_HIP(hipMemcpyAsync(points_out, b->out_points, size_t(3) * b->npt * 8, hipMemcpyDeviceToHost, b->stream));
+      SGPU_HIP(hipStreamSynchronize(b->stream));
     }
     if (initial_cost) SGPU_HIP(hipMemcpy(initial_cost, d.init_merit, P * 8, hipMemcpyDeviceToHost));
     if (final_cost) SGPU_HIP(hipMemcpy(final_cost, d.merit, P * 8, hipMemcpyDeviceToHost));
