@@ -24,8 +24,8 @@
 // all its terms to S with LDS atomics, 36 a pair at about 40 cycles a wavefront: 621k to
 // 668k for the three); factor 71k in panels of 12 columns (258k to 544k with one thread per 6x6
 // pivot); solves 18k, back-substitution 33k, merit 27k (57k with a search for the point of
-// each observation).  24 windows of 6 to 31 cameras, 20 persistent iterations: 16.1 -> 5.55 ms;
-// 1000 windows of 6 to 11 cameras, FP32 products, 10 launches: 33.8 -> 12.2 ms.
+// each observation).  24 windows of 5 to 30 cameras, 20 persistent iterations: 16.1 -> 5.55 ms;
+// 1000 such windows, FP32 products, 10 launches: 33.8 -> 12.2 ms.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -146,23 +146,58 @@ __global__ void k_gather_u32(const int32_t* __restrict__ src, const uint32_t* __
   if (e < n) keys[e] = uint32_t(src[order[e]]);
 }
 
+// Where each value starts in sorted keys: start[v] = the number of keys below v, 0 <= v <= m.
+template <typename P>
+__global__ void k_starts(const uint32_t* __restrict__ key, int64_t n, int64_t m, P* __restrict__ start) {
+  const int64_t k = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (k > n) return;
+  const int64_t lo = k == 0 ? 0 : int64_t(key[k - 1]) + 1, hi = k == n ? m : min(int64_t(key[k]), m);
+  for (int64_t v = lo; v <= hi; ++v) start[v] = P(k);
+}
+
 // ---- S pattern ----------------------------------------------------------------------------
-// One thread per active point: a bit for every pair of its observations' free cameras (row =
-// the larger block, column = the smaller) in the nb x nb bitmap (W words per row).
-__global__ void k_pattern_bits(int32_t npt, const int32_t* __restrict__ pt_ptr,
-                               const int32_t* __restrict__ pt_block, const int32_t* __restrict__ obs_pose,
-                               const int32_t* __restrict__ pose_block, int32_t W,
-                               unsigned long long* __restrict__ bits) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= npt || pt_block[b] < 0) return;
-  for (int i = pt_ptr[b]; i < pt_ptr[b + 1]; ++i) {
-    const int ci = pose_block[obs_pose[i]];
-    if (ci < 0) continue;
+// One thread per observation of an active point: a bit for the pair of its free camera and
+// that of each earlier observation of the point (row = the larger block, column = the smaller)
+// in the nb x nb bitmap (W words per row).  Nearly every bit is set many times, so a thread
+// reads the word first and writes only a bit that is missing: with an atomic for each of the
+// 15 million pairs of 120 cameras, in 240 words, the kernel took 12.1 ms.  kLds: each workgroup
+// gathers its bits in LDS, for bitmaps of up to kPatternLds words, which leaves several
+// workgroups per CU; larger bitmaps have fewer pairs per word, read at the agent's scope (L2).
+constexpr int kPatternLds = 4096, kPatternBlocks = 1024;
+template <bool kLds>
+__global__ void __launch_bounds__(kThreads)
+    k_pattern_bits(int32_t nobs, const int32_t* __restrict__ pt_ptr, const int32_t* __restrict__ pt_block,
+                   const int32_t* __restrict__ obs_point, const int32_t* __restrict__ obs_pose,
+                   const int32_t* __restrict__ pose_block, int32_t W, int32_t nwords,
+                   unsigned long long* __restrict__ bits) {
+  __shared__ unsigned long long part[kLds ? kPatternLds : 1];
+  if constexpr (kLds) {
+    for (int w = threadIdx.x; w < nwords; w += kThreads) part[w] = 0;
+    __syncthreads();
+  }
+  for (int64_t i = int64_t(blockIdx.x) * kThreads + threadIdx.x; i < nobs; i += int64_t(gridDim.x) * kThreads) {
+    const int b = obs_point[i], ci = pose_block[obs_pose[i]];
+    if (ci < 0 || pt_block[b] < 0) continue;
     for (int j = pt_ptr[b]; j < i; ++j) {
       const int cj = pose_block[obs_pose[j]];
       if (cj < 0) continue;
       const int r = max(ci, cj), c = min(ci, cj);
-      atomicOr(&bits[int64_t(r) * W + (c >> 6)], 1ull << (c & 63));
+      const int64_t w = int64_t(r) * W + (c >> 6);
+      const unsigned long long bit = 1ull << (c & 63);
+      if constexpr (kLds) {
+        if (!(__hip_atomic_load(&part[w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) & bit))
+          atomicOr(&part[w], bit);
+      } else {
+        if (!(__hip_atomic_load(&bits[w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & bit))
+          atomicOr(&bits[w], bit);
+      }
+    }
+  }
+  if constexpr (kLds) {
+    __syncthreads();
+    for (int w = threadIdx.x; w < nwords; w += kThreads) {
+      const unsigned long long v = part[w];
+      if (v & ~__hip_atomic_load(&bits[w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicOr(&bits[w], v);
     }
   }
 }
@@ -176,25 +211,23 @@ __device__ __forceinline__ uint32_t slot_of(const unsigned long long* bits, cons
   return uint32_t(wpre[w] + __popcll(below));
 }
 
-// Pairs (i, j), i != j, of one active point's observations with free cameras c_j <= c_i:
-// count per point (pass 0) or write them in the host's loop order from the point's offset
-// (pass 1): slot key, position, and the two observations' camera-major positions.
-__global__ void k_pairs(int pass, int32_t npt, const int32_t* __restrict__ pt_ptr,
-                        const int32_t* __restrict__ pt_block, const int32_t* __restrict__ obs_pose,
-                        const int32_t* __restrict__ pose_block, const int32_t* __restrict__ cam_pos,
-                        const unsigned long long* __restrict__ bits, const int32_t* __restrict__ wpre,
-                        int32_t W, int64_t* __restrict__ count_or_off, uint32_t* __restrict__ key,
-                        uint32_t* __restrict__ val, int32_t* __restrict__ pi, int32_t* __restrict__ pj) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= npt) return;
-  if (pt_block[b] < 0) {
-    if (pass == 0) count_or_off[b] = 0;
-    return;
-  }
-  int64_t at = pass == 0 ? 0 : count_or_off[b];
-  for (int i = pt_ptr[b]; i < pt_ptr[b + 1]; ++i) {
-    const int ci = pose_block[obs_pose[i]];
-    if (ci < 0) continue;
+// Pairs (i, j), i != j, of one active point's observations with free cameras c_j <= c_i, a
+// thread per observation i: count them (pass 0) or write them in the host's loop order from
+// the observation's offset (pass 1): slot key, position, and the two observations'
+// camera-major positions.
+__global__ void k_pairs(int pass, int32_t nobs, const int32_t* __restrict__ pt_ptr,
+                        const int32_t* __restrict__ pt_block, const int32_t* __restrict__ obs_point,
+                        const int32_t* __restrict__ obs_pose, const int32_t* __restrict__ pose_block,
+                        const int32_t* __restrict__ cam_pos, const unsigned long long* __restrict__ bits,
+                        const int32_t* __restrict__ wpre, int32_t W, int64_t* __restrict__ count_or_off,
+                        uint32_t* __restrict__ key, uint32_t* __restrict__ val, int32_t* __restrict__ pi,
+                        int32_t* __restrict__ pj) {
+  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i >= nobs) return;
+  const int b = obs_point[i], ci = pose_block[obs_pose[i]];
+  const bool use = ci >= 0 && pt_block[b] >= 0;
+  int64_t at = pass == 0 ? 0 : count_or_off[i];
+  if (use)
     for (int j = pt_ptr[b]; j < pt_ptr[b + 1]; ++j) {
       const int cj = pose_block[obs_pose[j]];
       if (cj < 0 || cj > ci || j == i) continue;
@@ -206,21 +239,17 @@ __global__ void k_pairs(int pass, int32_t npt, const int32_t* __restrict__ pt_pt
       }
       ++at;
     }
-  }
-  if (pass == 0) count_or_off[b] = at;
+  if (pass == 0) count_or_off[i] = at;
 }
 
-// Sorted pair k: its two positions, and its slot counted into per-slot counts.
-__global__ void k_pairs_gather(int64_t n, const uint32_t* __restrict__ key,
-                               const uint32_t* __restrict__ order, const int32_t* __restrict__ pi,
-                               const int32_t* __restrict__ pj, int32_t* __restrict__ pairs,
-                               int64_t* __restrict__ slot_count) {
+// Sorted pair k: its two positions.
+__global__ void k_pairs_gather(int64_t n, const uint32_t* __restrict__ order, const int32_t* __restrict__ pi,
+                               const int32_t* __restrict__ pj, int32_t* __restrict__ pairs) {
   const int64_t k = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (k >= n) return;
   const uint32_t src = order[k];
   pairs[2 * k] = pi[src];
   pairs[2 * k + 1] = pj[src];
-  atomicAdd(reinterpret_cast<unsigned long long*>(&slot_count[key[k]]), 1ull);
 }
 
 template <typename T>
@@ -318,14 +347,21 @@ Symbolic analyze_device(const HostProblem& P, hipStream_t s, DeviceArena& arena,
   // S pattern: the points' bits on the device, the other entries on the host
   int32_t* d_pt_ptr = upload_vec(tmp, S.pt_ptr);
   int32_t* d_pt_block = upload_vec(tmp, points.block);
+  int32_t* d_obs_point = upload_vec(tmp, P.obs_point);
   int32_t* d_obs_pose = upload_vec(tmp, P.obs_pose);
   int32_t* d_pose_block = upload_vec(tmp, poses.block);
   const size_t nwords = size_t(nb) * size_t(W);
   unsigned long long* d_bits = tmp.alloc<unsigned long long>(std::max<size_t>(nwords, 1));
   SGPU_HIP(hipMemsetAsync(d_bits, 0, nwords * 8, s));
-  if (S.npt > 0)
-    hipLaunchKernelGGL(k_pattern_bits, dim3(blocks_of(S.npt, kThreads)), dim3(kThreads), 0, s,
-                       S.npt, d_pt_ptr, d_pt_block, d_obs_pose, d_pose_block, W, d_bits);
+  if (S.nobs > 0) {
+    const dim3 g(std::min(blocks_of(S.nobs, kThreads), kPatternBlocks));
+    if (nwords <= size_t(kPatternLds))
+      hipLaunchKernelGGL(k_pattern_bits<true>, g, dim3(kThreads), 0, s, S.nobs, d_pt_ptr, d_pt_block, d_obs_point,
+                         d_obs_pose, d_pose_block, W, int32_t(nwords), d_bits);
+    else
+      hipLaunchKernelGGL(k_pattern_bits<false>, g, dim3(kThreads), 0, s, S.nobs, d_pt_ptr, d_pt_block, d_obs_point,
+                         d_obs_pose, d_pose_block, W, 0, d_bits);
+  }
   std::vector<unsigned long long> bits(nwords);
   SGPU_HIP(hipMemcpyAsync(bits.data(), d_bits, nwords * 8, hipMemcpyDeviceToHost, s));
   SGPU_HIP(hipStreamSynchronize(s));
@@ -355,40 +391,39 @@ Symbolic analyze_device(const HostProblem& P, hipStream_t s, DeviceArena& arena,
   std::vector<int32_t> cam_pos(size_t(S.nobs), -1);
   for (int32_t q = 0; q < int32_t(S.cam_obs.size()); ++q) cam_pos[S.cam_obs[q]] = q;
   int32_t* d_cam_pos = upload_vec(tmp, cam_pos);
-  int64_t* d_off = tmp.alloc<int64_t>(size_t(S.npt) + 1);
-  const int gp = std::max(1, blocks_of(S.npt, kThreads));
+  int64_t* d_off = tmp.alloc<int64_t>(size_t(S.nobs) + 1);
+  const int gp = std::max(1, blocks_of(S.nobs, kThreads));
   int64_t total = 0;
-  if (S.npt > 0) {
-    hipLaunchKernelGGL(k_pairs, dim3(gp), dim3(kThreads), 0, s, 0, S.npt, d_pt_ptr, d_pt_block,
+  if (S.nobs > 0) {
+    hipLaunchKernelGGL(k_pairs, dim3(gp), dim3(kThreads), 0, s, 0, S.nobs, d_pt_ptr, d_pt_block, d_obs_point,
                        d_obs_pose, d_pose_block, d_cam_pos, d_bits, d_wpre, W, d_off, nullptr,
                        nullptr, nullptr, nullptr);
-    SGPU_HIP(hipMemsetAsync(d_off + S.npt, 0, 8, s));
-    exclusive_scan_i64(s, tmp, d_off, int64_t(S.npt) + 1);
-    SGPU_HIP(hipMemcpyAsync(&total, d_off + S.npt, 8, hipMemcpyDeviceToHost, s));
+    SGPU_HIP(hipMemsetAsync(d_off + S.nobs, 0, 8, s));
+    exclusive_scan_i64(s, tmp, d_off, int64_t(S.nobs) + 1);
+    SGPU_HIP(hipMemcpyAsync(&total, d_off + S.nobs, 8, hipMemcpyDeviceToHost, s));
     SGPU_HIP(hipStreamSynchronize(s));
   }
   if (total > int64_t(INT32_MAX) / 2) throw Error(SGPU_ERR_UNSUPPORTED, "too many Schur pairs");
   *d_pairs = arena.alloc<int32_t>(size_t(std::max<int64_t>(2 * total, 1)));
-  int64_t* d_slot_count = tmp.alloc<int64_t>(size_t(nslot) + 1);
-  SGPU_HIP(hipMemsetAsync(d_slot_count, 0, (size_t(nslot) + 1) * 8, s));
+  S.pair_ptr.assign(size_t(nslot) + 1, 0);
   if (total > 0) {
+    int64_t* d_pair_ptr = tmp.alloc<int64_t>(size_t(nslot) + 1);
     uint32_t* key = tmp.alloc<uint32_t>(size_t(total));
     uint32_t* val = tmp.alloc<uint32_t>(size_t(total));
     uint32_t* key2 = tmp.alloc<uint32_t>(size_t(total));
     uint32_t* val2 = tmp.alloc<uint32_t>(size_t(total));
     int32_t* pi = tmp.alloc<int32_t>(size_t(total));
     int32_t* pj = tmp.alloc<int32_t>(size_t(total));
-    hipLaunchKernelGGL(k_pairs, dim3(gp), dim3(kThreads), 0, s, 1, S.npt, d_pt_ptr, d_pt_block,
+    hipLaunchKernelGGL(k_pairs, dim3(gp), dim3(kThreads), 0, s, 1, S.nobs, d_pt_ptr, d_pt_block, d_obs_point,
                        d_obs_pose, d_pose_block, d_cam_pos, d_bits, d_wpre, W, d_off, key, val,
                        pi, pj);
     radix_sort_pairs(s, tmp, key, val, key2, val2, total, bit_width(uint64_t(nslot)));
-    hipLaunchKernelGGL(k_pairs_gather, dim3(blocks_of(total, kThreads)), dim3(kThreads), 0, s, total,
-                       key, val, pi, pj, *d_pairs, d_slot_count);
+    hipLaunchKernelGGL(k_pairs_gather, dim3(blocks_of(total, kThreads)), dim3(kThreads), 0, s, total, val, pi, pj,
+                       *d_pairs);
+    hipLaunchKernelGGL(k_starts<int64_t>, dim3(blocks_of(total + 1, kThreads)), dim3(kThreads), 0, s, key, total,
+                       nslot, d_pair_ptr);
+    SGPU_HIP(hipMemcpyAsync(S.pair_ptr.data(), d_pair_ptr, (size_t(nslot) + 1) * 8, hipMemcpyDeviceToHost, s));
   }
-  exclusive_scan_i64(s, tmp, d_slot_count, nslot + 1);
-  S.pair_ptr.resize(size_t(nslot) + 1);
-  SGPU_HIP(hipMemcpyAsync(S.pair_ptr.data(), d_slot_count, (size_t(nslot) + 1) * 8,
-                          hipMemcpyDeviceToHost, s));
   SGPU_HIP(hipStreamSynchronize(s));
   S.num_schur_pairs = total + S.cam_ptr[S.nb];
   analyze_chunks(S);
