@@ -239,13 +239,11 @@ struct sgpu_optimizer {
     SGPU_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
     // symbolic analysis: the term sort, the S pattern and the pair lists on the device (the
     // pairs stay there), or all of it on the host
-    int32_t* d_pairs = nullptr;
-    if (params.host_symbolic) {
+    DeviceTerms T;
+    if (params.host_symbolic)
       S = analyze(P);
-    } else {
-      sort_terms_on_device(P, stream);
-      S = analyze_device(P, stream, arena, &d_pairs);
-    }
+    else
+      S = analyze_device(P, stream, arena, T);
     SGPU_HIP(hipHostMalloc(reinterpret_cast<void**>(&h_sc), sizeof(DevScalars), hipHostMallocDefault));
     for (auto& e : ev) SGPU_HIP(hipEventCreate(&e));
     for (auto& e : phase_ev) SGPU_HIP(hipEventCreate(&e));
@@ -261,25 +259,23 @@ struct sgpu_optimizer {
     SGPU_HIP(hipMemcpy(points[0], xf.members.data(), xf.members.size() * 8, hipMemcpyHostToDevice));
     for (int i = 0; i < 2; ++i) intr[i] = arena.upload(kf.members, stream);
     // problem arrays
-    std::vector<int32_t> pt_block(xf.block.begin(), xf.block.end());
     dp.nb = S.nb;
     dp.npt = S.npt;
     dp.nobs = S.nobs;
     dp.npose = S.npose;
     dp.nintr = int32_t(kf.n);
-    dp.obs_pose = arena.upload(P.obs_pose, stream);
-    dp.obs_point = arena.upload(P.obs_point, stream);
-    dp.obs_intr = arena.upload(P.obs_intr, stream);
-    dp.obs_uv = arena.upload(P.obs_uv, stream);
-    dp.pt_ptr = arena.upload(S.pt_ptr, stream);
-    dp.pt_nu = arena.upload(S.pt_nu, stream);
-    dp.pt_block = arena.upload(pt_block, stream);
-    dp.cam_nu = arena.upload(S.cam_nu, stream);
-    dp.pose_block = arena.upload(S.pose_block, stream);
-    dp.cam_member = arena.upload(P.cam_member, stream);
-    dp.cam_ptr = arena.upload(S.cam_ptr, stream);
-    dp.cam_obs = arena.upload(S.cam_obs, stream);
-    {
+    if (params.host_symbolic) {
+      T.obs_pose = arena.upload(P.obs_pose, stream);
+      T.obs_point = arena.upload(P.obs_point, stream);
+      T.obs_intr = arena.upload(P.obs_intr, stream);
+      T.obs_uv = arena.upload(P.obs_uv, stream);
+      T.pt_ptr = arena.upload(S.pt_ptr, stream);
+      T.pt_nu = arena.upload(S.pt_nu, stream);
+      T.pt_block = arena.upload(xf.block, stream);
+      T.cam_nu = arena.upload(S.cam_nu, stream);
+      T.pose_block = arena.upload(S.pose_block, stream);
+      T.cam_ptr = arena.upload(S.cam_ptr, stream);
+      T.cam_obs = arena.upload(S.cam_obs, stream);
       const size_t ncm = S.cam_obs.size();
       std::vector<int32_t> cm_point(ncm), cm_intr(ncm);
       std::vector<double> cm_uv(2 * ncm);
@@ -290,10 +286,26 @@ struct sgpu_optimizer {
         cm_uv[2 * q] = P.obs_uv[2 * size_t(o)];
         cm_uv[2 * q + 1] = P.obs_uv[2 * size_t(o) + 1];
       }
-      dp.cm_point = arena.upload(cm_point, stream);
-      dp.cm_intr = arena.upload(cm_intr, stream);
-      dp.cm_uv = arena.upload(cm_uv, stream);
+      T.cm_point = arena.upload(cm_point, stream);
+      T.cm_intr = arena.upload(cm_intr, stream);
+      T.cm_uv = arena.upload(cm_uv, stream);
+      T.pairs = arena.upload(S.pairs, stream);
     }
+    dp.obs_pose = T.obs_pose;
+    dp.obs_point = T.obs_point;
+    dp.obs_intr = T.obs_intr;
+    dp.obs_uv = T.obs_uv;
+    dp.pt_ptr = T.pt_ptr;
+    dp.pt_nu = T.pt_nu;
+    dp.pt_block = T.pt_block;
+    dp.cam_nu = T.cam_nu;
+    dp.pose_block = T.pose_block;
+    dp.cam_member = arena.upload(P.cam_member, stream);
+    dp.cam_ptr = T.cam_ptr;
+    dp.cam_obs = T.cam_obs;
+    dp.cm_point = T.cm_point;
+    dp.cm_intr = T.cm_intr;
+    dp.cm_uv = T.cm_uv;
     dp.s_ptr = arena.upload(S.s_ptr, stream);
     dp.s_col = arena.upload(S.s_col, stream);
     {
@@ -303,7 +315,7 @@ struct sgpu_optimizer {
       dp.s_row = arena.upload(srow, stream);
     }
     dp.pair_ptr = arena.upload(S.pair_ptr, stream);
-    dp.pairs = d_pairs ? d_pairs : arena.upload(S.pairs, stream);
+    dp.pairs = T.pairs;
     dp.own_chunks = arena.upload(S.own_chunks, stream);
     dp.cam_chunk_ptr = arena.upload(S.cam_chunk_ptr, stream);
     dp.n_own_chunks = int32_t(S.own_chunks.size() / 3);

@@ -322,25 +322,6 @@ HostProblem build_host_problem_sorted(const sgpu_var_family* families, int64_t n
   return P;
 }
 
-void apply_term_order(HostProblem& P, const std::vector<int32_t>& ord) {
-  const size_t n = ord.size();
-  std::vector<int32_t> pose(n), point(n), intr(n);
-  std::vector<double> uv(2 * n);
-  for (size_t t = 0; t < n; ++t) {
-    const int32_t o = ord[t];
-    pose[t] = P.obs_pose[o];
-    point[t] = P.obs_point[o];
-    intr[t] = P.obs_intr[o];
-    uv[2 * t] = P.obs_uv[2 * size_t(o)];
-    uv[2 * t + 1] = P.obs_uv[2 * size_t(o) + 1];
-  }
-  P.obs_pose.swap(pose);
-  P.obs_point.swap(point);
-  P.obs_intr.swap(intr);
-  P.obs_uv.swap(uv);
-  P.terms_sorted = true;
-}
-
 // ---- nested dissection ----------------------------------------------------------------
 
 std::vector<int32_t> nested_dissection(int32_t n, const std::vector<std::vector<int32_t>>& adj,

@@ -74,12 +74,11 @@ HostProblem build_host_problem(const sgpu_var_family* families, int64_t num_fami
                                const sgpu_cost_fn* cost_fns, int64_t num_cost_fns,
                                const sgpu_eq_fn* eq_fns = nullptr, int64_t num_eq_fns = 0);
 // build_host_problem with the term sort optional (sort_terms = false keeps the caller's order
-// for a sort elsewhere, applied with apply_term_order: ord[sorted] = caller's index).
+// for a sort elsewhere).
 HostProblem build_host_problem_sorted(const sgpu_var_family* families, int64_t num_families,
                                       const sgpu_cost_fn* cost_fns, int64_t num_cost_fns,
                                       const sgpu_eq_fn* eq_fns, int64_t num_eq_fns,
                                       bool sort_terms);
-void apply_term_order(HostProblem& P, const std::vector<int32_t>& ord);
 // Most equality-constraint sets one handle takes (the KKT block is solved densely per step).
 constexpr int32_t kMaxEqSets = 16;
 

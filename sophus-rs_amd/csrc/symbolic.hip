@@ -139,6 +139,91 @@ __global__ void k_iota(uint32_t* __restrict__ v, int64_t n) {
   if (e < n) v[e] = uint32_t(e);
 }
 
+// The terms in sorted order, the block of each term's pose (nb for a constant one) as the
+// key of the camera-major sort, and that sort's input order.
+__global__ void k_apply_order(int64_t n, const uint32_t* __restrict__ order, const int32_t* __restrict__ point,
+                              const int32_t* __restrict__ pose, const int32_t* __restrict__ intr,
+                              const double2* __restrict__ uv, const int32_t* __restrict__ pose_block, int32_t nb,
+                              int32_t* __restrict__ s_point, int32_t* __restrict__ s_pose,
+                              int32_t* __restrict__ s_intr, double2* __restrict__ s_uv,
+                              uint32_t* __restrict__ key, uint32_t* __restrict__ pos) {
+  const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (t >= n) return;
+  const uint32_t o = order[t];
+  const int32_t c = pose[o], b = pose_block[c];
+  s_point[t] = point[o];
+  s_pose[t] = c;
+  s_intr[t] = intr[o];
+  s_uv[t] = uv[o];
+  key[t] = uint32_t(b < 0 ? nb : b);
+  pos[t] = uint32_t(t);
+}
+
+// The camera-major copies of the terms, and each term's place there.
+__global__ void k_cam_lists(int32_t ncm, const int32_t* __restrict__ cam_obs, const int32_t* __restrict__ point,
+                            const int32_t* __restrict__ intr, const double2* __restrict__ uv,
+                            int32_t* __restrict__ cm_point, int32_t* __restrict__ cm_intr,
+                            double2* __restrict__ cm_uv, int32_t* __restrict__ cam_pos) {
+  const int64_t q = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (q >= ncm) return;
+  const int32_t o = cam_obs[q];
+  cm_point[q] = point[o];
+  cm_intr[q] = intr[o];
+  cm_uv[q] = uv[o];
+  cam_pos[o] = int32_t(q);
+}
+
+// A reduced term is a run of terms equal in every non-conditioned argument: whether o starts one.
+__device__ __forceinline__ bool starts_term(int64_t o, const int32_t* point, const int32_t* pose,
+                                            const int32_t* intr, bool intr_key) {
+  return o == 0 || point[o] != point[o - 1] || pose[o] != pose[o - 1] || (intr_key && intr[o] != intr[o - 1]);
+}
+
+// Reduced terms per point (a thread each).
+__global__ void k_point_terms(int32_t npt, const int32_t* __restrict__ pt_ptr, const int32_t* __restrict__ point,
+                              const int32_t* __restrict__ pose, const int32_t* __restrict__ intr, bool intr_key,
+                              int32_t* __restrict__ pt_nu) {
+  const int64_t b = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (b >= npt) return;
+  int n = 0;
+  for (int o = pt_ptr[b]; o < pt_ptr[b + 1]; ++o) n += starts_term(o, point, pose, intr, intr_key);
+  pt_nu[b] = n;
+}
+
+// Reduced terms per free block (a workgroup each); the intrinsics block starts at 0.
+__global__ void __launch_bounds__(kThreads)
+    k_block_terms(int32_t intr_block, const int32_t* __restrict__ cam_ptr, const int32_t* __restrict__ cam_obs,
+                  const int32_t* __restrict__ point, const int32_t* __restrict__ pose,
+                  const int32_t* __restrict__ intr, bool intr_key, int32_t* __restrict__ cam_nu) {
+  __shared__ int total;
+  const int c = blockIdx.x;
+  if (threadIdx.x == 0) total = 0;
+  __syncthreads();
+  int n = 0;
+  if (c != intr_block)
+    for (int64_t q = cam_ptr[c] + int64_t(threadIdx.x); q < cam_ptr[c + 1]; q += kThreads)
+      n += starts_term(cam_obs[q], point, pose, intr, intr_key);
+  if (n) atomicAdd(&total, n);
+  __syncthreads();
+  if (threadIdx.x == 0) cam_nu[c] = total;
+}
+
+// Those of the intrinsics block: every term that uses its member.
+__global__ void __launch_bounds__(kThreads)
+    k_intr_terms(int32_t nobs, int32_t intr_member, const int32_t* __restrict__ point,
+                 const int32_t* __restrict__ pose, const int32_t* __restrict__ intr, bool intr_key,
+                 int32_t* __restrict__ nu) {
+  __shared__ int total;
+  if (threadIdx.x == 0) total = 0;
+  __syncthreads();
+  int n = 0;
+  for (int64_t o = int64_t(blockIdx.x) * kThreads + threadIdx.x; o < nobs; o += int64_t(gridDim.x) * kThreads)
+    n += intr[o] == intr_member && starts_term(o, point, pose, intr, intr_key);
+  if (n) atomicAdd(&total, n);
+  __syncthreads();
+  if (threadIdx.x == 0 && total) atomicAdd(nu, total);
+}
+
 // keys[i] = src[order[i]]
 __global__ void k_gather_u32(const int32_t* __restrict__ src, const uint32_t* __restrict__ order,
                              uint32_t* __restrict__ keys, int64_t n) {
@@ -301,66 +386,89 @@ void radix_sort_pairs(hipStream_t s, DeviceArena& arena, uint32_t* keys, uint32_
   }
 }
 
-void sort_terms_on_device(HostProblem& P, hipStream_t s) {
-  if (P.terms_sorted) return;
-  const int64_t n = int64_t(P.obs_point.size());
-  if (n <= 1) {
-    P.terms_sorted = true;
-    return;
-  }
-  DeviceArena tmp;
-  int32_t* d_point = upload_vec(tmp, P.obs_point);
-  int32_t* d_pose = upload_vec(tmp, P.obs_pose);
-  int32_t* d_intr = upload_vec(tmp, P.obs_intr);
-  uint32_t* key = tmp.alloc<uint32_t>(size_t(n));
-  uint32_t* val = tmp.alloc<uint32_t>(size_t(n));
-  uint32_t* key2 = tmp.alloc<uint32_t>(size_t(n));
-  uint32_t* val2 = tmp.alloc<uint32_t>(size_t(n));
-  const int g = blocks_of(n, kThreads);
-  hipLaunchKernelGGL(k_iota, dim3(g), dim3(kThreads), 0, s, val, n);
-  // LSD over the sort key (point, k1, k2): the conditioned argument first, the point last
-  const bool intr_free = P.intr_kind == SGPU_VAR_FREE;
-  const int32_t* by_key[3] = {intr_free ? d_pose : d_intr, intr_free ? d_intr : d_pose, d_point};
-  const std::vector<int32_t>* host_key[3] = {intr_free ? &P.obs_pose : &P.obs_intr,
-                                             intr_free ? &P.obs_intr : &P.obs_pose, &P.obs_point};
-  for (int k = 0; k < 3; ++k) {
-    const int32_t mx = host_key[k]->empty() ? 0 : *std::max_element(host_key[k]->begin(), host_key[k]->end());
-    const int bits = bit_width(uint64_t(std::max(mx, 0)));
-    if (bits == 0) continue;  // one value: nothing to order
-    hipLaunchKernelGGL(k_gather_u32, dim3(g), dim3(kThreads), 0, s, by_key[k], val, key, n);
-    radix_sort_pairs(s, tmp, key, val, key2, val2, n, bits);
-  }
-  std::vector<int32_t> ord(static_cast<size_t>(n));
-  SGPU_HIP(hipMemcpyAsync(ord.data(), val, size_t(n) * 4, hipMemcpyDeviceToHost, s));
-  SGPU_HIP(hipStreamSynchronize(s));
-  apply_term_order(P, ord);
-}
-
-Symbolic analyze_device(const HostProblem& P, hipStream_t s, DeviceArena& arena,
-                        int32_t** d_pairs) {
+Symbolic analyze_device(const HostProblem& P, hipStream_t s, DeviceArena& arena, DeviceTerms& T) {
   Symbolic S;
-  analyze_points(P, S);
   const Family& poses = P.fams[P.f_pose];
   const Family& points = P.fams[P.f_point];
-  DeviceArena tmp;
+  const Family& intrs = P.fams[P.f_intr];
+  const int64_t n = int64_t(P.obs_point.size());
+  S.nb = int32_t(P.num_free_blocks);
+  S.npt = int32_t(points.n);
+  S.npose = int32_t(poses.n);
+  S.nobs = int32_t(n);
+  S.pose_block = poses.block;
   const int32_t nb = S.nb, W = (S.nb + 63) / 64;
+  const bool intr_key = P.intr_kind != SGPU_VAR_CONDITIONED;
+  const int g = std::max(1, blocks_of(n, kThreads));
+  DeviceArena tmp;
+  // the sorted terms, point by point and camera by camera
+  T.pose_block = upload_vec(arena, poses.block);
+  T.pt_block = upload_vec(arena, points.block);
+  T.obs_point = arena.alloc<int32_t>(size_t(n));
+  T.obs_pose = arena.alloc<int32_t>(size_t(n));
+  T.obs_intr = arena.alloc<int32_t>(size_t(n));
+  T.obs_uv = arena.alloc<double>(2 * size_t(n));
+  T.pt_ptr = arena.alloc<int32_t>(size_t(S.npt) + 1);
+  T.pt_nu = arena.alloc<int32_t>(size_t(S.npt));
+  T.cam_ptr = arena.alloc<int32_t>(size_t(nb) + 1);
+  T.cam_nu = arena.alloc<int32_t>(size_t(nb));
+  uint32_t* key = tmp.alloc<uint32_t>(4 * size_t(n));
+  uint32_t *val = key + n, *key2 = val + n, *val2 = key2 + n;
+  {
+    DeviceArena raw;  // the caller's order, given back before the pair arrays are allocated
+    const int32_t* point = upload_vec(raw, P.obs_point);
+    const int32_t* pose = upload_vec(raw, P.obs_pose);
+    const int32_t* intr = upload_vec(raw, P.obs_intr);
+    const double* uv = upload_vec(raw, P.obs_uv);
+    hipLaunchKernelGGL(k_iota, dim3(g), dim3(kThreads), 0, s, val, n);
+    if (!P.terms_sorted) {
+      // LSD over the sort key (point, k1, k2): the conditioned argument first, the point last
+      const bool intr_free = P.intr_kind == SGPU_VAR_FREE;
+      const int32_t* by_key[3] = {intr_free ? pose : intr, intr_free ? intr : pose, point};
+      const int64_t members[3] = {intr_free ? poses.n : intrs.n, intr_free ? intrs.n : poses.n, points.n};
+      for (int k = 0; k < 3; ++k) {
+        const int bits = bit_width(uint64_t(std::max<int64_t>(members[k] - 1, 0)));
+        if (bits == 0) continue;  // one value: nothing to order
+        hipLaunchKernelGGL(k_gather_u32, dim3(g), dim3(kThreads), 0, s, by_key[k], val, key, n);
+        radix_sort_pairs(s, tmp, key, val, key2, val2, n, bits);
+      }
+    }
+    hipLaunchKernelGGL(k_apply_order, dim3(g), dim3(kThreads), 0, s, n, val, point, pose, intr,
+                       reinterpret_cast<const double2*>(uv), T.pose_block, nb, T.obs_point, T.obs_pose, T.obs_intr,
+                       reinterpret_cast<double2*>(T.obs_uv), key, key2);
+  }
+  std::swap(val, key2);  // the camera sort's input order
+  hipLaunchKernelGGL(k_starts<int32_t>, dim3(blocks_of(n + 1, kThreads)), dim3(kThreads), 0, s,
+                     reinterpret_cast<const uint32_t*>(T.obs_point), n, int64_t(S.npt), T.pt_ptr);
+  radix_sort_pairs(s, tmp, key, val, key2, val2, n, bit_width(uint64_t(nb)));
+  hipLaunchKernelGGL(k_starts<int32_t>, dim3(blocks_of(n + 1, kThreads)), dim3(kThreads), 0, s, key, n, int64_t(nb),
+                     T.cam_ptr);
+  const int32_t* cam_order = reinterpret_cast<const int32_t*>(val);
+  if (S.npt > 0)
+    hipLaunchKernelGGL(k_point_terms, dim3(blocks_of(S.npt, kThreads)), dim3(kThreads), 0, s, S.npt, T.pt_ptr,
+                       T.obs_point, T.obs_pose, T.obs_intr, intr_key, T.pt_nu);
+  if (nb > 0)
+    hipLaunchKernelGGL(k_block_terms, dim3(nb), dim3(kThreads), 0, s, P.intr_block, T.cam_ptr, cam_order,
+                       T.obs_point, T.obs_pose, T.obs_intr, intr_key, T.cam_nu);
+  if (P.intr_block >= 0)
+    hipLaunchKernelGGL(k_intr_terms, dim3(std::min(g, 512)), dim3(kThreads), 0, s, S.nobs, P.intr_member, T.obs_point,
+                       T.obs_pose, T.obs_intr, intr_key, T.cam_nu + P.intr_block);
+  S.pt_ptr.resize(size_t(S.npt) + 1);
+  S.cam_ptr.resize(size_t(nb) + 1);
+  SGPU_HIP(hipMemcpyAsync(S.pt_ptr.data(), T.pt_ptr, S.pt_ptr.size() * 4, hipMemcpyDeviceToHost, s));
+  SGPU_HIP(hipMemcpyAsync(S.cam_ptr.data(), T.cam_ptr, S.cam_ptr.size() * 4, hipMemcpyDeviceToHost, s));
   // S pattern: the points' bits on the device, the other entries on the host
-  int32_t* d_pt_ptr = upload_vec(tmp, S.pt_ptr);
-  int32_t* d_pt_block = upload_vec(tmp, points.block);
-  int32_t* d_obs_point = upload_vec(tmp, P.obs_point);
-  int32_t* d_obs_pose = upload_vec(tmp, P.obs_pose);
-  int32_t* d_pose_block = upload_vec(tmp, poses.block);
   const size_t nwords = size_t(nb) * size_t(W);
   unsigned long long* d_bits = tmp.alloc<unsigned long long>(std::max<size_t>(nwords, 1));
   SGPU_HIP(hipMemsetAsync(d_bits, 0, nwords * 8, s));
   if (S.nobs > 0) {
     const dim3 g(std::min(blocks_of(S.nobs, kThreads), kPatternBlocks));
     if (nwords <= size_t(kPatternLds))
-      hipLaunchKernelGGL(k_pattern_bits<true>, g, dim3(kThreads), 0, s, S.nobs, d_pt_ptr, d_pt_block, d_obs_point,
-                         d_obs_pose, d_pose_block, W, int32_t(nwords), d_bits);
+      hipLaunchKernelGGL(k_pattern_bits<true>, g, dim3(kThreads), 0, s, S.nobs, T.pt_ptr, T.pt_block, T.obs_point,
+                         T.obs_pose, T.pose_block, W, int32_t(nwords), d_bits);
     else
-      hipLaunchKernelGGL(k_pattern_bits<false>, g, dim3(kThreads), 0, s, S.nobs, d_pt_ptr, d_pt_block, d_obs_point,
-                         d_obs_pose, d_pose_block, W, 0, d_bits);
+      hipLaunchKernelGGL(k_pattern_bits<false>, g, dim3(kThreads), 0, s, S.nobs, T.pt_ptr, T.pt_block, T.obs_point,
+                         T.obs_pose, T.pose_block, W, 0, d_bits);
   }
   std::vector<unsigned long long> bits(nwords);
   SGPU_HIP(hipMemcpyAsync(bits.data(), d_bits, nwords * 8, hipMemcpyDeviceToHost, s));
@@ -388,15 +496,24 @@ Symbolic analyze_device(const HostProblem& P, hipStream_t s, DeviceArena& arena,
   SGPU_HIP(hipMemcpyAsync(d_bits, bits.data(), nwords * 8, hipMemcpyHostToDevice, s));
   int32_t* d_wpre = upload_vec(tmp, wpre);
   // pairs: count per point, offsets, fill in point order, stable sort by slot
-  std::vector<int32_t> cam_pos(size_t(S.nobs), -1);
-  for (int32_t q = 0; q < int32_t(S.cam_obs.size()); ++q) cam_pos[S.cam_obs[q]] = q;
-  int32_t* d_cam_pos = upload_vec(tmp, cam_pos);
+  const int32_t ncm = S.cam_ptr[nb];
+  T.cam_obs = arena.alloc<int32_t>(size_t(ncm));
+  T.cm_point = arena.alloc<int32_t>(size_t(ncm));
+  T.cm_intr = arena.alloc<int32_t>(size_t(ncm));
+  T.cm_uv = arena.alloc<double>(2 * size_t(ncm));
+  int32_t* d_cam_pos = tmp.alloc<int32_t>(size_t(n));  // read for the terms of free cameras only
+  if (ncm > 0) {
+    SGPU_HIP(hipMemcpyAsync(T.cam_obs, cam_order, size_t(ncm) * 4, hipMemcpyDeviceToDevice, s));
+    hipLaunchKernelGGL(k_cam_lists, dim3(blocks_of(ncm, kThreads)), dim3(kThreads), 0, s, ncm, T.cam_obs, T.obs_point,
+                       T.obs_intr, reinterpret_cast<const double2*>(T.obs_uv), T.cm_point, T.cm_intr,
+                       reinterpret_cast<double2*>(T.cm_uv), d_cam_pos);
+  }
   int64_t* d_off = tmp.alloc<int64_t>(size_t(S.nobs) + 1);
   const int gp = std::max(1, blocks_of(S.nobs, kThreads));
   int64_t total = 0;
   if (S.nobs > 0) {
-    hipLaunchKernelGGL(k_pairs, dim3(gp), dim3(kThreads), 0, s, 0, S.nobs, d_pt_ptr, d_pt_block, d_obs_point,
-                       d_obs_pose, d_pose_block, d_cam_pos, d_bits, d_wpre, W, d_off, nullptr,
+    hipLaunchKernelGGL(k_pairs, dim3(gp), dim3(kThreads), 0, s, 0, S.nobs, T.pt_ptr, T.pt_block, T.obs_point,
+                       T.obs_pose, T.pose_block, d_cam_pos, d_bits, d_wpre, W, d_off, nullptr,
                        nullptr, nullptr, nullptr);
     SGPU_HIP(hipMemsetAsync(d_off + S.nobs, 0, 8, s));
     exclusive_scan_i64(s, tmp, d_off, int64_t(S.nobs) + 1);
@@ -404,22 +521,20 @@ Symbolic analyze_device(const HostProblem& P, hipStream_t s, DeviceArena& arena,
     SGPU_HIP(hipStreamSynchronize(s));
   }
   if (total > int64_t(INT32_MAX) / 2) throw Error(SGPU_ERR_UNSUPPORTED, "too many Schur pairs");
-  *d_pairs = arena.alloc<int32_t>(size_t(std::max<int64_t>(2 * total, 1)));
+  T.pairs = arena.alloc<int32_t>(size_t(std::max<int64_t>(2 * total, 1)));
   S.pair_ptr.assign(size_t(nslot) + 1, 0);
   if (total > 0) {
     int64_t* d_pair_ptr = tmp.alloc<int64_t>(size_t(nslot) + 1);
-    uint32_t* key = tmp.alloc<uint32_t>(size_t(total));
-    uint32_t* val = tmp.alloc<uint32_t>(size_t(total));
-    uint32_t* key2 = tmp.alloc<uint32_t>(size_t(total));
-    uint32_t* val2 = tmp.alloc<uint32_t>(size_t(total));
-    int32_t* pi = tmp.alloc<int32_t>(size_t(total));
-    int32_t* pj = tmp.alloc<int32_t>(size_t(total));
-    hipLaunchKernelGGL(k_pairs, dim3(gp), dim3(kThreads), 0, s, 1, S.nobs, d_pt_ptr, d_pt_block, d_obs_point,
-                       d_obs_pose, d_pose_block, d_cam_pos, d_bits, d_wpre, W, d_off, key, val,
+    uint32_t* key = tmp.alloc<uint32_t>(6 * size_t(total));
+    uint32_t *val = key + total, *key2 = val + total, *val2 = key2 + total;
+    int32_t* pi = reinterpret_cast<int32_t*>(val2 + total);
+    int32_t* pj = pi + total;
+    hipLaunchKernelGGL(k_pairs, dim3(gp), dim3(kThreads), 0, s, 1, S.nobs, T.pt_ptr, T.pt_block, T.obs_point,
+                       T.obs_pose, T.pose_block, d_cam_pos, d_bits, d_wpre, W, d_off, key, val,
                        pi, pj);
     radix_sort_pairs(s, tmp, key, val, key2, val2, total, bit_width(uint64_t(nslot)));
     hipLaunchKernelGGL(k_pairs_gather, dim3(blocks_of(total, kThreads)), dim3(kThreads), 0, s, total, val, pi, pj,
-                       *d_pairs);
+                       T.pairs);
     hipLaunchKernelGGL(k_starts<int64_t>, dim3(blocks_of(total + 1, kThreads)), dim3(kThreads), 0, s, key, total,
                        nslot, d_pair_ptr);
     SGPU_HIP(hipMemcpyAsync(S.pair_ptr.data(), d_pair_ptr, (size_t(nslot) + 1) * 8, hipMemcpyDeviceToHost, s));
@@ -467,21 +582,42 @@ extern "C" sgpu_status sgpu_symbolic_check(const sgpu_var_family* families, int6
     const Symbolic Sh = analyze(Ph);
     const auto t1 = clk::now();
     DeviceArena arena;
-    int32_t* d_pairs = nullptr;
+    DeviceTerms T;
     HostProblem Pd = build_host_problem_sorted(families, num_families, cost_fns, num_cost_fns,
                                                nullptr, 0, false);
-    sort_terms_on_device(Pd, s);
-    Symbolic Sd = analyze_device(Pd, s, arena, &d_pairs);
+    Symbolic Sd = analyze_device(Pd, s, arena, T);
     const auto t2 = clk::now();
+    const auto fetch = [](auto& v, const auto* d, size_t n) {
+      v.resize(n);
+      if (n) SGPU_HIP(hipMemcpy(v.data(), d, n * sizeof(v[0]), hipMemcpyDeviceToHost));
+    };
+    const size_t nobs = Pd.obs_point.size(), ncm = size_t(Sd.cam_ptr.back());
+    fetch(Pd.obs_pose, T.obs_pose, nobs);
+    fetch(Pd.obs_point, T.obs_point, nobs);
+    fetch(Pd.obs_intr, T.obs_intr, nobs);
+    fetch(Pd.obs_uv, T.obs_uv, 2 * nobs);
+    fetch(Sd.pt_nu, T.pt_nu, size_t(Sd.npt));
+    fetch(Sd.cam_nu, T.cam_nu, size_t(Sd.nb));
+    fetch(Sd.cam_obs, T.cam_obs, ncm);
+    std::vector<int32_t> cm_point, cm_intr;
+    std::vector<double> cm_uv;
+    fetch(cm_point, T.cm_point, ncm);
+    fetch(cm_intr, T.cm_intr, ncm);
+    fetch(cm_uv, T.cm_uv, 2 * ncm);
     Sd.pairs.resize(Sh.pairs.size());
     if (!Sh.pairs.empty() && Sd.pair_ptr.size() == Sh.pair_ptr.size() &&
         Sd.pair_ptr.back() * 2 == int64_t(Sh.pairs.size()))
-      SGPU_HIP(hipMemcpy(Sd.pairs.data(), d_pairs, Sh.pairs.size() * 4, hipMemcpyDeviceToHost));
+      SGPU_HIP(hipMemcpy(Sd.pairs.data(), T.pairs, Sh.pairs.size() * 4, hipMemcpyDeviceToHost));
     int64_t d = 0;
     d += count_diff(Ph.obs_pose, Pd.obs_pose) + count_diff(Ph.obs_point, Pd.obs_point) +
          count_diff(Ph.obs_intr, Pd.obs_intr) + count_diff(Ph.obs_uv, Pd.obs_uv);
     d += count_diff(Sh.pt_ptr, Sd.pt_ptr) + count_diff(Sh.pt_nu, Sd.pt_nu) + count_diff(Sh.cam_nu, Sd.cam_nu);
     d += count_diff(Sh.cam_ptr, Sd.cam_ptr) + count_diff(Sh.cam_obs, Sd.cam_obs);
+    for (size_t q = 0; q < ncm && ncm == Sh.cam_obs.size(); ++q) {
+      const size_t o = size_t(Sh.cam_obs[q]);
+      d += cm_point[q] != Ph.obs_point[o] || cm_intr[q] != Ph.obs_intr[o] || cm_uv[2 * q] != Ph.obs_uv[2 * o] ||
+           cm_uv[2 * q + 1] != Ph.obs_uv[2 * o + 1];
+    }
     d += count_diff(Sh.s_ptr, Sd.s_ptr) + count_diff(Sh.s_col, Sd.s_col);
     d += count_diff(Sh.pair_ptr, Sd.pair_ptr) + count_diff(Sh.pairs, Sd.pairs);
     d += count_diff(Sh.own_chunks, Sd.own_chunks) + count_diff(Sh.cam_chunk_ptr, Sd.cam_chunk_ptr);

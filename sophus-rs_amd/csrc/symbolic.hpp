@@ -22,14 +22,24 @@ void radix_sort_pairs(hipStream_t s, DeviceArena& arena, uint32_t* keys, uint32_
 // Exclusive prefix sum of n int64 counts (in place), on the device.
 void exclusive_scan_i64(hipStream_t s, DeviceArena& arena, int64_t* data, int64_t n);
 
-// The term sort of a problem built with build_host_problem_sorted(.., false), on the device
-// (stable radix passes over the sort key's arguments, the last argument first), applied to
-// P: the HostProblem build_host_problem returns.
-void sort_terms_on_device(HostProblem& P, hipStream_t s);
+// The arrays of the term sort and the analysis that the numeric kernels read, on the device:
+// the reprojection terms in sorted order, the point and camera lists over them, the members'
+// blocks, and the pairs of S slots (2 per pair).
+struct DeviceTerms {
+  int32_t *obs_point = nullptr, *obs_pose = nullptr, *obs_intr = nullptr;
+  double* obs_uv = nullptr;
+  int32_t *pt_ptr = nullptr, *pt_nu = nullptr, *pt_block = nullptr, *pose_block = nullptr;
+  int32_t *cam_ptr = nullptr, *cam_nu = nullptr, *cam_obs = nullptr;
+  int32_t *cm_point = nullptr, *cm_intr = nullptr;
+  double* cm_uv = nullptr;
+  int32_t* pairs = nullptr;
+};
 
-// analyze() with the S pattern and the pair lists built on the device.  The pairs stay on
-// the device (*d_pairs, 2 per pair, allocated from `arena`); S.pairs is left empty.
-Symbolic analyze_device(const HostProblem& P, hipStream_t s, DeviceArena& arena,
-                        int32_t** d_pairs);
+// analyze() of a problem built with build_host_problem_sorted(.., false), with the term sort
+// (stable radix passes over the sort key's arguments, the last argument first), the lists over
+// the sorted terms, the S pattern and the pair lists built on the device.  They stay there
+// (T, allocated from `arena`): P keeps the caller's order, and S.pt_nu, cam_nu, cam_obs and
+// pairs are left empty.
+Symbolic analyze_device(const HostProblem& P, hipStream_t s, DeviceArena& arena, DeviceTerms& T);
 
 }  // namespace sgpu
