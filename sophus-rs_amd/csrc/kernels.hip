@@ -1833,8 +1833,13 @@ __global__ void __launch_bounds__(kTriMax)
 // node's (children one after another, so the adds are plain), then panel by panel y_P =
 // L_PP^-1 b_P (the stored L_PP^-T), z_P = D^+ y_P and b_r -= L_r y_P for every
 // row below the panel, the same eliminations the factorization applies to the step's own
-// right-hand side.
-__global__ void __launch_bounds__(kThreads)
+// right-hand side.  A panel is a chain of two loads and two dot products of 48; what bounds it
+// is the latency of the loads.  So the first wavefront forms y_P, the others take a row each,
+// and each thread has its 48 operands on the way (its column of L_PP^-T, or its first row's
+// entries of L) before the panel's right-hand side is there.  With loads inside loops of the
+// panel's width it took 74 us a level for a tree of 150 cameras, now 30.
+constexpr int kFwdThreads = 512;
+__global__ void __launch_bounds__(kFwdThreads)
     k_mf_fwd(DevFactor f, const int32_t* __restrict__ nodes, double* __restrict__ z) {
   const int X = nodes[blockIdx.x];
   const int F = 6 * f.sn_nf[X], K = 6 * f.sn_nc[X], c0 = f.sn_c0[X];
@@ -1842,35 +1847,49 @@ __global__ void __launch_bounds__(kThreads)
   const double* L = f.lbuf + f.sn_loff[X];
   const double* Tn = f.tinv + f.sn_poff[X];
   const int tid = threadIdx.x;
+  const bool solver = __builtin_amdgcn_readfirstlane(tid >> 6) == 0;  // the first wavefront
   __shared__ double sb[kPW], sy[kPW];
   for (int ci = f.sn_child_ptr[X]; ci < f.sn_child_ptr[X + 1]; ++ci) {
     const int C = f.sn_child[ci];
     const int FC = 6 * f.sn_nf[C], KC = 6 * f.sn_nc[C];
     const double* bc = f.usolve + f.sn_uoff[C];
-    for (int u = tid; u < FC - KC; u += blockDim.x) b[parent_row(f, C, u)] += bc[KC + u];
+    for (int u = tid; u < FC - KC; u += kFwdThreads) b[parent_row(f, C, u)] += bc[KC + u];
     __syncthreads();
   }
   const int npan = (K + kPW - 1) / kPW;
   for (int p = 0; p < npan; ++p) {
-    const int k0 = kPW * p, np = min(kPW, K - k0);
-    const double* Tg = Tn + int64_t(p) * kPW * kPW;
-    if (tid < np) sb[tid] = b[k0 + tid];
+    const int k0 = kPW * p, np = min(kPW, K - k0), r0 = k0 + np;
+    // L_PP^-T (t, c) = L_PP^-1 (c, t); entries past the panel's width meet zeros of sb and sy
+    const double* at = solver ? Tn + int64_t(p) * kPW * kPW : L + int64_t(k0) * F;
+    const int ld = solver ? kPW : F, last = solver ? kPW - 1 : np - 1;
+    const auto load = [&](double (&v)[kPW], unsigned col) __attribute__((always_inline)) {
+#pragma unroll
+      for (int t = 0; t < kPW; ++t) v[t] = (at + int64_t(min(t, last)) * ld)[col];
+    };
+    double cur[kPW];
+    load(cur, unsigned(solver ? min(tid, kPW - 1) : min(r0 + tid - 64, F - 1)));
+    if (tid < kPW) sb[tid] = tid < np ? b[k0 + tid] : 0.0;
     __syncthreads();
-    if (tid < np) {
-      double y = 0.0;
-      for (int t = 0; t < np; ++t) y += Tg[t * kPW + tid] * sb[t];  // L_PP^-T (t, c) = L_PP^-1 (c, t)
-      sy[tid] = y;
+    if (solver) {
+      double y[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int t = 0; t < kPW; ++t) y[t & 3] += cur[t] * sb[t];
+      const double v = (y[0] + y[1]) + (y[2] + y[3]);
+      if (tid < kPW) sy[tid] = tid < np ? v : 0.0;
+      if (tid < np) {
+        const int64_t e = 6 * int64_t(c0) + k0 + tid;
+        z[e] = v * f.piv_r[e];
+      }
     }
     __syncthreads();
-    if (tid < np) {
-      const int64_t at = 6 * int64_t(c0) + k0 + tid;
-      z[at] = sy[tid] * f.piv_r[at];
-    }
-    for (int r = k0 + np + tid; r < F; r += blockDim.x) {
-      double acc = 0.0;
-      for (int t = 0; t < np; ++t) acc += L[int64_t(k0 + t) * F + r] * sy[t];
-      b[r] -= acc;
-    }
+    if (!solver)
+      for (int r = r0 + tid - 64; r < F; r += kFwdThreads - 64) {
+        double acc[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int t = 0; t < kPW; ++t) acc[t & 3] += cur[t] * sy[t];
+        b[r] -= (acc[0] + acc[1]) + (acc[2] + acc[3]);
+        if (r + kFwdThreads - 64 < F) load(cur, unsigned(r + kFwdThreads - 64));
+      }
     __syncthreads();
   }
 }
@@ -3059,7 +3078,7 @@ void launch_rcs_forward(hipStream_t s, const DevFactor& f, const double* b_nat, 
   const int nlev = int(S.lvl_ptr.size()) - 1;
   for (int l = 0; l < nlev; ++l) {
     const int n = S.lvl_ptr[l + 1] - S.lvl_ptr[l];
-    hipLaunchKernelGGL(k_mf_fwd, dim3(n), dim3(kThreads), 0, s, f, f.lvl_sn + S.lvl_ptr[l], z);
+    hipLaunchKernelGGL(k_mf_fwd, dim3(n), dim3(kFwdThreads), 0, s, f, f.lvl_sn + S.lvl_ptr[l], z);
   }
 }
 
