@@ -777,17 +777,100 @@ __global__ void k_zero_scalars(DevScalars* sc) {
 // Fronts are dense column-major F x F (F = 6 * front rows); the first K = 6 * node columns
 // are eliminated as L D L^T with the reference's 6x6 pivot rule (its block LDLt,
 // block_sparse_ldlt.rs:614-747: pivot block j gives (L_jj, d_j) = ldlt6(C_jj) and
-// L_ij = C_ij L_jj^-T D^+ L_jj^-1).  Here L is the scalar unit lower factor, the reference's
-// times blockdiag(L_jj): its columns are U D^+ with U = C L_PP^-T, so a panel's rows need one
-// product and a scaling.  Panels of kPanelBlocks pivot blocks are factored by one
+// L_ij = C_ij L_jj^-T D^+ L_jj^-1).  L has one of two forms, kBlocks of the kernels:
+//   false  the scalar unit lower factor, the reference's times blockdiag(L_jj): its columns are
+//          U D^+ with U = C L_PP^-T, so a panel's rows need one product and a scaling;
+//   true   the reference's own, unit block lower with M_j = (L_jj D_j L_jj^T)^+: a second product
+//          by blockdiag(M_j), and a diagonal block of 48 columns takes 45k cycles instead of 17k.
+//          For S of FP32 Schur products (launch_rcs_factor): once nu has fallen that S is not
+//          definite (smallest eigenvalue -4e-4 beside 6e7), its component along the free scale is
+//          decided by the rounding here, and the next products quantise the difference.  Runs
+//          depend on the form by 1e-4 to 1e-2, and the block form loses fewer of them: of 24 runs of
+//          2000 cameras (8 problems, inputs 1e-14 apart) 1 ended over 5% above the FP64 run's cost (6%),
+//          with the scalar factor 4 (up to 43%).
+// Panels of kPanelBlocks pivot blocks are factored by one
 // workgroup per node; the rank-48 trailing update runs as 64x64 tiles over many workgroups.
 
 constexpr int kPW = 6 * kPanelBlocks;
+
+// x <- x L^-T D^-1 L^-1 for a 6x6 pivot (unit lower L, dinv = reciprocal pivots, 0 for a
+// zero pivot)
+__device__ __forceinline__ void right_solve6(const double* L, const double* dinv, double x[6]) {
+#pragma unroll
+  for (int c = 0; c < 6; ++c) {
+    double v = x[c];
+    for (int t = 0; t < c; ++t) v -= x[t] * L[6 * c + t];
+    x[c] = v;
+  }
+#pragma unroll
+  for (int c = 0; c < 6; ++c) x[c] *= dinv[c];
+#pragma unroll
+  for (int c = 5; c >= 0; --c) {
+    double v = x[c];
+    for (int t = c + 1; t < 6; ++t) v -= x[t] * L[6 * t + c];
+    x[c] = v;
+  }
+}
 
 // View a [kPW][kTile + 1] LDS tile as a [kPW][kPW + 1] square (kPW <= kTile).
 static_assert(kPW <= kTile, "the next diagonal block lies inside tile (0, 0)");
 __device__ __forceinline__ double (*as_square(double (*t)[kTile + 1]))[kPW + 1] {
   return reinterpret_cast<double (*)[kPW + 1]>(&t[0][0]);
+}
+
+// Trailing update of pivot JB of a diagonal block: the rows below the next pivot block,
+// four threads per row (thread t3 of 192), each forming the row's L from its W and
+// updating every fourth column; the updated values of the next pivot's columns are also
+// kept in Wd (the next pivot's W).  The pivot index is a template argument so that the
+// column loop has a fixed length and its LDS reads can be issued together.
+template <int JB>
+__device__ __forceinline__ void diag_trailing(int t3, int np, const double* cL, const double* cdi,
+                                              double (*D)[kPW + 1], double (*Wd)[kPW + 1]) {
+  constexpr int J0 = 6 * JB, J1 = J0 + 6, kSplit = 4;
+  const int rr = t3 / kSplit, cg = t3 % kSplit;
+  const int r = J1 + 6 + rr;
+  if (J1 + 6 >= kPW || r >= np) return;
+  double x[6];
+#pragma unroll
+  for (int t = 0; t < 6; ++t) x[t] = Wd[r][J0 + t];
+  right_solve6(cL, cdi, x);
+  if (cg == 0)
+#pragma unroll
+    for (int t = 0; t < 6; ++t) D[r][J0 + t] = x[t];
+  constexpr int kCols = J1 < kPW ? (kPW - 1 - J1) / kSplit + 1 : 0;
+#pragma unroll
+  for (int i = 0; i < kCols; ++i) {
+    const int c = J1 + cg + kSplit * i;
+    if (c <= r) {
+      double acc = 0.0;
+#pragma unroll
+      for (int t = 0; t < 6; ++t) acc += x[t] * Wd[c][J0 + t];
+      const double v = D[r][c] - acc;
+      D[r][c] = v;
+      if (i < 2 && c < J1 + 6) Wd[r][c] = v;
+    }
+  }
+}
+
+// Row block JB of T = L^-1 for the unit block-lower L held below the pivot blocks of D
+// (its column blocks < JB are final), kept transposed in D's free upper triangle:
+// D[c][r] = T[r][c] for block(c) < block(r).  Entries slot, slot + stride, ...; each a
+// fixed-length sum (terms outside the entry's range masked) in four partial sums.
+template <int JB>
+__device__ __forceinline__ void diag_trows(int slot, int stride, double (*D)[kPW + 1]) {
+  constexpr int J0 = 6 * JB;
+  for (int e = slot; e < 6 * J0; e += stride) {
+    const int a = e % 6, c = e / 6, cb = c / 6;
+    double acc[4] = {-D[J0 + a][c], 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int kb = 1; kb < JB; ++kb)
+#pragma unroll
+      for (int t = 0; t < 6; ++t) {
+        const double tv = D[c][6 * kb + t];
+        acc[(6 * kb + t) & 3] -= D[J0 + a][6 * kb + t] * (kb > cb ? tv : 0.0);
+      }
+    D[c][J0 + a] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+  }
 }
 
 typedef double mfma_d4 __attribute__((ext_vector_type(4)));
@@ -1013,16 +1096,290 @@ __device__ __forceinline__ void factor_panel_diag(const DevFactor& f, const Diag
   }
 }
 
+// factor_panel_diag in the block form (6x6 pivots with the solver's rule): the pivots (L_jj, d_j,
+// M_j) go to piv_L / piv_d / piv_M and the block L_PP^-T to the panel's slot of tinv.  Called by all
+// threads of one workgroup.  D holds the block's lower triangle already when `loaded` (else it is
+// read from the front).  sL / sdi hold each pivot's factor (L_jj, then d_j in
+// sL[j][36..41]; 1 / d_j in sdi[j]).
+//
+// Per pivot j (one barrier each):
+//   wavefront 0   the next pivot block: lane (a, b), a >= b, of 21 forms row j1 + a of L
+//                 from its W (the row's values before the solve) and subtracts L_a W_b^T;
+//                 thread 0 gathers the 21 entries and factors the block, so its factor is
+//                 ready at the next barrier;
+//   wavefronts 1-3  the trailing update of the rows below the next pivot block (four
+//                 consecutive threads per row, each row's L formed from its W; the updated
+//                 values of the next pivot's columns are also kept in Wd, the next
+//                 pivot's W) and row block j of T = L_PP^-1 (its L columns are final),
+//                 spread from the last thread down so that it falls on the threads whose
+//                 rows have no trailing work.
+// The pivots' inverses M_j and the stores follow the loop.
+__device__ __forceinline__ void factor_panel_diag_blocks(const DevFactor& f, const DiagNode& dn, double* A,
+                                                         int F, int k0, int np, DevScalars* sc,
+                                                         double (*D)[kPW + 1], double (*Wd)[kPW + 1],
+                                                         double (*sL)[42], double (*sdi)[6], bool loaded,
+                                                         double* __restrict__ z) {
+  const int tid = threadIdx.x;
+  if (!loaded) {
+    stage_lds<(kPW * kPW + kThreads - 1) / kThreads>(
+        np * np,
+        [&](int e, bool ok) {
+          const int r = e % np, c = e / np;
+          return load_or_zero(A, int64_t(k0 + c) * F + k0 + r, ok && r >= c);
+        },
+        [&](int e, double v) { D[e % np][e / np] = v; });
+    __syncthreads();
+  }
+  // W of the first pivot: its columns below its block
+  for (int e = 36 + tid; e < 6 * np; e += blockDim.x) Wd[e / 6][e % 6] = D[e / 6][e % 6];
+  // L_PP^-T (row-major kPW x kPW) for the panel rows: its unit diagonal blocks and zeros
+  // here, the blocks above the diagonal as T's row blocks are formed
+  double* Tg = f.tinv + dn.poff + int64_t(k0 / kPW) * kPW * kPW;
+  for (int e = tid - 64; e >= 0 && e < kPW * kPW; e += blockDim.x - 64) {  // beside pivot 0
+    const int r = e / kPW, c = e % kPW;
+    if (r / 6 >= c / 6 || c >= np) Tg[e] = r == c && r < np ? 1.0 : 0.0;
+  }
+  // thread 0 factors the 6x6 block a6 into slot s
+  auto factor_pivot = [&](const double* a6, int s) {
+    double L[36], d[6], di[6];
+    const bool ok = f.scalar_pivots ? ldlt6<true>(a6, L, d, di) : ldlt6<false>(a6, L, d, di);
+    if (!ok) {
+      atomicOr(&sc->bad_pivot, 1);
+      for (int k = 0; k < 36; ++k) L[k] = (k % 7 == 0) ? 1.0 : 0.0;
+      for (int k = 0; k < 6; ++k) d[k] = di[k] = 0.0;
+    }
+    for (int k = 0; k < 36; ++k) sL[s][k] = L[k];
+    for (int k = 0; k < 6; ++k) {
+      sL[s][36 + k] = d[k];
+      sdi[s][k] = di[k];
+    }
+  };
+  if (tid == 0) {
+    double a6[36];
+    for (int a = 0; a < 6; ++a)
+      for (int b = 0; b < 6; ++b) a6[6 * a + b] = a >= b ? D[a][b] : D[b][a];
+    factor_pivot(a6, 0);
+  }
+  for (int j0 = 0; j0 < np; j0 += 6) {
+    __syncthreads();  // pivot j0 is in slot j0 / 6; the previous pivot's work is done
+    const int jb = j0 / 6;
+    const double* cL = sL[jb];
+    const double* cdi = sdi[jb];
+    const int j1 = j0 + 6, m = np - j1;  // the next pivot; rows of the block below this one
+    if (tid < 64) {
+      if (m > 0) {
+        const int e = tid < 21 ? tid : 0;
+        int a = 0;
+        while ((a + 1) * (a + 2) / 2 <= e) ++a;
+        const int b = e - a * (a + 1) / 2;
+        double x[6];
+#pragma unroll
+        for (int t = 0; t < 6; ++t) x[t] = Wd[j1 + a][j0 + t];
+        right_solve6(cL, cdi, x);
+        if (tid < 21 && b == 0)
+#pragma unroll
+          for (int t = 0; t < 6; ++t) D[j1 + a][j0 + t] = x[t];
+        double acc = D[j1 + a][j1 + b];
+#pragma unroll
+        for (int t = 0; t < 6; ++t) acc -= x[t] * Wd[j1 + b][j0 + t];
+        // gather the 21 entries into thread 0 (uniform reads of lanes 0..20)
+        const int2 bits = __builtin_bit_cast(int2, acc);
+        double a6[36];
+#pragma unroll
+        for (int q = 0; q < 21; ++q) {
+          int qa = 0;
+          while ((qa + 1) * (qa + 2) / 2 <= q) ++qa;
+          const int qb = q - qa * (qa + 1) / 2;
+          const int2 vb = make_int2(__builtin_amdgcn_readlane(bits.x, q),
+                                    __builtin_amdgcn_readlane(bits.y, q));
+          const double v = __builtin_bit_cast(double, vb);
+          a6[6 * qa + qb] = v;
+          a6[6 * qb + qa] = v;
+        }
+        if (tid == 0) factor_pivot(a6, jb + 1);
+      }
+    } else {
+      static_assert(kThreads - 64 == 4 * kPW && kPanelBlocks == 8, "four threads per block row");
+      switch (jb) {
+#define SGPU_TRAIL(J) \
+  case J: diag_trailing<J>(tid - 64, np, cL, cdi, D, Wd); break;
+        SGPU_TRAIL(0) SGPU_TRAIL(1) SGPU_TRAIL(2) SGPU_TRAIL(3)
+        SGPU_TRAIL(4) SGPU_TRAIL(5) SGPU_TRAIL(6) SGPU_TRAIL(7)
+#undef SGPU_TRAIL
+      }
+    }
+    // Beside the look-ahead: row block jb of T = L_PP^-1 (its L columns are final), kept
+    // transposed in the free upper triangle, D[c][r] = T[r][c] for block(c) < block(r),
+    // four partial sums per entry; then the outputs of pivot jb - 1 (M_j, L_jj, d_j) and
+    // the stores of L's column block jb - 1 and T's row block jb - 1.  The entries of T go
+    // first to the wavefronts with the least trailing work (wavefront 1, then 3 and 2 while
+    // wavefront 2's rows are updated, 2 and 3 after); the last pivot has no look-ahead,
+    // so there wavefront 0 joins and also handles that pivot's outputs.
+    const bool look = m > 0;
+    const int wv = tid >> 6, lane = tid & 63;
+    if (!look || wv > 0) {
+      const int pos = !look ? wv : (jb >= 4 ? wv - 1 : (wv == 1 ? 0 : (wv == 3 ? 1 : 2)));
+      const int slot = 64 * pos + lane, stride = look ? kThreads - 64 : kThreads;
+      switch (jb) {
+#define SGPU_TROWS(J) \
+  case J: diag_trows<J>(slot, stride, D); break;
+        SGPU_TROWS(1) SGPU_TROWS(2) SGPU_TROWS(3) SGPU_TROWS(4)
+        SGPU_TROWS(5) SGPU_TROWS(6) SGPU_TROWS(7)
+#undef SGPU_TROWS
+      }
+      // M_j = L^-T D^+ L^-1 (lane (a, b) of 36, from the columns of L^-1), L_jj and d_j
+      auto pivot_outputs = [&](int j) {
+        const int gb = dn.c0 + k0 / 6 + j;
+        if (lane < 36) {
+          const int a = lane / 6, b = lane % 6;
+          double ua[6], ub[6];
+#pragma unroll
+          for (int k = 0; k < 6; ++k) {
+            ua[k] = k == a ? 1.0 : 0.0;
+            ub[k] = k == b ? 1.0 : 0.0;
+          }
+#pragma unroll
+          for (int k = 1; k < 6; ++k)
+#pragma unroll
+            for (int t = 0; t < k; ++t) {
+              ua[k] -= sL[j][6 * k + t] * ua[t];
+              ub[k] -= sL[j][6 * k + t] * ub[t];
+            }
+          double mm = 0.0;
+#pragma unroll
+          for (int k = 0; k < 6; ++k) mm += ua[k] * sdi[j][k] * ub[k];
+          f.piv_M[36 * int64_t(gb) + lane] = mm;
+          f.piv_L[36 * int64_t(gb) + lane] = sL[j][lane];
+        } else if (lane < 42) {
+          f.piv_d[6 * int64_t(gb) + lane - 36] = sL[j][lane];
+        }
+      };
+      if (jb > 0 && wv == (jb >= 4 ? 2 : 3)) {
+        pivot_outputs(jb - 1);
+        const int p0 = j0 - 6;
+        for (int e = lane; e < 6 * p0; e += 64) {
+          const int cp = e / 6, a = e % 6;
+          Tg[cp * kPW + p0 + a] = D[cp][p0 + a];
+        }
+      }
+      if (!look && wv == 0) pivot_outputs(jb);
+    }
+  }
+  __syncthreads();  // T's last row block is in D
+  const int pl = np - 6;
+  for (int e = tid; e < 6 * pl; e += blockDim.x) {
+    const int cp = e / 6, a = e % 6;
+    Tg[cp * kPW + pl + a] = D[cp][pl + a];
+  }
+  if (k0 + np == F) {
+    // no rows below the panel (the last panel of a root), so no panel step follows: its
+    // right-hand side is final here; z_P = D^-1 L_PP^-1 b_P for the panel's columns
+    const double* bx = f.usolve + dn.uoff + k0;
+    double* yv = Wd[0];  // the block's W copy is done with
+    if (tid < np) {
+      double y = bx[tid];
+      for (int r = 0; r < 6 * (tid / 6); ++r) y += D[r][tid] * bx[r];  // T[c][r] = D[r][c]
+      yv[tid] = y;
+    }
+    __syncthreads();
+    if (tid < np / 6) {
+      const int j = tid;
+      double v[6];
+#pragma unroll
+      for (int i = 0; i < 6; ++i) {
+        double t = yv[6 * j + i];
+        for (int k = 0; k < i; ++k) t -= sL[j][6 * i + k] * v[k];
+        v[i] = t;
+      }
+#pragma unroll
+      for (int i = 0; i < 6; ++i) v[i] *= sdi[j][i];
+#pragma unroll
+      for (int i = 5; i >= 0; --i) {
+        double t = v[i];
+        for (int k = i + 1; k < 6; ++k) t -= sL[j][6 * k + i] * v[k];
+        v[i] = t;
+      }
+#pragma unroll
+      for (int i = 0; i < 6; ++i) z[6 * int64_t(dn.c0) + k0 + 6 * j + i] = v[i];
+    }
+  }
+}
+
 // First panel diagonal of the leaves (whose fronts are assembled before the factorization
 // starts; every other node's is factored by the last step of its last child).
+template <bool kBlocks>
 __global__ void __launch_bounds__(kThreads)
     k_mf_diag0(DevFactor f, const int32_t* __restrict__ nodes, DevScalars* sc, double* __restrict__ z) {
   const int X = nodes[blockIdx.x];
   const int F = 6 * f.sn_nf[X], K = 6 * f.sn_nc[X];
-  __shared__ double D[kPW][kPW + 1], Xs[kDiagScratch], T[kPW][kPW + 1];
-  factor_panel_diag(f, diag_node(f, X), f.front + f.sn_off[X], F, 0, min(K, kPW), sc, D, Xs, T,
-                    false, z);
+  double* A = f.front + f.sn_off[X];
+  if constexpr (kBlocks) {
+    __shared__ double D[kPW][kPW + 1], Wd[kPW][kPW + 1], sL[kPanelBlocks][42], sdi[kPanelBlocks][6];
+    factor_panel_diag_blocks(f, diag_node(f, X), A, F, 0, min(K, kPW), sc, D, Wd, sL, sdi, false, z);
+  } else {
+    __shared__ double D[kPW][kPW + 1], Xs[kDiagScratch], T[kPW][kPW + 1];
+    factor_panel_diag(f, diag_node(f, X), A, F, 0, min(K, kPW), sc, D, Xs, T, false, z);
+  }
 }
+
+// The form's middle factor of a panel in LDS: 1 / d of the pivots, or the M_j of the pivot blocks.
+template <bool kBlocks>
+struct PanelPivots {
+  static constexpr int kSize = kBlocks ? 36 * kPanelBlocks : kPW;
+  static constexpr int kLoads = (kSize + kThreads - 1) / kThreads;
+
+  // thread tid's loads of the panel with first column c (of 6 nb), np wide, and their LDS stores
+  static __device__ __forceinline__ void load(const DevFactor& f, int64_t c, int np, int tid, double (&v)[kLoads]) {
+#pragma unroll
+    for (int it = 0; it < kLoads; ++it) {
+      const int e = tid + kThreads * it;
+      if constexpr (kBlocks) v[it] = load_or_zero(f.piv_M, 6 * c + e, e < 6 * np);
+      else v[it] = load_or_zero(f.piv_r, c + e, e < np);
+    }
+  }
+  static __device__ __forceinline__ void store(double* s, int tid, const double (&v)[kLoads]) {
+#pragma unroll
+    for (int it = 0; it < kLoads; ++it)
+      if (tid + kThreads * it < kSize) s[tid + kThreads * it] = v[it];
+  }
+  // entry k of z_P = D^+ y_P (blockwise M_j)
+  static __device__ __forceinline__ double z(const double* s, const double* y, int k) {
+    if constexpr (!kBlocks) return y[k] * s[k];
+    const int jb = k / 6, a = k % 6;
+    double zz = 0.0;
+#pragma unroll
+    for (int t = 0; t < 6; ++t) zz += s[36 * jb + 6 * a + t] * y[6 * jb + t];
+    return zz;
+  }
+  // L = W D^+ for a wavefront's 16 rows of W, in registers as column tiles w[ct] (component q:
+  // row lc + 4 q, column 16 ct + lr) and as at(k, row); for blocks column tile ct meets the
+  // pivot blocks with rows [kL0[ct], kL1[ct]) and the block-diagonal operand is read from the M_j
+  template <typename At>
+  static __device__ __forceinline__ void scale(const double* s, int lr, int lc, At at, mfma_d4 (&w)[3]) {
+    if constexpr (!kBlocks) {
+#pragma unroll
+      for (int ct = 0; ct < 3; ++ct) w[ct] *= s[16 * ct + lr];
+    } else {
+      constexpr int kL0[3] = {0, 12, 30}, kL1[3] = {18, 36, 48};
+#pragma unroll
+      for (int ct = 0; ct < 3; ++ct) w[ct] = mfma_d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int k4 = 0; k4 < kPW; k4 += 4) {
+        const int k = k4 + lc;
+        const double av = at(k, lr);
+#pragma unroll
+        for (int ct = 0; ct < 3; ++ct)
+          if (k4 + 4 > kL0[ct] && k4 < kL1[ct]) {
+            const int n = 16 * ct + lr;
+            const double mv = k / 6 == n / 6 ? s[36 * (k / 6) + 6 * (k % 6) + n % 6] : 0.0;
+            w[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, mv, w[ct], 0, 0, 0);
+          }
+      }
+    }
+  }
+  // row at which column tile ct of L_PP^-T ends: it is (block) upper triangular
+  static constexpr int kW[3] = {kBlocks ? 18 : 16, kBlocks ? 36 : 32, 48};
+};
 
 // Position in the parent's front of row u of node X's update matrix (front row K + u):
 // update row block b is the parent's row block upos[b].
@@ -1145,6 +1502,7 @@ __device__ __forceinline__ void extend_tile_hand(const DevFactor& f, int X, int 
 // y_P = L_PP^-1 b_P (sb: b_P, bt: the rows' b, sy: the wavefront's copy of y_P), into the
 // parent's right-hand side on the node's last step (P >= 0); with zp, z_P = D^-1 y_P for
 // the panel's columns.
+template <bool kBlocks>
 __device__ __forceinline__ void panel_rows_out(const DevFactor& f, const DiagNode& dn, int P, int X,
                                                int F, int K, int k0, int np, int r0,
                                                const mfma_d4 (&L4)[3], const double (*sT)[kPW + 1],
@@ -1193,7 +1551,7 @@ __device__ __forceinline__ void panel_rows_out(const DevFactor& f, const DiagNod
           f.usolve[f.sn_uoff[P] + parent_row(f, X, r - K)] += bt[i] - part[q];
       }
     }
-  if (zp && lane < np) z[6 * int64_t(dn.c0) + k0 + lane] = sy[lane] * sR[lane];  // z_P = D^+ y_P
+  if (zp && lane < np) z[6 * int64_t(dn.c0) + k0 + lane] = PanelPivots<kBlocks>::z(sR, sy, lane);
 }
 
 // One round of panel steps, one workgroup per item (node, panel, tr, tc): the 64x64 tile
@@ -1222,6 +1580,7 @@ __device__ __forceinline__ void panel_rows_out(const DevFactor& f, const DiagNod
 // Each tile forms the L and W rows it needs itself (a row block is formed again by every
 // tile of its tile row and column), so a panel step is one launch with no panel-row pass
 // before it.
+template <bool kBlocks>
 __global__ void __launch_bounds__(kThreads)
     k_mf_step(DevFactor f, const int32_t* __restrict__ tiles, DevScalars* sc,
               double* __restrict__ z) {
@@ -1254,7 +1613,8 @@ __global__ void __launch_bounds__(kThreads)
   const int rw = 16 * wv;                              // the wavefront's 16-row slice
   __shared__ double sA[kPW][kTile + 1], sB[kPW][kTile + 1];  // C^T, then L^T / W^T
   __shared__ double sT[kPW][kPW + 1];                          // L_PP^-T
-  __shared__ double sR[kPW];  // 1 / d of the panel's pivots
+  using Pivots = PanelPivots<kBlocks>;
+  __shared__ double sR[Pivots::kSize];
   __shared__ double sb[kPW], sy[kThreads / 64][kPW];
   __shared__ double sbt[kTile];  // the output row block's rows of the right-hand side
   // the node's last panel step: its update matrix goes to the parent (-1: none)
@@ -1277,7 +1637,8 @@ __global__ void __launch_bounds__(kThreads)
     }
 #pragma unroll
     for (int it = 0; it < kNT; ++it) vt[it] = Tg[tid + kThreads * it];
-    const double vr = load_or_zero(f.piv_r, 6 * int64_t(dn.c0) + k0 + tid, tid < np);
+    double vr[Pivots::kLoads];
+    Pivots::load(f, 6 * int64_t(dn.c0) + k0, np, tid, vr);
     const double vbb = load_or_zero(bx, k0 + tid, out && tid < np);
     const double vbt = load_or_zero(bx, ro + tid - kPW, out && tid >= kPW && tid < kPW + kTile &&
                                                             ro + tid - kPW < F);
@@ -1292,10 +1653,8 @@ __global__ void __launch_bounds__(kThreads)
       const int e = tid + kThreads * it;
       sT[e / kPW][e % kPW] = vt[it];
     }
-    if (tid < kPW) {
-      sb[tid] = vbb;
-      sR[tid] = vr;
-    }
+    if (tid < kPW) sb[tid] = vbb;
+    Pivots::store(sR, tid, vr);
     if (tid >= kPW && tid < kPW + kTile) sbt[tid - kPW] = vbt;
   }
   __syncthreads();
@@ -1314,7 +1673,7 @@ __global__ void __launch_bounds__(kThreads)
       }
   // W = C L_PP^-T for the wavefront's slice of both row blocks; L_PP^-T is upper
   // triangular, so column tile ct stops at row kW[ct] (C and L_PP^-T are zero past np)
-  constexpr int kW[3] = {16, 32, 48};
+  constexpr auto& kW = Pivots::kW;
   mfma_d4 wa[3], wb[3];
 #pragma unroll
   for (int ct = 0; ct < 3; ++ct) wa[ct] = wb[ct] = mfma_d4{0.0, 0.0, 0.0, 0.0};
@@ -1342,21 +1701,35 @@ __global__ void __launch_bounds__(kThreads)
   }
   // L^T = D^+ W^T of the row block and W^T of the column block (a diagonal tile's is its row
   // block's) replace C; a wavefront has read only its own slice of C, so no barrier
+  if constexpr (kBlocks) {  // the product with the M_j reads W from LDS
 #pragma unroll
-  for (int ct = 0; ct < 3; ++ct) {
-    const double rd = sR[16 * ct + lr];
+    for (int ct = 0; ct < 3; ++ct)
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      sA[16 * ct + lr][rw + lc + 4 * q] = wa[ct][q] * rd;
-      sB[16 * ct + lr][rw + lc + 4 * q] = dg ? wa[ct][q] : wb[ct][q];
+      for (int q = 0; q < 4; ++q) {
+        sA[16 * ct + lr][rw + lc + 4 * q] = wa[ct][q];
+        sB[16 * ct + lr][rw + lc + 4 * q] = dg ? wa[ct][q] : wb[ct][q];
+      }
+    Pivots::scale(sR, lr, lc, [&](int k, int i) { return sA[k][rw + i]; }, wa);
+#pragma unroll
+    for (int ct = 0; ct < 3; ++ct)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) sA[16 * ct + lr][rw + lc + 4 * q] = wa[ct][q];
+  } else {
+#pragma unroll
+    for (int ct = 0; ct < 3; ++ct) {
+      const double rd = sR[16 * ct + lr];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        sA[16 * ct + lr][rw + lc + 4 * q] = wa[ct][q] * rd;
+        sB[16 * ct + lr][rw + lc + 4 * q] = dg ? wa[ct][q] : wb[ct][q];
+      }
     }
   }
   if (own0) {
-    // row block 0's outputs, from L of the block (the column block's W times 1 / d) in
+    // row block 0's outputs, from L of the block (the column block's W times D^+) in
     // registers: component q of wb[ct] is L row rw + lc + 4 q, column 16 ct + lr
-#pragma unroll
-    for (int ct = 0; ct < 3; ++ct) wb[ct] *= sR[16 * ct + lr];
-    panel_rows_out(f, dn, P, X, F, K, k0, np, ro + rw, wb, sT, sb, sR, sbt + rw, sy[wv], z,
+    Pivots::scale(sR, lr, lc, [&](int k, int i) { return sB[k][rw + i]; }, wb);
+    panel_rows_out<kBlocks>(f, dn, P, X, F, K, k0, np, ro + rw, wb, sT, sb, sR, sbt + rw, sy[wv], z,
                    lane, wv == 0);
   }
   __syncthreads();  // the update reads every row of L^T and W^T
@@ -1429,7 +1802,7 @@ __global__ void __launch_bounds__(kThreads)
     }
     // row block 0: z_P = D^+ y_P
     if (ro == kend && wv == 0 && lane < np)
-      z[6 * int64_t(dn.c0) + k0 + lane] = sy[0][lane] * sR[lane];
+      z[6 * int64_t(dn.c0) + k0 + lane] = Pivots::z(sR, sy[0], lane);
   }
   if (tr == 0 && tc == 0 && kend < K) {
     // the next panel's diagonal block is the top-left of this tile: hand the updated
@@ -1451,8 +1824,14 @@ __global__ void __launch_bounds__(kThreads)
   if (diag || hand) {
     __syncthreads();  // the block is in sB; the work above that reads sA is done
     const int Y = diag ? X : P, kd = diag ? kend : 0;
-    factor_panel_diag(f, diag_node(f, Y), f.front + f.sn_off[Y], 6 * f.sn_nf[Y], kd,
-                      min(6 * f.sn_nc[Y] - kd, kPW), sc, as_square(sB), &sA[0][0], sT, true, z);
+    double* AY = f.front + f.sn_off[Y];
+    const int FY = 6 * f.sn_nf[Y], npY = min(6 * f.sn_nc[Y] - kd, kPW);
+    if constexpr (kBlocks) {
+      __shared__ double sL[kPanelBlocks][42], sdi[kPanelBlocks][6];
+      factor_panel_diag_blocks(f, diag_node(f, Y), AY, FY, kd, npY, sc, as_square(sB), as_square(sA), sL, sdi, true, z);
+    } else {
+      factor_panel_diag(f, diag_node(f, Y), AY, FY, kd, npY, sc, as_square(sB), &sA[0][0], sT, true, z);
+    }
   }
 }
 
@@ -1466,6 +1845,7 @@ __global__ void __launch_bounds__(kThreads)
 // with L_PP^-T from the diagonal factorization.  It runs on the matrix cores as 4 x 3
 // tiles of v_mfma_f64_16x16x4, three per wavefront.  W goes to the node's W scratch, L to
 // the factor and, for the node's own rows, to its row-major copy.
+template <bool kBlocks>
 __global__ void __launch_bounds__(kThreads)
     k_mf_panel(DevFactor f, const int32_t* __restrict__ items, double* __restrict__ z) {
   static_assert(kPanelRows == 64 && kPW == 48 && kThreads == 256, "4 x 3 tiles, 3 per wavefront");
@@ -1484,7 +1864,8 @@ __global__ void __launch_bounds__(kThreads)
   __shared__ double sC[kPW][kPanelRows + 1];  // the rows' panel columns, C^T
   __shared__ double sT[kPW][kPW + 1];         // L_PP^-T
   __shared__ double sW[kPanelRows][kPW + 1];
-  __shared__ double sR[kPW];  // 1 / d of the panel's pivots
+  using Pivots = PanelPivots<kBlocks>;
+  __shared__ double sR[Pivots::kSize];
   __shared__ double sb[kPW], sy[kThreads / 64][kPW];  // the panel's RHS; y_P per wavefront
   double* bx = f.usolve + f.sn_uoff[X];  // the node's right-hand side (front row order)
   // every global load of the thread first, then the LDS stores
@@ -1497,7 +1878,8 @@ __global__ void __launch_bounds__(kThreads)
   }
 #pragma unroll
   for (int it = 0; it < kNT; ++it) vt[it] = Tg[tid + kThreads * it];
-  const double vr = load_or_zero(f.piv_r, 6 * int64_t(f.sn_c0[X]) + k0 + tid, tid < np);
+  double vr[Pivots::kLoads];
+  Pivots::load(f, 6 * int64_t(f.sn_c0[X]) + k0, np, tid, vr);
   const double vb = load_or_zero(bx, k0 + tid, tid < np);
 #pragma unroll
   for (int it = 0; it < kNC; ++it) {
@@ -1509,10 +1891,8 @@ __global__ void __launch_bounds__(kThreads)
     const int e = tid + kThreads * it;
     sT[e / kPW][e % kPW] = vt[it];
   }
-  if (tid < kPW) {
-    sb[tid] = vb;
-    sR[tid] = vr;
-  }
+  if (tid < kPW) sb[tid] = vb;
+  Pivots::store(sR, tid, vr);
   __syncthreads();
   // forward elimination of the right-hand side: y_P = L_PP^-1 b_P (each wavefront forms
   // its own copy; lane c < kPW entry c), and z_P = D^-1 y_P to the solve vector
@@ -1523,12 +1903,12 @@ __global__ void __launch_bounds__(kThreads)
     sy[wv][lane] = (a4[0] + a4[1]) + (a4[2] + a4[3]);
   }
   if (chunk == 0 && wv == 0 && lane < np)
-    z[6 * int64_t(f.sn_c0[X]) + k0 + lane] = sy[0][lane] * sR[lane];
+    z[6 * int64_t(f.sn_c0[X]) + k0 + lane] = Pivots::z(sR, sy[0], lane);
   // Wavefront wv owns row tile wv (16 rows) and its three 16-column tiles; it reads only
   // its own rows of C, W and L after the barrier above, so it needs no further barrier.
   // W = C L_PP^-T: L_PP^-T is upper triangular, so column tile ct stops at row
   // kW[ct] (C and L_PP^-T are zero past np).
-  constexpr int kW[3] = {16, 32, 48};
+  constexpr auto& kW = Pivots::kW;
   const int rw = 16 * wv;
   mfma_d4 acc[3];
 #pragma unroll
@@ -1543,14 +1923,14 @@ __global__ void __launch_bounds__(kThreads)
   }
   // W, and L^T = D^+ W^T into this wavefront's columns of sC
 #pragma unroll
-  for (int ct = 0; ct < 3; ++ct) {
-    const double rd = sR[16 * ct + lr];
+  for (int ct = 0; ct < 3; ++ct)
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      sW[rw + lk + 4 * q][16 * ct + lr] = acc[ct][q];
-      sC[16 * ct + lr][rw + lk + 4 * q] = acc[ct][q] * rd;
-    }
-  }
+    for (int q = 0; q < 4; ++q) sW[rw + lk + 4 * q][16 * ct + lr] = acc[ct][q];
+  Pivots::scale(sR, lr, lk, [&](int k, int i) { return sW[rw + i][k]; }, acc);
+#pragma unroll
+  for (int ct = 0; ct < 3; ++ct)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) sC[16 * ct + lr][rw + lk + 4 * q] = acc[ct][q];
   // the right-hand side of the wavefront's 16 rows: b_r -= L_r y_P (four lanes per row,
   // every fourth column, combined by two xor shuffles)
   {
@@ -1593,6 +1973,7 @@ __global__ void __launch_bounds__(kThreads)
 // go into the parent's front (extend-add).  The tile (0, 0), which holds the next panel's
 // diagonal block, then factors that block (on the last child's last step: the parent's
 // first one).  Two workgroups per CU (the tiles are many, and short).
+template <bool kBlocks>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
     k_mf_update(DevFactor f, const int32_t* __restrict__ tiles, DevScalars* sc,
                 double* __restrict__ z) {
@@ -1614,7 +1995,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
   const int lr = lane & 15, lc = lane >> 4;
   const int rb = 32 * (wv >> 1), cb = 32 * (wv & 1);  // the wavefront's quadrant
   __shared__ double sA[kPW][kTile + 1], sB[kPW][kTile + 1];
-  __shared__ double sT[kPW][kPW + 1];
+  __shared__ double sT[kBlocks ? 1 : kPW][kPW + 1];
   // the node's last panel step: its update matrix goes to the parent (-1: none)
   const int P = kend == K ? f.sn_parent[X] : -1;
   // the last child of its parent (in round order) factors the parent's first diagonal
@@ -1700,8 +2081,14 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
   if (diag || hand) {
     __syncthreads();  // the block is in sB; the work above that reads sA is done
     const int Y = diag ? X : P, kd = diag ? kend : 0;
-    factor_panel_diag(f, diag_node(f, Y), f.front + f.sn_off[Y], 6 * f.sn_nf[Y], kd,
-                      min(6 * f.sn_nc[Y] - kd, kPW), sc, as_square(sB), &sA[0][0], sT, true, z);
+    double* AY = f.front + f.sn_off[Y];
+    const int FY = 6 * f.sn_nf[Y], npY = min(6 * f.sn_nc[Y] - kd, kPW);
+    if constexpr (kBlocks) {
+      __shared__ double sL[kPanelBlocks][42], sdi[kPanelBlocks][6];
+      factor_panel_diag_blocks(f, diag_node(f, Y), AY, FY, kd, npY, sc, as_square(sB), as_square(sA), sL, sdi, true, z);
+    } else {
+      factor_panel_diag(f, diag_node(f, Y), AY, FY, kd, npY, sc, as_square(sB), &sA[0][0], sT, true, z);
+    }
   }
 }
 
@@ -1840,6 +2227,7 @@ __global__ void __launch_bounds__(kTriMax)
 // entries of L) before the panel's right-hand side is there.  With loads inside loops of the
 // panel's width it took 74 us a level for a tree of 150 cameras, now 30.
 constexpr int kFwdThreads = 512;
+template <bool kBlocks>
 __global__ void __launch_bounds__(kFwdThreads)
     k_mf_fwd(DevFactor f, const int32_t* __restrict__ nodes, double* __restrict__ z) {
   const int X = nodes[blockIdx.x];
@@ -1850,6 +2238,7 @@ __global__ void __launch_bounds__(kFwdThreads)
   const int tid = threadIdx.x;
   const bool solver = __builtin_amdgcn_readfirstlane(tid >> 6) == 0;  // the first wavefront
   __shared__ double sb[kPW], sy[kPW];
+  constexpr int kSums = kBlocks ? 1 : 4;  // partial sums of a product
   for (int ci = f.sn_child_ptr[X]; ci < f.sn_child_ptr[X + 1]; ++ci) {
     const int C = f.sn_child[ci];
     const int FC = 6 * f.sn_nf[C], KC = 6 * f.sn_nc[C];
@@ -1871,24 +2260,28 @@ __global__ void __launch_bounds__(kFwdThreads)
     load(cur, unsigned(solver ? min(tid, kPW - 1) : min(r0 + tid - 64, F - 1)));
     if (tid < kPW) sb[tid] = tid < np ? b[k0 + tid] : 0.0;
     __syncthreads();
-    if (solver) {
+    const auto product = [&](const double* x) __attribute__((always_inline)) {
       double y[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-      for (int t = 0; t < kPW; ++t) y[t & 3] += cur[t] * sb[t];
-      const double v = (y[0] + y[1]) + (y[2] + y[3]);
+      for (int t = 0; t < kPW; ++t) y[t % kSums] += cur[t] * x[t];
+      return kSums == 1 ? y[0] : (y[0] + y[1]) + (y[2] + y[3]);
+    };
+    if (solver) {
+      const double v = product(sb);
       if (tid < kPW) sy[tid] = tid < np ? v : 0.0;
-      if (tid < np) {
+      if (!kBlocks && tid < np) {
         const int64_t e = 6 * int64_t(c0) + k0 + tid;
         z[e] = v * f.piv_r[e];
       }
     }
     __syncthreads();
+    if (kBlocks && tid < np) {
+      const int64_t e = 6 * int64_t(c0) + k0 + tid;
+      z[e] = PanelPivots<true>::z(f.piv_M + 6 * (e - tid), sy, tid);
+    }
     if (!solver)
       for (int r = r0 + tid - 64; r < F; r += kFwdThreads - 64) {
-        double acc[4] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-        for (int t = 0; t < kPW; ++t) acc[t & 3] += cur[t] * sy[t];
-        b[r] -= (acc[0] + acc[1]) + (acc[2] + acc[3]);
+        b[r] -= product(sy);
         if (r + kFwdThreads - 64 < F) load(cur, unsigned(r + kFwdThreads - 64));
       }
     __syncthreads();
@@ -3024,19 +3417,20 @@ void launch_rcs_factor(hipStream_t s, const DevFactor& f, DevScalars* sc, const 
   hipLaunchKernelGGL(k_permute_in, dim3(g), dim3(kThreads), 0, s, f.nb, f.perm, rhs_nat, y);
   hipLaunchKernelGGL(k_mf_rhs_init, dim3(S.nsn), dim3(kThreads), 0, s, f, y);
   // the leaves' first diagonal blocks; every other node's is factored in a round
+  const bool blocks = f.block_form != 0;
   if (!S.leaves.empty())
-    hipLaunchKernelGGL(k_mf_diag0, dim3(S.leaves.size()), dim3(kThreads), 0, s, f, f.leaves, sc, y);
+    hipLaunchKernelGGL((blocks ? k_mf_diag0<true> : k_mf_diag0<false>), dim3(S.leaves.size()), dim3(kThreads), 0, s, f, f.leaves, sc, y);
   for (size_t li = 0; li < S.launches.size(); ++li) {
     const auto& L = S.launches[li];
     if (L.tile_count == 0) continue;
     const int32_t* items = f.launch_tiles + 4 * int64_t(L.tile_begin);
     if (f.step_events) SGPU_HIP(hipEventRecord(f.step_events[2 * li], s));
     if (L.fused) {
-      hipLaunchKernelGGL(k_mf_step, dim3(L.tile_count), dim3(kThreads), 0, s, f, items, sc, y);
+      hipLaunchKernelGGL((blocks ? k_mf_step<true> : k_mf_step<false>), dim3(L.tile_count), dim3(kThreads), 0, s, f, items, sc, y);
     } else {
-      hipLaunchKernelGGL(k_mf_panel, dim3(L.item_count), dim3(kThreads), 0, s, f,
+      hipLaunchKernelGGL((blocks ? k_mf_panel<true> : k_mf_panel<false>), dim3(L.item_count), dim3(kThreads), 0, s, f,
                          f.panel_items + 3 * int64_t(L.item_begin), y);
-      hipLaunchKernelGGL(k_mf_update, dim3(L.tile_count), dim3(kThreads), 0, s, f, items, sc, y);
+      hipLaunchKernelGGL((blocks ? k_mf_update<true> : k_mf_update<false>), dim3(L.tile_count), dim3(kThreads), 0, s, f, items, sc, y);
     }
     if (f.step_events) SGPU_HIP(hipEventRecord(f.step_events[2 * li + 1], s));
   }
@@ -3079,7 +3473,8 @@ void launch_rcs_forward(hipStream_t s, const DevFactor& f, const double* b_nat, 
   const int nlev = int(S.lvl_ptr.size()) - 1;
   for (int l = 0; l < nlev; ++l) {
     const int n = S.lvl_ptr[l + 1] - S.lvl_ptr[l];
-    hipLaunchKernelGGL(k_mf_fwd, dim3(n), dim3(kFwdThreads), 0, s, f, f.lvl_sn + S.lvl_ptr[l], z);
+    hipLaunchKernelGGL((f.block_form ? k_mf_fwd<true> : k_mf_fwd<false>), dim3(n), dim3(kFwdThreads), 0, s, f,
+                       f.lvl_sn + S.lvl_ptr[l], z);
   }
 }
 

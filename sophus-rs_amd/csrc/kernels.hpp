@@ -111,7 +111,9 @@ struct DevFactor {
   double* front;   // all fronts, column-major (workspace)
   double* lbuf;    // per node F x K: the factor's L columns (column-major, ld F)
   double* piv_d;   // nb x 6
-  double* piv_r;   // nb x 6: 1 / piv_d, 0 for a zero pivot
+  double* piv_r;   // nb x 6: 1 / piv_d, 0 for a zero pivot (scalar form; null with block_form)
+  double* piv_L;   // block form, else null: nb x 36 unit-lower pivot factors (row-major)
+  double* piv_M;   // and nb x 36 (L_jj D_j L_jj^T)^+ = L_jj^-T D_j^-1 L_jj^-1 (0 rows for zero pivots)
   int64_t front_elems;
   const Symbolic* host;  // launch schedule
   const int32_t* sn_child_ptr;  // children of each node (standalone forward solve; may be null
@@ -119,6 +121,9 @@ struct DevFactor {
   // pivot rule: 0 the 6x6 block rule of BlockSparseLdlt (dense_ldlt.rs:164-256), 1 the
   // scalar rule of SparseLdlt (sparse_ldlt.rs:399-445)
   int32_t scalar_pivots;
+  // form of L: 0 the scalar unit lower factor, 1 unit block lower with 6x6 pivots L_jj D_j L_jj^T
+  // (handles with FP32 Schur products)
+  int32_t block_form = 0;
 };
 
 constexpr int kPtRec = 18;  // doubles per packed point record (DevLin::prec)

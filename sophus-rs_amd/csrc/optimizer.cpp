@@ -389,7 +389,13 @@ struct sgpu_optimizer {
       df.wbuf = arena.alloc<double>(size_t(S.w_elems));
     }
     df.piv_d = arena.alloc<double>(size_t(6) * S.nb);
-    df.piv_r = arena.alloc<double>(size_t(6) * S.nb);
+    df.block_form = !iterative() && params.precision == SGPU_PRECISION_MIXED ? 1 : 0;
+    if (df.block_form) {
+      df.piv_L = arena.alloc<double>(size_t(36) * S.nb);
+      df.piv_M = arena.alloc<double>(size_t(36) * S.nb);
+    } else {
+      df.piv_r = arena.alloc<double>(size_t(6) * S.nb);
+    }
     df.front_elems = S.front_elems;
     df.host = &S;
     // workspace
@@ -630,7 +636,7 @@ struct sgpu_optimizer {
   // The matrix is the damped Hessian of build_solution's final linearization at the current
   // variables (nu = 0, or the current nu with skip_final_hessian), as DampedHessian holds it
   // (damped_hessian.rs:98).  S is factored with the direct solver's kernels, S = L diag(d) L^T
-  // with unit lower L.  Like the reference's min-norm LDLt
+  // with unit lower L (in the block form the factor's L times blockdiag(L_jj)).  Like the reference's min-norm LDLt
   // (block_sparse_min_norm_ldlt.rs:63-88), only positive pivots span the range: with S' = S
   // minus the non-positive pivots' terms, S'^+ b = P S'^- P b where S'^- = L^-T diag(d+)^-1 L^-1
   // (non-positive pivots give 0), and P projects off the null space of S', spanned by
@@ -659,7 +665,10 @@ struct sgpu_optimizer {
     launch_rcs_factor(stream, df, d_sc, dl.rhs_nat, dl.x_perm);
     SGPU_HIP(hipMemcpyAsync(h_sc, d_sc, sizeof(DevScalars), hipMemcpyDeviceToHost, stream));
     std::vector<double> d(n), sdiag(n);
+    std::vector<double> Lp(df.block_form ? size_t(6) * n : 0);
     SGPU_HIP(hipMemcpyAsync(d.data(), df.piv_d, n * 8, hipMemcpyDeviceToHost, stream));
+    if (df.block_form)
+      SGPU_HIP(hipMemcpyAsync(Lp.data(), df.piv_L, size_t(6) * n * 8, hipMemcpyDeviceToHost, stream));
     SGPU_HIP(hipMemcpyAsync(sdiag.data(), cov_sdiag, n * 8, hipMemcpyDeviceToHost, stream));
     SGPU_HIP(hipStreamSynchronize(stream));
     if (h_sc->singular_marg) throw Error(SGPU_ERR_NON_FINITE, "singular marginal block in the final Hessian");
@@ -675,15 +684,44 @@ struct sgpu_optimizer {
       cov_pivot_ratio = std::isfinite(lo) ? lo : 0.0;
     }
     std::vector<double> e(n), v(n);
+    // L_jj^-1 of pivot block gb (unit lower, row-major) by forward substitution; the identity in
+    // the scalar form
+    const auto pivot_inverse = [&](int64_t gb, double (&Li)[36]) {
+      for (int c = 0; c < 6; ++c)
+        for (int r = 0; r < 6; ++r) {
+          double x = r == c ? 1.0 : 0.0;
+          if (df.block_form)
+            for (int t = c; t < r; ++t) x -= Lp[36 * gb + 6 * r + t] * Li[6 * t + c];
+          Li[6 * r + c] = r < c ? 0.0 : x;
+        }
+    };
     const double zero = 0.0;
-    for (int64_t i = 0; i < n; ++i) {
-      if (d[i] > 0.0) continue;
-      SGPU_HIP(hipMemcpyAsync(df.piv_r + i, &zero, 8, hipMemcpyHostToDevice, stream));
+    for (int64_t gb = 0; gb < S.nb; ++gb) {
+      if (std::all_of(&d[6 * gb], &d[6 * gb] + 6, [](double x) { return x > 0.0; })) continue;
+      double r[6], Li[36], Mj[36];
+      for (int c = 0; c < 6; ++c) r[c] = d[6 * gb + c] > 0.0 ? 1.0 / d[6 * gb + c] : 0.0;
+      if (df.block_form) {  // M_j = L_jj^-T diag(1/d+) L_jj^-1
+        pivot_inverse(gb, Li);
+        for (int a = 0; a < 6; ++a)
+          for (int b = 0; b < 6; ++b) {
+            double acc = 0.0;
+            for (int k = 0; k < 6; ++k)
+              if (d[6 * gb + k] > 0.0) acc += Li[6 * k + a] * r[k] * Li[6 * k + b];
+            Mj[6 * a + b] = acc;
+          }
+        SGPU_HIP(hipMemcpyAsync(df.piv_M + 36 * gb, Mj, 36 * 8, hipMemcpyHostToDevice, stream));
+      } else {
+        for (int c = 0; c < 6; ++c)
+          if (r[c] == 0.0)
+            SGPU_HIP(hipMemcpyAsync(df.piv_r + 6 * gb + c, &zero, 8, hipMemcpyHostToDevice, stream));
+      }
     }
     for (int64_t i = 0; i < n; ++i) {
       if (d[i] > 0.0) continue;
+      double Li[36];
+      pivot_inverse(i / 6, Li);
       std::fill(e.begin(), e.end(), 0.0);
-      e[i] = 1.0;
+      for (int r = 0; r < 6; ++r) e[i / 6 * 6 + r] = Li[6 * (i % 6) + r];  // L_jj^-T e_c
       SGPU_HIP(hipMemcpyAsync(cov_z, e.data(), n * 8, hipMemcpyHostToDevice, stream));
       launch_rcs_solve(stream, df, cov_z, cov_x);
       SGPU_HIP(hipMemcpyAsync(v.data(), cov_x, n * 8, hipMemcpyDeviceToHost, stream));
