@@ -231,13 +231,21 @@ __global__ void k_gather_u32(const int32_t* __restrict__ src, const uint32_t* __
   if (e < n) keys[e] = uint32_t(src[order[e]]);
 }
 
-// Where each value starts in sorted keys: start[v] = the number of keys below v, 0 <= v <= m.
+// Where each value starts in sorted keys: start[v] = the number of keys below v, 0 <= v <= m.  A
+// thread per value searches for it: its neighbours read the same words on the way.  A thread per
+// key that writes the values up to the next one is a serial chain where values are missing (2M
+// points of which 500 are observed: 62.8 ms an analysis, so 14.3).
 template <typename P>
 __global__ void k_starts(const uint32_t* __restrict__ key, int64_t n, int64_t m, P* __restrict__ start) {
-  const int64_t k = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (k > n) return;
-  const int64_t lo = k == 0 ? 0 : int64_t(key[k - 1]) + 1, hi = k == n ? m : min(int64_t(key[k]), m);
-  for (int64_t v = lo; v <= hi; ++v) start[v] = P(k);
+  const int64_t v = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (v > m) return;
+  int64_t lo = 0, hi = n;  // key[lo - 1] < v <= key[hi]
+  while (lo < hi) {
+    const int64_t mid = (lo + hi) >> 1;
+    if (int64_t(key[mid]) < v) lo = mid + 1;
+    else hi = mid;
+  }
+  start[v] = P(lo);
 }
 
 // ---- S pattern ----------------------------------------------------------------------------
@@ -438,11 +446,11 @@ Symbolic analyze_device(const HostProblem& P, hipStream_t s, DeviceArena& arena,
                        reinterpret_cast<double2*>(T.obs_uv), key, key2);
   }
   std::swap(val, key2);  // the camera sort's input order
-  hipLaunchKernelGGL(k_starts<int32_t>, dim3(blocks_of(n + 1, kThreads)), dim3(kThreads), 0, s,
+  hipLaunchKernelGGL(k_starts<int32_t>, dim3(blocks_of(int64_t(S.npt) + 1, kThreads)), dim3(kThreads), 0, s,
                      reinterpret_cast<const uint32_t*>(T.obs_point), n, int64_t(S.npt), T.pt_ptr);
   radix_sort_pairs(s, tmp, key, val, key2, val2, n, bit_width(uint64_t(nb)));
-  hipLaunchKernelGGL(k_starts<int32_t>, dim3(blocks_of(n + 1, kThreads)), dim3(kThreads), 0, s, key, n, int64_t(nb),
-                     T.cam_ptr);
+  hipLaunchKernelGGL(k_starts<int32_t>, dim3(blocks_of(int64_t(nb) + 1, kThreads)), dim3(kThreads), 0, s, key, n,
+                     int64_t(nb), T.cam_ptr);
   const int32_t* cam_order = reinterpret_cast<const int32_t*>(val);
   if (S.npt > 0)
     hipLaunchKernelGGL(k_point_terms, dim3(blocks_of(S.npt, kThreads)), dim3(kThreads), 0, s, S.npt, T.pt_ptr,
@@ -535,7 +543,7 @@ Symbolic analyze_device(const HostProblem& P, hipStream_t s, DeviceArena& arena,
     radix_sort_pairs(s, tmp, key, val, key2, val2, total, bit_width(uint64_t(nslot)));
     hipLaunchKernelGGL(k_pairs_gather, dim3(blocks_of(total, kThreads)), dim3(kThreads), 0, s, total, val, pi, pj,
                        T.pairs);
-    hipLaunchKernelGGL(k_starts<int64_t>, dim3(blocks_of(total + 1, kThreads)), dim3(kThreads), 0, s, key, total,
+    hipLaunchKernelGGL(k_starts<int64_t>, dim3(blocks_of(nslot + 1, kThreads)), dim3(kThreads), 0, s, key, total,
                        nslot, d_pair_ptr);
     SGPU_HIP(hipMemcpyAsync(S.pair_ptr.data(), d_pair_ptr, (size_t(nslot) + 1) * 8, hipMemcpyDeviceToHost, s));
   }

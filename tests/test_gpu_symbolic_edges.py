@@ -25,3 +25,20 @@ def test_pattern_sizes_match_host(sg, cams, points, constant):
     r = sg.symbolic_check(v, p.cost_fns(1.0))
     assert r["mismatches"] == 0
     assert r["s_blocks"] >= cams - constant
+
+
+@pytest.mark.parametrize("first", [0, 700_000, 1_999_500])
+def test_mostly_unobserved_points(sg, first):
+    """2M points of which 500 are observed, at the start, inside and at the end: the lists over the
+    points have to be made in parallel where values are missing too (a serial chain there took
+    48 of 63 ms)."""
+    p = sg.generate_ba(sg.BaSpec(layout=0, num_cameras=10, num_points=500, obs_per_point_ring=5, seed=1))
+    points = np.zeros((2_000_000, 3))
+    points[:, 2] = 5.0
+    points[first:first + 500] = p.points_init
+    p = dataclasses.replace(p, points_init=points, obs_idx=p.obs_idx + np.array([0, 0, first]))
+    runs = [sg.symbolic_check(p.variables(), p.cost_fns(1.0)) for _ in range(4)]
+    assert all(r["mismatches"] == 0 for r in runs)
+    device, host = (min(r[k] for r in runs) for k in ("device_ms", "host_ms"))
+    print(f"first {first}: device {device:.2f} ms, host {host:.2f} ms", flush=True)
+    assert device <= 2.0 * host
