@@ -573,7 +573,9 @@ sgpu_status sgpu_precond_train(const sgpu_precond_train_params* params, float* w
  * (Marginalized) and pinhole reprojection terms (Huber if huber_delta > 0).  Each
  * window runs the same LM as sgpu_optimize_nlls (same rules, tolerances and
  * termination) with its reduced camera system solved densely in LDS; at most 31
- * cameras per window.  Arrays are concatenated over windows with prefix offsets. */
+ * cameras per window.  Arrays are concatenated over windows with prefix offsets.
+ * A batch holds lists besides its data: 4 bytes and up to 2 of segments for each pair of a
+ * point's observations by two cameras (other than camera 0), 24 bytes for each observation. */
 typedef struct sgpu_batch sgpu_batch;
 typedef struct sgpu_batch_desc {
   int64_t num_problems;

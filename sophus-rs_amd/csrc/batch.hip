@@ -46,6 +46,11 @@ constexpr int kBatchMaxCams = 31;
 constexpr int kRec = 21;     // doubles of a point's record
 constexpr int kSegment = 8;  // most pairs of a segment
 
+// Two camera blocks of a window: its first pair and its first full and partial segment there.
+struct BatchSlot {
+  int64_t pair, full, part;
+};
+
 struct BatchDev {
   int32_t nprob;
   const int32_t* order;      // launch slot -> problem (largest first)
@@ -64,12 +69,12 @@ struct BatchDev {
   const int32_t* cam_pt;     // observations camera by camera: their point within the problem
   const double* cam_uv;      // and uv
   const int32_t* cam_ptr;    // camera -> its first entry of those (prefix)
-  const int32_t* seg;        // (camera block i, block j < i, first pair in the problem, pairs)
-  const int32_t* seg_ptr;    // problem -> first segment (prefix, nprob + 1)
+  const int4* seg;           // segments of pairs (see segment())
+  const int64_t* seg_ptr;    // problem -> first segment (prefix, nprob + 1)
   const int64_t* pair_ptr;   // problem -> its first pair (prefix, nprob + 1)
   const int32_t* pair_pt;    // point within the problem of each pair
   const int32_t* same;       // an observation per pair of observations of a point by one camera
-  const int32_t* same_ptr;   // problem -> first entry of same (prefix, nprob + 1)
+  const int64_t* same_ptr;   // problem -> first entry of same (prefix, nprob + 1)
   const int32_t* pt_nu;      // reduced terms per point
   const int32_t* cam_nu;     // reduced terms per camera
   double* rec;               // kRec per point: x, H_ll^-1 (all 9: its triangles differ by rounding), damped
@@ -98,6 +103,11 @@ namespace {
 
 __host__ __device__ __forceinline__ int pk(int r, int c) {  // r >= c
   return int((unsigned(r) * unsigned(r + 1)) >> 1) + c;
+}
+
+// n pairs of camera blocks i and j < i from pair `first` of the problem (which may lie past 2^31).
+__device__ __forceinline__ int4 segment(int i, int j, int n, int64_t first) {
+  return make_int4(i | j << 8 | n << 16, 0, int(uint32_t(first)), int(first >> 32));
 }
 
 template <int NT>
@@ -683,18 +693,20 @@ __device__ __forceinline__ void batch_iteration(const BatchDev& d, int p, double
   }
   // cross terms: a thread per segment of points shared by two cameras
   const int32_t* pairs = d.pair_pt + d.pair_ptr[p];
-  for (int e = d.seg_ptr[p] + tid; e < d.seg_ptr[p + 1]; e += NT) {
-    const int4 sg = reinterpret_cast<const int4*>(d.seg)[e];
+  for (int64_t e = d.seg_ptr[p] + tid; e < d.seg_ptr[p + 1]; e += NT) {
+    const int4 sg = d.seg[e];
+    const int bi = sg.x & 255, bj = sg.x >> 8 & 255;
     double acc[36], ci[12], cj[12];
 #pragma unroll
     for (int k = 0; k < 36; ++k) acc[k] = 0.0;
 #pragma unroll
     for (int k = 0; k < 12; ++k) {
-      ci[k] = cams[15 * (sg.x + 1) + k];
-      cj[k] = cams[15 * (sg.y + 1) + k];
+      ci[k] = cams[15 * (bi + 1) + k];
+      cj[k] = cams[15 * (bj + 1) + k];
     }
-    for (int q = sg.z; q < sg.z + sg.w; ++q) {
-      const double* h = d.rec + kRec * int64_t(q0 + pairs[q]);
+    const int32_t* pt = pairs + (int64_t(sg.w) << 32 | uint32_t(sg.z));
+    for (int q = 0; q < sg.x >> 16; ++q) {
+      const double* h = d.rec + kRec * int64_t(q0 + pt[q]);
       const double x[3] = {h[0], h[1], h[2]};
       const T xt[3] = {T(x[0]), T(x[1]), T(x[2])};
       const T Hi[9] = {T(h[3]), T(h[4]), T(h[5]), T(h[6]), T(h[7]), T(h[8]), T(h[9]), T(h[10]), T(h[11])};
@@ -705,14 +717,14 @@ __device__ __forceinline__ void batch_iteration(const BatchDev& d, int p, double
       mul3(Z, M, N);
       lift<false>(xt, N, [&](int a, int b2, T val) { acc[6 * a + b2] -= double(val); });
     }
-    double* row = S + pk(6 * sg.x, 6 * sg.y);
+    double* row = S + pk(6 * bi, 6 * bj);
 #pragma unroll
     for (int a = 0; a < 6; ++a)
 #pragma unroll
-      for (int b2 = 0; b2 < 6; ++b2) atomicAdd(row + (6 * sg.x * a + a * (a + 1) / 2 + b2), acc[6 * a + b2]);
+      for (int b2 = 0; b2 < 6; ++b2) atomicAdd(row + (6 * bi * a + a * (a + 1) / 2 + b2), acc[6 * a + b2]);
   }
   // a point's repeated observations of one camera: the pair in both orders, B + B^T
-  for (int e = d.same_ptr[p] + tid; e < d.same_ptr[p + 1]; e += NT) {
+  for (int64_t e = d.same_ptr[p] + tid; e < d.same_ptr[p + 1]; e += NT) {
     const int ci = d.obs_cam[d.same[e]] - 1;
     const double* h = d.rec + kRec * int64_t(q0 + d.obs_pt[d.same[e]]);
     const double x[3] = {h[0], h[1], h[2]};
@@ -912,15 +924,15 @@ __global__ void __launch_bounds__(256)
 
 // The lists of a window that follow from its sorted observations, one workgroup per window:
 // the point of each observation, the observations camera by camera, and the points that two
-// cameras share.  A wavefront takes a camera and goes through the window's observations 64 at
+// cameras share with their segments.  A wavefront takes a camera and goes through the window's observations 64 at
 // a time, in order; an entry's place is the camera's (the pair's) count so far plus the
 // entries of lower lanes, so the lists come out as if written one by one.  Built on the host
 // they cost 250 ms for 1000 windows of 5300 observations, most of it page faults of 230 MB.
 constexpr int kListThreads = 512;
 __global__ void __launch_bounds__(kListThreads)
-    k_batch_lists(BatchDev d, const int32_t* __restrict__ slots, const int32_t* __restrict__ slot_ptr,
+    k_batch_lists(BatchDev d, const BatchSlot* __restrict__ slots, const int64_t* __restrict__ slot_ptr,
                   int32_t* obs_pt, int32_t* __restrict__ cam_pt, double* __restrict__ cam_uv,
-                  int32_t* __restrict__ pair_pt) {
+                  int32_t* __restrict__ pair_pt, int4* __restrict__ seg) {
   const int p = blockIdx.x, lane = threadIdx.x & 63;
   const int c0 = d.cam0[p], nc = d.cam0[p + 1] - c0, q0 = d.pt0[p], np = d.pt0[p + 1] - q0;
   const int o0 = d.obs0[p], o1 = d.obs0[p + 1];
@@ -929,11 +941,22 @@ __global__ void __launch_bounds__(kListThreads)
   __syncthreads();
   const unsigned long long below = (1ull << lane) - 1;
   int32_t* pairs = pair_pt + d.pair_ptr[p];
+  const BatchSlot* sl = slots + slot_ptr[p];  // one more than there are slots: the end
+  seg += d.seg_ptr[p];
+  for (int ci = 1, k = 0; ci < nc - 1; ++ci)
+    for (int cj = 0; cj < ci; ++cj, ++k) {
+      if (k % (kListThreads / 64) != threadIdx.x >> 6) continue;
+      const BatchSlot z = sl[k];
+      const int64_t n = sl[k + 1].pair - z.pair, full = n / kSegment;
+      for (int64_t t = lane; t < full; t += 64) seg[z.full + t] = segment(ci, cj, kSegment, z.pair + t * kSegment);
+      if (lane == 0 && n % kSegment)
+        seg[z.part] = segment(ci, cj, int(n % kSegment), z.pair + full * kSegment);
+    }
   for (int c = threadIdx.x >> 6; c < nc; c += kListThreads / 64) {
     const int ci = c - 1;
     int q = d.cam_ptr[c0 + c];
     // lane j: where the next pair of blocks ci and j goes
-    int to = lane < ci ? slots[slot_ptr[p] + ci * (ci - 1) / 2 + lane] : 0;
+    long long to = lane < ci ? sl[ci * (ci - 1) / 2 + lane].pair : 0;
     for (int z = o0; z < o1; z += 64) {
       const int o = z + lane;
       const bool mine = o < o1 && d.obs_cam[min(o, o1 - 1)] == c;
@@ -975,7 +998,7 @@ __global__ void __launch_bounds__(kListThreads)
           before = sum - n;
           all = __shfl(sum, 63);
         }
-        const int at = __shfl(to, cj) + before;
+        const long long at = __shfl(to, cj) + before;
         for (int k = 0; k < n; ++k) pairs[at + k] = b;
         if (lane == cj) to += all;
       }
@@ -1129,8 +1152,9 @@ sgpu_status sgpu_batch_create(const sgpu_batch_desc* desc, const sgpu_opt_params
       throw Error(SGPU_ERR_INVALID_ARGUMENT, "bad prefix arrays");
     int n_max = 0;
     std::vector<int32_t> cam0(P + 1), pt0(P + 1), obs0(P + 1), pt_obs(Q + 1), pt_nu(Q, 0), cam_nu(C, 0),
-        cam_ptr(C + 1, 0), seg, seg_ptr(P + 1, 0), same, same_ptr(P + 1, 0), slots, slot_ptr(P + 1, 0);
-    std::vector<int64_t> pair_ptr(P + 1, 0);
+        cam_ptr(C + 1, 0), same;
+    std::vector<int64_t> pair_ptr(P + 1, 0), seg_ptr(P + 1, 0), same_ptr(P + 1, 0), slot_ptr(P + 1, 0);
+    std::vector<BatchSlot> slots;
     for (int64_t p = 0; p <= P; ++p) {
       cam0[p] = int32_t(desc->cam_ptr[p]);
       pt0[p] = int32_t(desc->point_ptr[p]);
@@ -1216,22 +1240,20 @@ sgpu_status sgpu_batch_create(const sgpu_batch_desc* desc, const sgpu_opt_params
       for (int64_t c = 0; c < nc; ++c) cam_ptr[cam0[p] + c + 1] = obs0[p] + at[c + 1];
       // the points that two cameras share, pair by pair, in segments: full ones first, so that
       // the threads of a wavefront run alike
-      for (int64_t k = 0; k < nslot; ++k) slot[k + 1] += slot[k];
-      if (slot[nslot] > INT32_MAX) throw Error(SGPU_ERR_UNSUPPORTED, "too many Schur pairs in a window");
-      pair_ptr[p + 1] = pair_ptr[p] + slot[nslot];
-      for (int pass = 0; pass < 2; ++pass)
-        for (int32_t ci = 1, k = 0; ci < nc - 1; ++ci)
-          for (int32_t cj = 0; cj < ci; ++cj, ++k) {
-            const int32_t z = int32_t(slot[k]), n = int32_t(slot[k + 1]) - z, full = n / kSegment * kSegment;
-            if (pass == 0)
-              for (int32_t t = 0; t < full; t += kSegment) seg.insert(seg.end(), {ci, cj, z + t, kSegment});
-            else if (n > full)
-              seg.insert(seg.end(), {ci, cj, z + full, n - full});
-          }
-      slots.insert(slots.end(), slot, slot + nslot);
-      slot_ptr[p + 1] = int32_t(slots.size());
-      seg_ptr[p + 1] = int32_t(seg.size() / 4);
-      same_ptr[p + 1] = int32_t(same.size());
+      int64_t nseg = 0, pairs = 0;
+      const size_t s0 = slots.size();
+      for (int64_t k = 0; k < nslot; ++k) {
+        slots.push_back({pairs, nseg, 0});
+        pairs += slot[k + 1];
+        nseg += slot[k + 1] / kSegment;
+      }
+      for (int64_t k = 0; k < nslot; ++k)
+        if (slot[k + 1] % kSegment) slots[s0 + size_t(k)].part = nseg++;
+      slots.push_back({pairs, nseg, 0});
+      slot_ptr[p + 1] = int64_t(slots.size());
+      pair_ptr[p + 1] = pair_ptr[p] + pairs;
+      seg_ptr[p + 1] = seg_ptr[p] + nseg;
+      same_ptr[p + 1] = int64_t(same.size());
     }
     const int nt_max = 512;
     const size_t lds_doubles = size_t(pk(n_max + 1, 0)) + (params->precision == SGPU_PRECISION_MIXED ? 8 : 3) * size_t(n_max) + 15 * size_t(kBatchMaxCams);
@@ -1279,24 +1301,25 @@ sgpu_status sgpu_batch_create(const sgpu_batch_desc* desc, const sgpu_opt_params
       d.pt_obs = A.upload(pt_obs, nullptr);
       d.cam_ptr = A.upload(cam_ptr, nullptr);
       d.pair_ptr = A.upload(pair_ptr, nullptr);
-      d.seg = A.upload(seg, nullptr);
       d.seg_ptr = A.upload(seg_ptr, nullptr);
       {
         int32_t* obs_pt = A.alloc<int32_t>(O);
         int32_t* cam_pt = A.alloc<int32_t>(O);
         double* cam_uv = A.alloc<double>(2 * size_t(O));
         int32_t* pair_pt = A.alloc<int32_t>(size_t(pair_ptr[P]));
+        int4* seg = A.alloc<int4>(size_t(seg_ptr[P]));
         DeviceArena tmp;  // freed once the lists are there
-        const int32_t* sl = tmp.upload(slots, nullptr);
-        const int32_t* sp = tmp.upload(slot_ptr, nullptr);
+        const BatchSlot* sl = tmp.upload(slots, nullptr);
+        const int64_t* sp = tmp.upload(slot_ptr, nullptr);
         hipLaunchKernelGGL(k_batch_lists, dim3(unsigned(P)), dim3(kListThreads), 0, b->stream, d, sl, sp, obs_pt,
-                           cam_pt, cam_uv, pair_pt);
+                           cam_pt, cam_uv, pair_pt, seg);
         SGPU_HIP(hipGetLastError());
         SGPU_HIP(hipStreamSynchronize(b->stream));
         d.obs_pt = obs_pt;
         d.cam_pt = cam_pt;
         d.cam_uv = cam_uv;
         d.pair_pt = pair_pt;
+        d.seg = seg;
       }
       d.same = A.upload(same, nullptr);
       d.same_ptr = A.upload(same_ptr, nullptr);
