@@ -31,6 +31,7 @@
 #include <algorithm>
 #include <cfloat>
 #include <chrono>
+#include <cstring>
 #include <cmath>
 #include <numeric>
 #include <vector>
@@ -1123,6 +1124,44 @@ struct sgpu_batch {
 };
 
 namespace {
+
+// Device arrays in one allocation.  A small batch's creation is bound by the calls: with an
+// allocation, a copy and a free for each of its 40 arrays four windows of 2 cameras took 1.06 ms
+// (creation and destruction), so 0.75.  Up to kStage bytes of host values go up in one copy, more go
+// from where they are (a second pass over them would cost more).
+struct DeviceBlock {
+  static constexpr size_t kStage = size_t(1) << 20;
+  struct Part {
+    void* dst;  // where the array's address goes
+    const void* src;
+    size_t at, bytes;
+  };
+  std::vector<Part> parts;
+  size_t size = 0, filled = 0;  // bytes in all, and up to the end of the last host values
+  template <typename T>
+  void add(T*& dst, size_t n, const std::remove_const_t<T>* src = nullptr) {
+    parts.push_back({&dst, src, size, n * sizeof(T)});
+    size = (size + std::max<size_t>(n * sizeof(T), 1) + 255) & ~size_t(255);
+    if (src) filled = parts.back().at + parts.back().bytes;
+  }
+  template <typename T>
+  void add(const T*& dst, const std::vector<T>& v) {
+    add(dst, v.size(), v.data());
+  }
+  void commit(DeviceArena& arena) {
+    char* base = arena.alloc<char>(size);
+    std::vector<char> stage(filled <= kStage ? filled : 0);
+    for (const Part& p : parts) {
+      void* at = base + p.at;
+      std::memcpy(p.dst, &at, sizeof(at));
+      if (!p.src || !p.bytes) continue;
+      if (!stage.empty()) std::memcpy(stage.data() + p.at, p.src, p.bytes);
+      else SGPU_HIP(hipMemcpy(at, p.src, p.bytes, hipMemcpyHostToDevice));
+    }
+    if (!stage.empty()) SGPU_HIP(hipMemcpy(base, stage.data(), stage.size(), hipMemcpyHostToDevice));
+  }
+};
+
 template <typename F>
 void set_lds(F kernel, size_t bytes) {
   SGPU_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
@@ -1281,36 +1320,58 @@ sgpu_status sgpu_batch_create(const sgpu_batch_desc* desc, const sgpu_opt_params
       BatchDev& d = b->d;
       DeviceArena& A = b->arena;
       d.nprob = int32_t(P);
-      d.order = A.upload(order, nullptr);
-      d.cam0 = A.upload(cam0, nullptr);
-      d.pt0 = A.upload(pt0, nullptr);
-      d.obs0 = A.upload(obs0, nullptr);
-      d.intr = A.upload(std::vector<double>(desc->intrinsics, desc->intrinsics + 4 * P), nullptr);
-      d.poses_init = A.upload(std::vector<double>(desc->poses, desc->poses + 7 * C), nullptr);
-      d.points_init = A.upload(std::vector<double>(desc->points, desc->points + 3 * Q), nullptr);
+      // every array in one allocation, those with values from the host first
+      DeviceBlock B;
+      int32_t *obs_pt, *cam_pt, *pair_pt;
+      double* cam_uv;
+      int4* seg;
+      const int64_t* sp;
+      B.add(d.order, order);
+      B.add(d.cam0, cam0);
+      B.add(d.pt0, pt0);
+      B.add(d.obs0, obs0);
+      B.add(d.intr, size_t(4) * P, desc->intrinsics);
+      B.add(d.poses_init, size_t(7) * C, desc->poses);
+      B.add(d.points_init, size_t(3) * Q, desc->points);
+      B.add(d.obs_cam, size_t(O), obs_cam);
+      B.add(d.obs_uv, 2 * size_t(O), uv);
+      B.add(d.pt_obs, pt_obs);
+      B.add(d.cam_ptr, cam_ptr);
+      B.add(d.pair_ptr, pair_ptr);
+      B.add(d.seg_ptr, seg_ptr);
+      B.add(sp, slot_ptr);
+      B.add(d.same, same);
+      B.add(d.same_ptr, same_ptr);
+      B.add(d.pt_nu, pt_nu);
+      B.add(d.cam_nu, cam_nu);
+      B.add(obs_pt, size_t(O));
+      B.add(cam_pt, size_t(O));
+      B.add(cam_uv, 2 * size_t(O));
+      B.add(pair_pt, size_t(pair_ptr[P]));
+      B.add(seg, size_t(seg_ptr[P]));
       for (int i = 0; i < 2; ++i) {
-        d.poses[i] = A.alloc<double>(size_t(7) * C);
-        d.points[i] = A.alloc<double>(size_t(3) * Q);
+        B.add(d.poses[i], size_t(7) * C);
+        B.add(d.points[i], size_t(3) * Q);
       }
-      int32_t* oc = A.alloc<int32_t>(O);
-      double* ouv = A.alloc<double>(2 * size_t(O));
-      SGPU_HIP(hipMemcpy(oc, obs_cam, size_t(O) * sizeof(int32_t), hipMemcpyHostToDevice));
-      SGPU_HIP(hipMemcpy(ouv, uv, size_t(O) * 2 * sizeof(double), hipMemcpyHostToDevice));
-      d.obs_cam = oc;
-      d.obs_uv = ouv;
-      d.pt_obs = A.upload(pt_obs, nullptr);
-      d.cam_ptr = A.upload(cam_ptr, nullptr);
-      d.pair_ptr = A.upload(pair_ptr, nullptr);
-      d.seg_ptr = A.upload(seg_ptr, nullptr);
+      B.add(d.rec, size_t(kRec) * Q);
+      B.add(d.cur, P);
+      B.add(d.nu, P);
+      B.add(d.merit, P);
+      B.add(d.init_merit, P);
+      B.add(d.rejects, P);
+      B.add(d.steps, P);
+      B.add(d.done, P);
+      B.add(d.term, P);
+      B.add(b->out_poses, size_t(7) * C);
+      B.add(b->out_points, size_t(3) * Q);
+      B.add(b->queue, 1);
+      B.add(b->t_start, P);
+      B.add(b->t_end, P);
+      B.commit(A);
+      d.seg = seg;
       {
-        int32_t* obs_pt = A.alloc<int32_t>(O);
-        int32_t* cam_pt = A.alloc<int32_t>(O);
-        double* cam_uv = A.alloc<double>(2 * size_t(O));
-        int32_t* pair_pt = A.alloc<int32_t>(size_t(pair_ptr[P]));
-        int4* seg = A.alloc<int4>(size_t(seg_ptr[P]));
         DeviceArena tmp;  // freed once the lists are there
         const BatchSlot* sl = tmp.upload(slots, nullptr);
-        const int64_t* sp = tmp.upload(slot_ptr, nullptr);
         hipLaunchKernelGGL(k_batch_lists, dim3(unsigned(P)), dim3(kListThreads), 0, b->stream, d, sl, sp, obs_pt,
                            cam_pt, cam_uv, pair_pt, seg);
         SGPU_HIP(hipGetLastError());
@@ -1319,21 +1380,7 @@ sgpu_status sgpu_batch_create(const sgpu_batch_desc* desc, const sgpu_opt_params
         d.cam_pt = cam_pt;
         d.cam_uv = cam_uv;
         d.pair_pt = pair_pt;
-        d.seg = seg;
       }
-      d.same = A.upload(same, nullptr);
-      d.same_ptr = A.upload(same_ptr, nullptr);
-      d.pt_nu = A.upload(pt_nu, nullptr);
-      d.cam_nu = A.upload(cam_nu, nullptr);
-      d.rec = A.alloc<double>(size_t(kRec) * Q);
-      d.cur = A.alloc<int32_t>(P);
-      d.nu = A.alloc<double>(P);
-      d.merit = A.alloc<double>(P);
-      d.init_merit = A.alloc<double>(P);
-      d.rejects = A.alloc<int32_t>(P);
-      d.steps = A.alloc<int32_t>(P);
-      d.done = A.alloc<int32_t>(P);
-      d.term = A.alloc<int32_t>(P);
       d.robust = desc->huber_delta > 0.0 ? 1 : 0;
       d.delta = desc->huber_delta;
       d.nu0 = params->initial_lm_damping;
@@ -1356,11 +1403,6 @@ sgpu_status sgpu_batch_create(const sgpu_batch_desc* desc, const sgpu_opt_params
       set_lds(k_batch_persistent<float, 128>, lds_bytes);
       set_lds(k_batch_persistent<float, 256>, lds_bytes);
       set_lds(k_batch_persistent<float, 512>, lds_bytes);
-      b->out_poses = A.alloc<double>(size_t(7) * C);
-      b->out_points = A.alloc<double>(size_t(3) * Q);
-      b->queue = A.alloc<int32_t>(1);
-      b->t_start = A.alloc<unsigned long long>(P);
-      b->t_end = A.alloc<unsigned long long>(P);
       int khz = 0;
       SGPU_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, params->device));
       if (khz <= 0) throw Error(SGPU_ERR_HIP, "device wall-clock rate unavailable");

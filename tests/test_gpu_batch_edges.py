@@ -56,3 +56,21 @@ def test_window_edges_match_oracle(sg, orc, mode, mixed):
         assert np.max(np.abs(res["poses"][sl["poses"]] - vars_["poses"])) < 1e-7, p
         assert np.max(np.abs(res["points"][sl["points"]] - vars_["points"])) < 1e-7, p
     b.close()
+
+
+def test_small_and_large_batches_are_filled_alike(sg):
+    """Up to 1 MiB of host values go to the device in one copy, more array by array: a window of 60 kB
+    alone and 32 of it give the same runs."""
+    w = _window(sg, 9, 400, 6, 13)
+    params = sg.OptParams(num_iterations=8, initial_lm_damping=1.0)
+    results = []
+    for n in (1, 32):
+        b = sg.Batch([w] * n, params)
+        b.run(8)
+        results.append((b.results(), [b.window_slice(p) for p in range(n)]))
+        b.close()
+    one, many = results
+    for p, sl in enumerate(many[1]):
+        assert abs(many[0]["final_cost"][p] / one[0]["final_cost"][0] - 1.0) <= 1e-9, p
+        for name in ("poses", "points"):
+            assert np.max(np.abs(many[0][name][sl[name]] - one[0][name])) < 1e-7, (p, name)
