@@ -26,6 +26,11 @@ DEVICE = [
     "-munsafe-fp-atomics",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
+# The windows' persistent kernel is a loop around an LM iteration.  Hoisting out of that loop kept some
+# 80 registers of constants and addresses live through the whole iteration: with FP32 products 290, one
+# wavefront per SIMD less (2000 windows of 6 cameras, 20 iterations: 3.06 ms against 1.59 without), in FP64
+# 288 bytes of scratch at 512 threads (140 without).
+SOURCE_FLAGS = {"batch.hip": ["-mllvm", "-disable-machine-licm"]}
 
 
 def _hipcc() -> str:
@@ -51,7 +56,7 @@ def build_library(verbose: bool = False) -> Path:
     jobs = []
     for src in HIP_SOURCES:
         obj = objdir / (src + ".o")
-        jobs.append([hipcc, "-x", "hip", *COMMON, *DEVICE, "-c", str(CSRC / src), "-o", str(obj)])
+        jobs.append([hipcc, "-x", "hip", *COMMON, *DEVICE, *SOURCE_FLAGS.get(src, []), "-c", str(CSRC / src), "-o", str(obj)])
         objs.append(obj)
     for src in HOST_SOURCES:
         obj = objdir / (src + ".o")

@@ -901,8 +901,7 @@ __global__ void __launch_bounds__(NT)
     __syncthreads();
     for (int it = 0; it < iterations && !s_done; ++it) {
       // p is uniform, but read from LDS the compiler cannot know it: made a scalar so that
-      // the addresses derived from it stay in scalar registers (in vector registers the body
-      // takes 284 of them against 165, with spills at 512 threads)
+      // the addresses derived from it stay in scalar registers
       batch_iteration<T, NT>(d, __builtin_amdgcn_readfirstlane(p), lds, red, flags);
       __syncthreads();
       if (threadIdx.x == 0) s_done = d.done[p];

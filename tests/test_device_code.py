@@ -3,6 +3,9 @@
 The elimination's multiply-adds read one operand across lanes (DPP) in inline assembly, which the
 compiler's hazard handling does not look into: a vector instruction that writes that operand has to
 be two wait states away, or stale lanes are read silently.
+
+The windows' persistent kernels have to leave two wavefronts per SIMD their registers where that is
+what they had before (FP32 products), without scratch memory.
 """
 import re
 import struct
@@ -146,3 +149,23 @@ def test_cross_lane_operands_are_written_two_wait_states_before(code_objects):
         assert not bad, bad[:10]
         total += uses
     assert total > 1000, total
+
+
+def _resources(path):
+    """{kernel: (registers, scratch bytes)} from a code object's metadata."""
+    text = subprocess.run([LLVM / "llvm-readelf", "--notes", path], capture_output=True, text=True, check=True).stdout
+    out = {}
+    for entry in re.split(r"^  - ", text, flags=re.M)[1:]:
+        name = re.search(r"\.name:\s+(_Z\S+)", entry)
+        if name:
+            value = {k: int(re.search(rf"\.{k}:\s+(\d+)", entry).group(1))
+                     for k in ("vgpr_count", "private_segment_fixed_size")}
+            out[name.group(1)] = (value["vgpr_count"], value["private_segment_fixed_size"])
+    return out
+
+
+def test_persistent_windows_keep_two_wavefronts_per_simd(code_objects):
+    found = {n: r for path in code_objects for n, r in _resources(path).items() if "k_batch_persistentIf" in n}
+    assert len(found) == 3, found
+    for name, (registers, scratch) in found.items():
+        assert registers <= 256 and scratch == 0, (name, registers, scratch)
