@@ -40,6 +40,17 @@ def test_mixed_solves_keep_their_results(sg, name, spec, solver, iterations):
     assert _rel(s.variables.get_members("poses"), GOLDEN[name]) <= BAR
 
 
+@pytest.mark.parametrize("cams", [2, 3, 8, 9, 10, 17, 18])
+@pytest.mark.parametrize("solver", ["SchurBlockSparseLdlt", "SchurSparseLdlt"])
+def test_mixed_panel_widths_keep_their_results(sg, cams, solver):
+    """Diagonal blocks of one pivot block, of all eight and around panel boundaries."""
+    p = sg.generate_ba(sg.BaSpec(layout=0, num_cameras=cams, num_points=60, obs_per_point_ring=min(cams, 4), seed=cams))
+    params = sg.OptParams(num_iterations=6, initial_lm_damping=1.0, precision=sg.Precision.Mixed,
+                          solver=sg.Solver[solver])
+    s = sg.optimize_nlls(p.variables(), p.cost_fns(1.0), params)
+    assert _rel(s.variables.get_members("poses"), GOLDEN["rings"][str(cams)]) <= BAR
+
+
 def test_mixed_inverse_blocks_keep_their_values(sg):
     p = sg.generate_ba(sg.BaSpec(layout=1, num_cameras=100, num_points=3000, geometric_p=0.1, seed=3))
     m = np.arange(0, 100, 10)
