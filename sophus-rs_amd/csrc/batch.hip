@@ -443,12 +443,15 @@ __device__ __forceinline__ void window_backsolve(const double* S, int n, const d
 
 // The same system by 6x6 pivot blocks, L(:, k) = S(:, k) D_k^+ with D_k = L_6 diag(d) L_6^T
 // (stored in the packed diagonal block, strict lower L_6 and diagonal d), and its solution
-// into x.  The windows with FP32 Schur products keep this elimination: their S is near
-// singular once nu has fallen, and LM magnifies the rounding of single windows by 1e11.  Over
-// 12 batches of 1000 windows two runs of the same code differ by up to 6e-5 (norms, the
-// largest in one window; S is summed by atomics) and runs before and after the panels by no
-// more with this order, but by 7e-5 where repeated runs agree to 2e-7 with the order of
-// window_ldlt, which takes 9.9 ms for 10 iterations of such a batch instead of 12.2 ms.
+// into x.  The windows with FP32 Schur products keep this elimination so that they keep their
+// results: their S is near singular once nu has fallen, and LM magnifies the rounding of single
+// windows by 1e11.  Accuracy does not decide: of 36,000 runs of windows, 10 iterations each, 222 end
+// more than 1e-4 from the same window's FP64 run with this order and 222 with the order of
+// window_ldlt, 18 more than 0.1% above its cost and 18 below with either (geometric mean of the
+// distances 8.9e-7).  Runs before the sums per camera and segment, whose S depended on the order
+// of LDS atomics, differ among themselves by up to 5e-4 (norms over 1000 windows, 20 runs of a
+// batch); the present ones repeat to 1e-15 and lie among those.  The order of window_ldlt takes
+// 9.9 ms for 10 iterations of such a batch instead of 12.2 ms.
 __device__ __forceinline__ void d_solve(const double* S, int k, double v[6]) {
   const int o = 6 * k;
 #pragma unroll

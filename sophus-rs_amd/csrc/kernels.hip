@@ -1985,7 +1985,6 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
   double* A = f.front + f.sn_off[X];
   const double* Lo = f.lbuf + f.sn_loff[X];
   const double* Wo = f.wbuf + f.sn_woff[X];
-  const DiagNode dn = diag_node(f, X);
   const int k0 = kPW * panel;
   const int kend = min(K, k0 + kPW);
   const int np = kend - k0;

@@ -104,12 +104,13 @@ struct DevFactor {
   const int32_t* panel_items;  // (node, panel, kPanelRows-row chunk) per panel-row workgroup
   double* wbuf;                // per node F x kPW: unscaled W of the current panel (ld F)
   const int64_t* sn_woff;
-  double* tinv;                // per panel kPW x kPW row-major: L_PP^-T (unit block diagonal)
+  double* tinv;                // per panel kPW x kPW row-major: L_PP^-T
   const int64_t* sn_poff;
-  double* ltbuf;               // per node K x K: L_KK row-major (backward solve)
+  double* ltbuf;               // per node K x K: L_KK row-major (backward solve); the panels' own
+                               // diagonal blocks are never written here nor in lbuf (see tinv)
   const int64_t* sn_toff;
   double* front;   // all fronts, column-major (workspace)
-  double* lbuf;    // per node F x K: the factor's L columns (column-major, ld F)
+  double* lbuf;    // per node F x K: the factor's L columns below each panel (column-major, ld F)
   double* piv_d;   // nb x 6
   double* piv_r;   // nb x 6: 1 / piv_d, 0 for a zero pivot (scalar form; null with block_form)
   double* piv_L;   // block form, else null: nb x 36 unit-lower pivot factors (row-major)

@@ -503,7 +503,7 @@ Symbolic analyze_device(const HostProblem& P, hipStream_t s, DeviceArena& arena,
   if (nslot > int64_t(UINT32_MAX)) throw Error(SGPU_ERR_UNSUPPORTED, "too many S blocks");
   SGPU_HIP(hipMemcpyAsync(d_bits, bits.data(), nwords * 8, hipMemcpyHostToDevice, s));
   int32_t* d_wpre = upload_vec(tmp, wpre);
-  // pairs: count per point, offsets, fill in point order, stable sort by slot
+  // pairs: count per observation, offsets, fill in their order, stable sort by slot
   const int32_t ncm = S.cam_ptr[nb];
   T.cam_obs = arena.alloc<int32_t>(size_t(ncm));
   T.cm_point = arena.alloc<int32_t>(size_t(ncm));
