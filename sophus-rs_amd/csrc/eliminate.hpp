@@ -41,10 +41,13 @@ __device__ __forceinline__ void fmac_row_value(double& acc, double v, double m) 
 
 // Eliminates the first ncol (even) of kCols (<= 16) columns by one wavefront: lane i of each 16-lane
 // row holds pivot row i in p (the same in every row of lanes), every lane one row below in q.
-// No pivot test: a column is scaled by the reciprocal of what it finds.  (Quotients corrected by
-// their remainders give the same errors: backward 5e-17 to 1e-16 at 24 to 180 rows and condition
-// numbers 1e2 to 1e11, either way, and took a round of panel steps from 18.2 to 18.6 us.)  On
-// return p and q hold U = C L^-T and lane c (of each 16) the pivot d_c in dv.
+// No pivot test: a column is divided by what it finds.  The quotients are corrected by their
+// remainders (4 more instructions a column).  Products with the reciprocal alone have the same
+// errors (backward 5e-17 to 1e-16 at 24 to 180 rows and condition numbers 1e2 to 1e11, either way)
+// and take 18.2 instead of 18.6 us in a round of panel steps, but whole calls the same (2000 cameras
+// 1.000x, 500 cameras 0.998x); they would only move the results of long FP64 walks, where
+// the last bits decide whether a step is taken.  On return p and q
+// hold U = C L^-T and lane c (of each 16) the pivot d_c in dv.
 //
 // The next pivot's reciprocal is a chain of six dependent instructions; each is placed behind
 // some of the column's independent updates (the scheduling barriers keep that order, which
@@ -58,7 +61,10 @@ __device__ __forceinline__ void eliminate_columns(double (&p)[kCols], double (&q
     if (2 * pair >= ncol) return;
     static_for<2 * pair, 2 * pair + 2>([&](auto c) __attribute__((always_inline)) {
       dv = li == c ? d : dv;
-      const double lp = -(p[c] * r), lq = -(q[c] * r);
+      // -p / d and -q / d, each quotient corrected by its remainder
+      double lp = -(p[c] * r), lq = -(q[c] * r);
+      lp = fma(-fma(lp, d, p[c]), r, lp);
+      lq = fma(-fma(lq, d, q[c]), r, lq);
       // update k of the column: p[c + 1], then p and q in turn
       constexpr int kUp = 2 * (kCols - 1 - c);
       auto update = [&](auto k) __attribute__((always_inline)) {

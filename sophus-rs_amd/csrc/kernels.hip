@@ -963,7 +963,8 @@ static_assert(kDiagScratch <= kPW * (kTile + 1), "a staged tile's memory holds i
 //
 // Measured alone (one workgroup, loads and stores included) against 6x6 pivot blocks with
 // an LDS trailing update and a barrier each: 45.0k -> 17.1k cycles at np = 48, 20.0k -> 10.9k at
-// 24, 6.0k -> 5.3k at 6; a fused round of panel steps (500-camera walk) 29.0 -> 18.2 us.  Of
+// 24, 6.0k -> 5.3k at 6; a fused round of panel steps (500-camera walk) 29.0 -> 18.6 us
+// (18.2 before the quotients were corrected by their remainders).  Of
 // the 17.1k, 8.2k are the three parts, 3.6k the two exchanges.  A readlane and multiply-add per
 // update instead of the cross-lane operand took 24 cycles to its 5.
 __device__ __forceinline__ void factor_panel_diag(const DevFactor& f, const DiagNode& dn, double* A,
