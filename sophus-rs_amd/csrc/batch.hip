@@ -24,8 +24,8 @@
 // all its terms to S with LDS atomics, 36 a pair at about 40 cycles a wavefront: 621k to
 // 668k for the three); factor 71k in panels of 12 columns (258k to 544k with one thread per 6x6
 // pivot); solves 18k, back-substitution 33k, merit 27k (57k with a search for the point of
-// each observation).  24 windows of 5 to 30 cameras, 20 persistent iterations: 16.1 -> 5.55 ms;
-// 1000 such windows, FP32 products, 10 launches: 33.8 -> 12.2 ms.
+// each observation).  24 windows of 5 to 30 cameras, 20 persistent iterations: 16.0 -> 5.4 ms;
+// 1000 such windows, FP32 products, 10 launches: 33.9 -> 12.3 ms.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -451,7 +451,7 @@ __device__ __forceinline__ void window_backsolve(const double* S, int n, const d
 // distances 8.9e-7).  Runs before the sums per camera and segment, whose S depended on the order
 // of LDS atomics, differ among themselves by up to 5e-4 (norms over 1000 windows, 20 runs of a
 // batch); the present ones repeat to 1e-15 and lie among those.  The order of window_ldlt takes
-// 9.9 ms for 10 iterations of such a batch instead of 12.2 ms.
+// 9.9 ms for 10 iterations of such a batch instead of 12.3 ms.
 __device__ __forceinline__ void d_solve(const double* S, int k, double v[6]) {
   const int o = 6 * k;
 #pragma unroll
