@@ -52,6 +52,22 @@ def test_mixed_panel_widths_keep_their_results(sg, cams, solver):
     assert _rel(s.variables.get_members("poses"), GOLDEN["rings"][str(cams)]) <= BAR
 
 
+@pytest.mark.parametrize("solver", ["SchurBlockSparseLdlt", "SchurSparseLdlt"])
+def test_mixed_camera_without_observations(sg, solver):
+    """Six zero pivots: the camera stays where it is under the block rule and is NaN (null in the file)
+    under the scalar one, which divides by them."""
+    p = sg.generate_ba(sg.BaSpec(layout=0, num_cameras=10, num_points=60, obs_per_point_ring=4, seed=21))
+    keep = p.obs_idx[:, 1] != 4
+    p = dataclasses.replace(p, obs_idx=p.obs_idx[keep], obs_uv=p.obs_uv[keep])
+    params = sg.OptParams(num_iterations=6, initial_lm_damping=1.0, precision=sg.Precision.Mixed,
+                          solver=sg.Solver[solver])
+    poses = sg.optimize_nlls(p.variables(), p.cost_fns(1.0), params).variables.get_members("poses")
+    want = np.array([[np.nan if x is None else x for x in row] for row in GOLDEN["idle"][solver]])
+    lost = np.isnan(want)
+    assert np.array_equal(np.isnan(poses), lost) and lost.sum() == (7 if solver == "SchurSparseLdlt" else 0)
+    assert _rel(poses[~lost], want[~lost]) <= BAR
+
+
 def test_mixed_inverse_blocks_keep_their_values(sg):
     p = sg.generate_ba(sg.BaSpec(layout=1, num_cameras=100, num_points=3000, geometric_p=0.1, seed=3))
     m = np.arange(0, 100, 10)
